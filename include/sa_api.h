@@ -196,6 +196,24 @@ int sa_block_sparse_fwd_f32(const float* q, const int64_t q_strides[3], const fl
                             const int32_t* work_order, int64_t n_slots, void* stream);
 
 /*
+ * The same with a workspace: the products run on the bf16 matrix core, every fp32 operand
+ * (and P) split exactly into three bf16 terms and each product into the six term products down
+ * to 2^-18 of the largest, accumulated in fp32; errors against a 64-bit softmax are no larger
+ * than sa_block_sparse_fwd_f32's. The call first writes the split k and v to the workspace
+ * (`sa_block_sparse_fwd_f32_terms_workspace` bytes, 256-byte aligned). Heads whose |k| or |v|
+ * reach 2^60 (inf and NaN included) or whose |v| all lie below 2^-80, query blocks whose |q|
+ * reach 2^60, and heads with fewer than 3/2 listed tiles per key block are computed as
+ * sa_block_sparse_fwd_f32 does.
+ */
+int sa_block_sparse_fwd_f32_terms_workspace(int B, int H, int Lk, int D, int64_t* bytes);
+int sa_block_sparse_fwd_f32_terms(const float* q, const int64_t q_strides[3], const float* k,
+                                  const int64_t k_strides[3], const float* v, const int64_t v_strides[3], float* out,
+                                  const int64_t out_strides[3], int B, int H, int Lq, int Lk, int D,
+                                  const int32_t* kv_idx, const int32_t* kv_cnt, int max_cnt, float sm_scale,
+                                  const int32_t* work_order, int64_t n_slots, void* workspace,
+                                  int64_t workspace_bytes, void* stream);
+
+/*
  * Block-sparse attention with token-level masks inside cut blocks: as sa_block_sparse_fwd
  * (bf16, D = 64 or 128), plus kv_slot[row][i] = -1 (every pair of the tile attends) or the index of a 64x64
  * bitmask in tile_masks (uint64 [slots][64]: bit c of word r = query r of the block may

@@ -57,6 +57,12 @@ _PROTOTYPES = {
         [_P, _I64P, _P, _I64P, _P, _I64P, _P, _I64P, _I, _I, _I, _I, _I, _P, _P, _I, _P, _I64P, _F, _P,
          ctypes.c_int64, _P],
     ),
+    "sa_block_sparse_fwd_f32_terms_workspace": (_I, [_I, _I, _I, _I, _I64P]),
+    "sa_block_sparse_fwd_f32_terms": (
+        _I,
+        [_P, _I64P, _P, _I64P, _P, _I64P, _P, _I64P, _I, _I, _I, _I, _I, _P, _P, _I, _F, _P, ctypes.c_int64, _P,
+         ctypes.c_int64, _P],
+    ),
     "sa_block_sparse_fwd_tilemask": (
         _I,
         [_P, _I64P, _P, _I64P, _P, _I64P, _P, _I64P, _I, _I, _I, _I, _I, _P, _P, _P, _I, _I, _P, _F, _P,

@@ -21,6 +21,14 @@
 // rescale, no threshold), P = exp2(S * scale * log2(e) - m) in fp32, row sums in fp32.
 // Keys past Lk and list entries outside [0, nkb) get P = 0; their K/V loads are clamped to
 // the last key row, so every load is inside the tensors.
+//
+// With a workspace, bsa_fwd_f32_terms_kernel computes the same products on the bf16 matrix
+// core, 16 times the fp32 one's rate: every operand is split exactly into three bf16 terms
+// (x = hi + mid + lo, 8 significand bits each) and each product takes the six term products
+// down to 2^-18 of the largest (hi.hi, hi.mid, mid.hi, mid.mid, hi.lo, lo.hi; the dropped ones
+// are below 2^-26), accumulated in fp32. See that kernel below.
+#include <type_traits>
+
 #include "sa_common.h"
 
 #include <cmath>
@@ -58,6 +66,9 @@ struct F32Args {
   int pool_ncol;
   float* pool_lse;
   int pool_lpad;
+  // bsa_fwd_f32_terms_kernel: the split operands and the per-key-block flags (f32_terms_kernel).
+  const uint8_t* planes;
+  const uint4* flags;
 };
 
 __device__ inline sa_f32x4 mfma16x4(float a, float b, sa_f32x4 c) {
@@ -74,20 +85,14 @@ __device__ inline float slot_sum(float x) {
   return x + __shfl_xor(x, 32);
 }
 
-template <int kD, int kPool>
-__global__ __launch_bounds__(64 * kWavesF32, kD == 64 ? 2 : 1) void bsa_fwd_f32_kernel(F32Args a) {
-  static_assert(kD == 64 || kD == 128, "head dim 64 or 128");
-  static_assert(kPool == 0 || kPool == 32 || kPool == 64, "pooling columns of 32 or 64 keys");
+// One wave's fp32 pass over list positions it0, it0 + step, ... of query block qb: rows
+// 64 qb + row0 + (0 .. 16 kJ - 1). Leaves O^T (unnormalised), the running maxima and this
+// lane's row-sum parts in acc, m and l.
+template <int kD, int kPool, int kJ>
+__device__ __forceinline__ void f32_rows(const F32Args& a, int bh, int qb, int row0, int it0, int step, int lane,
+                                         sa_f32x4 (&acc)[kD / 16][kJ], float (&m)[kJ], float (&l)[kJ]) {
   constexpr int kHalf = kD / 64;   // 64-wide halves of d
   constexpr int kDB = kD / 16;     // 16-row d blocks of O^T
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int slot = blockIdx.x * kWavesF32 + wave;
-  if (slot >= a.n_slots) return;
-  const int item = __builtin_amdgcn_readfirstlane(a.order ? a.order[slot] : slot);
-  if (item < 0 || item >= a.n_items) return;
-  const int bh = item / a.nqb;
-  const int qb = item - bh * a.nqb;
   const int b = bh / a.H;
   const int h = bh - b * a.H;
   const int hk = a.kv_rep > 1 ? h / a.kv_rep : h;
@@ -103,14 +108,13 @@ __global__ __launch_bounds__(64 * kWavesF32, kD == 64 ? 2 : 1) void bsa_fwd_f32_
   const float* qbase = a.q + b * a.q_sb + h * a.q_sh;
   const float* khead = a.k + b * a.k_sb + hk * a.k_sh;
   const float* vhead = a.v + b * a.v_sb + hk * a.v_sh;
-  float* obase = a.o + b * a.o_sb + h * a.o_sh;
 
-  // Q^T B operands: qop[j][hf][s] = Q[qb * 64 + 16 j + r][64 hf + 16 g + s] (rows clamped into
-  // Lq; the clamped rows are never stored).
-  float qop[4][kHalf][16];
+  // Q^T B operands: qop[j][hf][s] = Q[qb * 64 + row0 + 16 j + r][64 hf + 16 g + s] (rows clamped
+  // into Lq; the clamped rows are never stored).
+  float qop[kJ][kHalf][16];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int row = min(qb * kBlk + 16 * j + r, a.Lq - 1);
+  for (int j = 0; j < kJ; ++j) {
+    const int row = min(qb * kBlk + row0 + 16 * j + r, a.Lq - 1);
 #pragma unroll
     for (int hf = 0; hf < kHalf; ++hf) {
       const float4* p = reinterpret_cast<const float4*>(qbase + (int64_t)row * a.q_sl + 64 * hf + 16 * g);
@@ -125,17 +129,16 @@ __global__ __launch_bounds__(64 * kWavesF32, kD == 64 ? 2 : 1) void bsa_fwd_f32_
     }
   }
 
-  sa_f32x4 acc[kDB][4];  // [dblk][j]: O^T[16 dblk + 4 g + i][16 j + r]
-  float m[4], l[4];      // per query column j: running max (log2 domain) and this lane's row-sum part
+  // acc[dblk][j]: O^T[16 dblk + 4 g + i][16 j + r]; m, l per query column j (log2 domain).
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
+  for (int j = 0; j < kJ; ++j) {
     m[j] = -INFINITY;
     l[j] = 0.f;
 #pragma unroll
     for (int dblk = 0; dblk < kDB; ++dblk) acc[dblk][j] = sa_f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
-  for (int it = 0; it < cnt; ++it) {
+  for (int it = it0; it < cnt; it += step) {
     const int kb = list[it];
     const bool ok = (unsigned)kb < (unsigned)a.nkb;
     const int key0 = ok ? kb * kBlk : 0;
@@ -143,7 +146,7 @@ __global__ __launch_bounds__(64 * kWavesF32, kD == 64 ? 2 : 1) void bsa_fwd_f32_
     const bool diag = kPool != 0 && a.causal && kb == qb;  // causal lists exist for pooling only
 
     // ---- S^T[16 kb16 + 4 g + i][16 j + r] in S[kb16][j][i].
-    sa_f32x4 S[4][4];
+    sa_f32x4 S[4][kJ];
 #pragma unroll
     for (int kb16 = 0; kb16 < 4; ++kb16) {
       const int key = min(key0 + 16 * kb16 + r, a.Lk - 1);
@@ -161,7 +164,7 @@ __global__ __launch_bounds__(64 * kWavesF32, kD == 64 ? 2 : 1) void bsa_fwd_f32_
         }
       }
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < kJ; ++j) {
         sa_f32x4 t = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int hf = 0; hf < kHalf; ++hf)
@@ -175,14 +178,14 @@ __global__ __launch_bounds__(64 * kWavesF32, kD == 64 ? 2 : 1) void bsa_fwd_f32_
     // column maxima, running maximum per query, then P = exp2(S * sc - m) in place and the
     // row sums.
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < kJ; ++j) {
       float mx = -INFINITY;
 #pragma unroll
       for (int kb16 = 0; kb16 < 4; ++kb16)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int kk = 16 * kb16 + 4 * g + i;
-          if (kk >= nvalid || (kPool != 0 && diag && kk > 16 * j + r)) S[kb16][j][i] = -INFINITY;
+          if (kk >= nvalid || (kPool != 0 && diag && kk > row0 + 16 * j + r)) S[kb16][j][i] = -INFINITY;
           mx = fmaxf(mx, S[kb16][j][i]);
         }
       if constexpr (kPool != 0) {
@@ -197,7 +200,8 @@ __global__ __launch_bounds__(64 * kWavesF32, kD == 64 ? 2 : 1) void bsa_fwd_f32_
               for (int i = 0; i < 4; ++i) x = fmaxf(x, S[kb16][j][i]);
             x = slot_max(x) * a.scale_log2;  // scale > 0
             if (g == 0)
-              a.pool_r[(((int64_t)bh * a.nqb + qb) * a.pool_ncol + kb * kCols + cc) * kBlk + 16 * j + r] = x;
+              a.pool_r[(((int64_t)bh * a.nqb + qb) * a.pool_ncol + kb * kCols + cc) * kBlk + row0 +
+                     16 * j + r] = x;
           }
         }
       }
@@ -234,25 +238,585 @@ __global__ __launch_bounds__(64 * kWavesF32, kD == 64 ? 2 : 1) void bsa_fwd_f32_
 #pragma unroll
         for (int dblk = 0; dblk < kDB; ++dblk)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) acc[dblk][j] = mfma16x4(vop[dblk], S[kb16][j][i], acc[dblk][j]);
+          for (int j = 0; j < kJ; ++j) acc[dblk][j] = mfma16x4(vop[dblk], S[kb16][j][i], acc[dblk][j]);
       }
   }
+}
 
-  // ---- Epilogue: out = acc / l; an empty list writes 0. Pooling: the row's log2-sum-exp2.
+// Epilogue of one wave: out = acc / l; an empty list writes 0. Pooling: the row's log2-sum-exp2.
+template <int kD, int kPool, int kJ>
+__device__ __forceinline__ void f32_store(const F32Args& a, int bh, int qb, int row0, int lane,
+                                          const sa_f32x4 (&acc)[kD / 16][kJ], const float (&m)[kJ],
+                                          const float (&l)[kJ]) {
+  const int b = bh / a.H;
+  const int h = bh - b * a.H;
+  const int r = lane & 15, g = lane >> 4;
+  float* obase = a.o + b * a.o_sb + h * a.o_sh;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
+  for (int j = 0; j < kJ; ++j) {
     const float l_tot = slot_sum(l[j]);
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-    const int row = qb * kBlk + 16 * j + r;
+    const int row = qb * kBlk + row0 + 16 * j + r;
     if constexpr (kPool != 0) {
       if (g == 0) a.pool_lse[(int64_t)bh * a.pool_lpad + row] = (m[j] == -INFINITY ? 0.f : m[j]) + log2f(l_tot);
     }
     if (row < a.Lq) {
       float* orow = obase + (int64_t)row * a.o_sl;
 #pragma unroll
-      for (int dblk = 0; dblk < kDB; ++dblk) {
+      for (int dblk = 0; dblk < kD / 16; ++dblk) {
         const sa_f32x4 A = acc[dblk][j];
         *reinterpret_cast<float4*>(orow + 16 * dblk + 4 * g) = make_float4(A[0] * inv, A[1] * inv, A[2] * inv, A[3] * inv);
+      }
+    }
+  }
+}
+
+template <int kD, int kPool>
+__global__ __launch_bounds__(64 * kWavesF32, kD == 64 ? 2 : 1) void bsa_fwd_f32_kernel(F32Args a) {
+  static_assert(kD == 64 || kD == 128, "head dim 64 or 128");
+  static_assert(kPool == 0 || kPool == 32 || kPool == 64, "pooling columns of 32 or 64 keys");
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int slot = blockIdx.x * kWavesF32 + wave;
+  if (slot >= a.n_slots) return;
+  const int item = __builtin_amdgcn_readfirstlane(a.order ? a.order[slot] : slot);
+  if (item < 0 || item >= a.n_items) return;
+  const int bh = item / a.nqb;
+  const int qb = item - bh * a.nqb;
+  sa_f32x4 acc[kD / 16][4];
+  float m[4], l[4];
+  f32_rows<kD, kPool, 4>(a, bh, qb, 0, 0, 1, lane, acc, m, l);
+  f32_store<kD, kPool, 4>(a, bh, qb, 0, lane, acc, m, l);
+}
+
+// ---------------------------------------------------------------------------------------
+// Split operands. f32_terms_kernel writes, per key/value head and 64-key block, the three bf16
+// terms of the block's K and V in the order in which bsa_fwd_f32_terms_kernel consumes them:
+// per 32-key chunk c, groups of six 1 KB operands (16 bytes per lane, lane l at 16 l), so that
+// every operand load is one coalesced 1 KB read and takes no LDS:
+//   K group i (d steps s = 2 i, 2 i + 1 of 16): operand 3 (s % 2) + term, lane (col, hh) holds
+//     K[32 c + col][16 s + 8 hh .. + 7], the A operand of S^T = K Q^T;
+//   V group (u, dp) (16 keys from 32 c + 16 u, d chunks dc = 2 dp, 2 dp + 1 of 32): operand
+//     3 (dc % 2) + term, lane (col, hh) holds V[32 c + 16 u + 8 (j / 4) + 4 hh + j % 4]
+//     [32 dc + col], j < 8: the A operand of O^T = V^T P^T for the key slots in which S^T leaves P.
+// Rows past Lk are zero. flags[head * nkb + block] = the largest |k| of the block's two chunks
+// and the largest |v| of its two chunks (fp32 bits): the attention takes the split operands only
+// where all are below kTermMax (no inf or NaN, no product near overflow) and the values not all
+// below kTermMin (their low terms would leave bf16's normal range); other heads run in fp32.
+// A head whose lists hold fewer than 3/2 tiles per key block is not worth the pass: its blocks
+// are only flagged (kTermSkip) and it runs in fp32. Measured on [2, 30, 17776, 64] (fp32 kernel
+// against this path, us): 2.1 tiles per block 586 / 609, 2.7 695 / 659, 4.3 993 / 801; with one
+// tile per block of [2, 30, 3000, 64] 49 / 92.
+constexpr uint32_t kTermMax = 0x5d800000u;  // 2^60
+constexpr uint32_t kTermMin = 0x17800000u;  // 2^-80
+constexpr uint32_t kTermSkip = 0xffffffffu;  // no |x| has these bits
+
+template <int kD>
+struct TermLayout {
+  static constexpr int kGroup = 6 * 1024;                  // bytes per group
+  static constexpr int kKGroups = kD / 32;                 // K groups per 32-key chunk
+  static constexpr int kGroups = kKGroups + 2 * (kD / 64);  // all groups per chunk
+  static constexpr int kTile = 2 * kGroups * kGroup;        // bytes per 64-key block: 768 kD
+};
+
+typedef unsigned f32_u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 f32_bf16x2 __attribute__((ext_vector_type(2)));
+
+__device__ inline uint32_t pack_bf16(float x0, float x1) {  // round to nearest even
+  const f32_bf16x2 r = {(__bf16)x0, (__bf16)x1};
+  return __builtin_bit_cast(uint32_t, r);
+}
+
+// The three bf16 terms of x0 and x1, packed: each remainder is exact in fp32, and the last one
+// has at most 8 significand bits, so hi + mid + lo = x (above bf16's subnormals).
+__device__ inline void split3(float x0, float x1, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+  hi = pack_bf16(x0, x1);
+  const float a0 = x0 - __uint_as_float(hi << 16), a1 = x1 - __uint_as_float(hi & 0xffff0000u);
+  mid = pack_bf16(a0, a1);
+  lo = pack_bf16(a0 - __uint_as_float(mid << 16), a1 - __uint_as_float(mid & 0xffff0000u));
+}
+
+__device__ inline uint32_t abs_bits(float x) { return __float_as_uint(x) & 0x7fffffffu; }
+
+__device__ inline uint32_t wave_max_u(uint32_t x) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) x = max(x, (uint32_t)__shfl_xor((int)x, o));
+  return x;
+}
+
+struct TermArgs {
+  const float* k;
+  const float* v;
+  int64_t k_sb, k_sh, k_sl;
+  int64_t v_sb, v_sh, v_sl;
+  int Hk, Lk, nkb;
+  const int32_t* kv_cnt;  // [B * Hk][nqb] list lengths, or null: every block is split
+  int nqb, max_cnt;
+  uint8_t* planes;
+  uint32_t* flags;  // [B * Hk * nkb][4]
+};
+
+// One workgroup per (head, key block): waves 0, 1 split the K chunks, waves 2, 3 the V chunks.
+// HBM-bound: 512 kD bytes read and 768 kD written per block.
+template <int kD>
+__global__ __launch_bounds__(256) void f32_terms_kernel(TermArgs a) {
+  typedef TermLayout<kD> Lay;
+  __shared__ int64_t tiles[4];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t blk = blockIdx.x;
+  const int bh = (int)(blk / a.nkb);
+  const int kb = (int)(blk - (int64_t)bh * a.nkb);
+  if (a.kv_cnt) {
+    int64_t n = 0;
+    for (int i = threadIdx.x; i < a.nqb; i += 256) n += min(max(a.kv_cnt[(int64_t)bh * a.nqb + i], 0), a.max_cnt);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
+    if (lane == 0) tiles[wave] = n;
+    __syncthreads();
+    if (2 * (tiles[0] + tiles[1] + tiles[2] + tiles[3]) < 3 * (int64_t)a.nkb) {
+      if (threadIdx.x < 4) a.flags[blk * 4 + threadIdx.x] = kTermSkip;
+      return;
+    }
+  }
+  const int b = bh / a.Hk, h = bh - b * a.Hk;
+  const int col = lane & 31, hh = lane >> 5;
+  const int c = wave & 1;
+  const int key0 = kb * kBlk + 32 * c;
+  uint8_t* dst = a.planes + blk * Lay::kTile + c * Lay::kGroups * Lay::kGroup + 16 * lane;
+  uint32_t amax = 0u;
+  auto put = [&](int group, int operand, const float (&x)[8]) {
+    f32_u32x4 t[3];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      uint32_t hi, mid, lo;
+      split3(x[2 * i], x[2 * i + 1], hi, mid, lo);
+      t[0][i] = hi;
+      t[1][i] = mid;
+      t[2][i] = lo;
+      amax = max(amax, max(abs_bits(x[2 * i]), abs_bits(x[2 * i + 1])));
+    }
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+      *reinterpret_cast<f32_u32x4*>(dst + group * Lay::kGroup + (operand + p) * 1024) = t[p];
+  };
+  if (wave < 2) {
+    const int key = key0 + col;
+    const float* row = a.k + b * a.k_sb + h * a.k_sh + (int64_t)min(key, a.Lk - 1) * a.k_sl + 8 * hh;
+#pragma unroll
+    for (int s = 0; s < kD / 16; ++s) {
+      const float4 x0 = *reinterpret_cast<const float4*>(row + 16 * s);
+      const float4 x1 = *reinterpret_cast<const float4*>(row + 16 * s + 4);
+      float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = key < a.Lk ? x[j] : 0.f;
+      put(s >> 1, 3 * (s & 1), x);
+    }
+  } else {
+    const float* base = a.v + b * a.v_sb + h * a.v_sh + col;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int dc = 0; dc < kD / 32; ++dc) {
+        float x[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const int key = key0 + 16 * u + 8 * (j >> 2) + 4 * hh + (j & 3);
+          const float y = base[(int64_t)min(key, a.Lk - 1) * a.v_sl + 32 * dc];
+          x[j] = key < a.Lk ? y : 0.f;
+        }
+        put(Lay::kKGroups + u * (kD / 64) + (dc >> 1), 3 * (dc & 1), x);
+      }
+  }
+  amax = wave_max_u(amax);
+  if (lane == 0) a.flags[blk * 4 + wave] = amax;
+}
+
+__device__ inline sa_f32x16 mfma_bf16(f32_u32x4 x, f32_u32x4 y, sa_f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(sa_bf16x8, x), __builtin_bit_cast(sa_bf16x8, y),
+                                                 c, 0, 0, 0);
+}
+
+// max / sum of x over lanes l and l ^ 32.
+__device__ inline float half_max(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ inline float half_sum(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// fp32 attention on split operands. A wave owns 32 kG query rows (head dim 64: a whole 64-row
+// block, 128: half of one) and walks its tiles in 32-key chunks with v_mfma_f32_32x32x16_bf16:
+// six MFMAs per fp32 product block, smallest terms first, S^T and O^T accumulated in fp32; the
+// softmax is the fp32 kernel's (running maximum, P and row sums in fp32; P is split like the
+// other operands). Each S takes 6 kD / 16 rounded accumulations and O^T 24 per 64 keys, where
+// the fp32 MFMA's fmaf chains take kD and 64.
+//   kKW = 1: four waves of a workgroup own four units (query blocks or halves);
+//   kKW = 4: they share one unit, wave w taking list positions w, w + 4, ..., and merge their
+//     partials through LDS: for launches too small to fill the card otherwise.
+// Bound: the matrix core (192 MFMAs, 6 144 cycles per 64 x 64 tile at head dim 64, against 512
+// and 16 384 in fp32). Q's hi terms stay in registers, mid and lo in LDS (16 KB per wave), K and
+// V operands are loaded straight from the split planes, kRing groups ahead, so two waves fit a
+// SIMD and one's softmax runs beside the other's MFMAs. Measured, splitting included: [2, 30,
+// 17776, 64] with a fifth of the blocks 9.61 -> 5.24 ms (1 130 TFLOP/s of bf16 products; the
+// MFMA pipes busy 69 % at a power-limited 1.54 GHz, the largest bf16 matrix products on the card
+// reach 1 380), the same at head dim 128 with 15 heads 11.9 -> 7.8 ms (there a wave's 32 rows
+// load each operand for half the MFMAs, 64 bytes per cycle and CU, the vector cache's rate), and
+// [1, 2, 2048, 64] with a quarter of the blocks 153 -> 37 us. Error against a 64-bit softmax 9.6e-7
+// where the fp32 MFMA's was 1.1e-6 (2-norm, relative).
+template <int kD, int kPool, int kKW>
+__global__ __launch_bounds__(256, 2) void bsa_fwd_f32_terms_kernel(F32Args a) {
+  static_assert(kD == 64 || kD == 128, "head dim 64 or 128");
+  static_assert(kPool == 0 || kPool == 32 || kPool == 64, "pooling columns of 32 or 64 keys");
+  static_assert(kKW == 1 || kKW == 4, "waves per unit");
+  typedef TermLayout<kD> Lay;
+  constexpr int kG = kD == 64 ? 2 : 1;   // 32-row query groups per wave
+  constexpr int kHalvesQ = 2 / kG;       // units per query block
+  constexpr int kRows = 32 * kG;
+  constexpr int kDS = kD / 16, kDC = kD / 32;
+  constexpr int kNG = Lay::kGroups;
+  constexpr int kRing = 2;  // operand groups in registers (a deeper ring spills at head dim 128)
+  static_assert(kNG % kRing == 0, "the ring's slots are static");
+  constexpr int kUnitsWg = 4 / kKW;
+  constexpr int kWgs = 4 * kHalvesQ / kUnitsWg;  // workgroups per dispatch group (4 slots)
+  // Per wave: Q mid and lo operands, [term][g][s] of 1 KB; later its partial [kRows][kD].
+  __shared__ __attribute__((aligned(1024))) f32_u32x4 q_lds[4][2 * kG * kDS * 64];
+  __shared__ float ml_lds[kKW == 4 ? 4 : 1][2][kRows];
+  static_assert(sizeof(q_lds[0]) == kRows * kD * sizeof(float), "a partial fits the Q operands' space");
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 31, hh = lane >> 5;
+  // Dispatch group w (four slots of the work order) stays on XCD w % 8.
+  const int x = blockIdx.x;
+  const int w8 = 8 * (x / (8 * kWgs)) + (x & 7);
+  const int unit = 4 * kHalvesQ * w8 + ((x >> 3) % kWgs) * kUnitsWg + (kKW == 1 ? wave : 0);
+  const int slot = unit / kHalvesQ;
+  if (slot >= a.n_slots) return;  // kKW = 4: the same for every wave of the workgroup
+  const int item = __builtin_amdgcn_readfirstlane(a.order ? a.order[slot] : slot);
+  if (item < 0 || item >= a.n_items) return;
+  const int row0 = (unit % kHalvesQ) * kRows;
+  const int bh = item / a.nqb;
+  const int qb = item - bh * a.nqb;
+  const int b = bh / a.H;
+  const int h = bh - b * a.H;
+  const int hk = a.kv_rep > 1 ? h / a.kv_rep : h;
+  const int bhk = b * (a.H / a.kv_rep) + hk;
+  const int it0 = kKW == 1 ? 0 : wave;
+
+  const int64_t list_row = (int64_t)bh * a.list_bh_stride + qb;
+  int cnt = a.kv_cnt[list_row];
+  cnt = cnt < 0 ? 0 : (cnt > a.max_cnt ? a.max_cnt : cnt);
+  const __attribute__((address_space(4))) int32_t* list =
+      (const __attribute__((address_space(4))) int32_t*)(a.kv_idx + list_row * a.max_cnt);
+
+  const uint4* fl = a.flags + (int64_t)bhk * a.nkb;
+  f32_u32x4 qhi[kG][kDS];
+  f32_u32x4* ql = q_lds[wave];
+  bool use_terms = (uint32_t)__builtin_amdgcn_readfirstlane((int)fl[0].x) != kTermSkip;
+  if (use_terms) {
+    // The head's largest |k| and |v| and this wave's largest |q|.
+    uint32_t kmax = 0u, vmax = 0u;
+    for (int j = 0; j < a.nkb; j += 64) {
+      const uint4 f = fl[min(j + lane, a.nkb - 1)];
+      kmax = max(kmax, max(f.x, f.y));
+      vmax = max(vmax, max(f.z, f.w));
+    }
+#pragma unroll
+    for (int g = 0; g < kG; ++g) {
+      const int row = min(qb * kBlk + row0 + 32 * g + col, a.Lq - 1);  // clamped rows are never stored
+      const float* p = a.q + b * a.q_sb + h * a.q_sh + (int64_t)row * a.q_sl + 8 * hh;
+#pragma unroll
+      for (int s = 0; s < kDS; ++s) {
+        const float4 x0 = *reinterpret_cast<const float4*>(p + 16 * s);
+        const float4 x1 = *reinterpret_cast<const float4*>(p + 16 * s + 4);
+        const float y[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+        f32_u32x4 mid, lo;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          uint32_t t0, t1, t2;
+          split3(y[2 * i], y[2 * i + 1], t0, t1, t2);
+          qhi[g][s][i] = t0;
+          mid[i] = t1;
+          lo[i] = t2;
+          kmax = max(kmax, max(abs_bits(y[2 * i]), abs_bits(y[2 * i + 1])));
+        }
+        ql[(g * kDS + s) * 64 + lane] = mid;
+        ql[((kG + g) * kDS + s) * 64 + lane] = lo;
+      }
+    }
+    kmax = wave_max_u(kmax);
+    vmax = wave_max_u(vmax);
+    use_terms = __builtin_amdgcn_readfirstlane(kmax < kTermMax && vmax < kTermMax &&
+                                               (vmax >= kTermMin || vmax == 0u));
+  }
+
+  float* part = reinterpret_cast<float*>(q_lds[wave]);  // kKW = 4: [row][16-byte chunk ^ row % 16]
+  if (!use_terms) {
+    // In passes of 16 kJ rows, which fit beside this kernel's registers.
+    constexpr int kJ = 2;
+    for (int r0 = 0; r0 < kRows; r0 += 16 * kJ) {
+      sa_f32x4 acc[kD / 16][kJ];
+      float m[kJ], l[kJ];
+      f32_rows<kD, kPool, kJ>(a, bh, qb, row0 + r0, it0, kKW, lane, acc, m, l);
+      if constexpr (kKW == 1) {
+        f32_store<kD, kPool, kJ>(a, bh, qb, row0 + r0, lane, acc, m, l);
+      } else {
+        const int r = lane & 15, g = lane >> 4;
+#pragma unroll
+        for (int j = 0; j < kJ; ++j) {
+          const int row = r0 + 16 * j + r;
+          const float l_tot = slot_sum(l[j]);
+#pragma unroll
+          for (int dblk = 0; dblk < kD / 16; ++dblk)
+            *reinterpret_cast<sa_f32x4*>(part + row * kD + 4 * ((4 * dblk + g) ^ (row & 15))) = acc[dblk][j];
+          if (g == 0) {
+            ml_lds[wave][0][row] = m[j];
+            ml_lds[wave][1][row] = l_tot;
+          }
+        }
+      }
+    }
+  } else {
+    sa_f32x16 acc[kDC][kG];
+    float m[kG], l[kG];
+#pragma unroll
+    for (int g = 0; g < kG; ++g) {
+      m[g] = -INFINITY;
+      l[g] = 0.f;
+#pragma unroll
+      for (int dc = 0; dc < kDC; ++dc) acc[dc][g] = sa_f32x16{};
+    }
+    const uint8_t* head = a.planes + (int64_t)bhk * a.nkb * Lay::kTile;
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(head), (short)0, (int)((uint32_t)a.nkb * Lay::kTile), 0x00020000);
+    f32_u32x4 ring[kRing][6];
+    auto load_group = [&](f32_u32x4 (&r)[6], uint32_t off) __attribute__((always_inline)) {
+#pragma unroll
+      for (int o = 0; o < 6; ++o)
+        r[o] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, 16 * lane + 1024 * (o & 3), off + 4096 * (o >> 2), 0);
+    };
+    auto tile_off = [&](int kb) -> uint32_t {  // an entry outside the grid reads block 0 (masked out)
+      return __builtin_amdgcn_readfirstlane(((unsigned)kb < (unsigned)a.nkb ? (uint32_t)kb : 0u) * Lay::kTile);
+    };
+    int kb = it0 < cnt ? list[it0] : 0;
+    uint32_t off = tile_off(kb);
+    if (it0 < cnt) {
+#pragma unroll
+      for (int i = 0; i < kRing; ++i) load_group(ring[i], off + i * Lay::kGroup);
+    }
+    for (int it = it0; it < cnt; it += kKW) {
+      // Past the end the prefetch re-reads the current tile.
+      const int kb_next = it + kKW < cnt ? list[it + kKW] : kb;
+      const uint32_t off_next = tile_off(kb_next);
+      const bool ok = (unsigned)kb < (unsigned)a.nkb;
+      const int nvalid = ok ? min(kBlk, a.Lk - kb * kBlk) : 0;
+      const bool diag = kPool != 0 && a.causal && kb == qb;
+      float pmax[kG];
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        // ---- S^T: S[g] element e is key 32 c + 8 (e / 4) + 4 hh + e % 4, row 32 g + col.
+        sa_f32x16 S[kG];
+#pragma unroll
+        for (int g = 0; g < kG; ++g) S[g] = sa_f32x16{};
+#pragma unroll
+        for (int i = 0; i < Lay::kKGroups; ++i) {
+          f32_u32x4(&r)[6] = ring[i % kRing];
+#pragma unroll
+          for (int s2 = 0; s2 < 2; ++s2) {
+            const int s = 2 * i + s2;
+            asm volatile("" ::: "memory");  // the LDS operands are read here, not kept in registers
+            f32_u32x4 qm[kG], qo[kG];
+#pragma unroll
+            for (int g = 0; g < kG; ++g) {
+              qm[g] = ql[(g * kDS + s) * 64 + lane];
+              qo[g] = ql[((kG + g) * kDS + s) * 64 + lane];
+            }
+            const f32_u32x4 khi = r[3 * s2], kmid = r[3 * s2 + 1], klo = r[3 * s2 + 2];
+#pragma unroll
+            for (int g = 0; g < kG; ++g) S[g] = mfma_bf16(klo, qhi[g][s], S[g]);
+#pragma unroll
+            for (int g = 0; g < kG; ++g) S[g] = mfma_bf16(kmid, qm[g], S[g]);
+#pragma unroll
+            for (int g = 0; g < kG; ++g) S[g] = mfma_bf16(khi, qo[g], S[g]);
+#pragma unroll
+            for (int g = 0; g < kG; ++g) S[g] = mfma_bf16(kmid, qhi[g][s], S[g]);
+#pragma unroll
+            for (int g = 0; g < kG; ++g) S[g] = mfma_bf16(khi, qm[g], S[g]);
+#pragma unroll
+            for (int g = 0; g < kG; ++g) S[g] = mfma_bf16(khi, qhi[g][s], S[g]);
+          }
+          const int next = c * kNG + i + kRing;  // (never past this tile: K groups come first)
+          load_group(r, off + next * Lay::kGroup);
+          __builtin_amdgcn_sched_barrier(0x38f);  // loads stay where they are issued
+        }
+        // ---- Masks, pooled column maxima, running maximum, P = exp2(S * sc - m), row sums.
+        if (nvalid < kBlk || diag) {
+#pragma unroll
+          for (int g = 0; g < kG; ++g)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+              const int kk = 32 * c + 8 * (e >> 2) + 4 * hh + (e & 3);
+              if (kk >= nvalid || (diag && kk > row0 + 32 * g + col)) S[g][e] = -INFINITY;
+            }
+        }
+        float cand[kG];
+        bool raise = false;
+#pragma unroll
+        for (int g = 0; g < kG; ++g) {
+          float mx = fmaxf(S[g][0], S[g][1]);
+#pragma unroll
+          for (int e = 2; e < 16; e += 2) mx = fmaxf(fmaxf(mx, S[g][e]), S[g][e + 1]);
+          cand[g] = half_max(mx) * a.scale_log2;  // scale > 0
+          raise |= cand[g] > m[g];
+        }
+        if constexpr (kPool != 0) {
+          // Lane l stores row l of the block (kG = 2), or lanes hh = 0 their unit's rows.
+          const int cc = kPool == 32 ? c : 0;
+#pragma unroll
+          for (int g = 0; g < kG; ++g) pmax[g] = (kPool == 32 || c == 0) ? cand[g] : fmaxf(pmax[g], cand[g]);
+          if (ok && (kPool == 32 || c == 1)) {
+            constexpr int kCols = kBlk / kPool;
+            float* rp = a.pool_r + (((int64_t)bh * a.nqb + qb) * a.pool_ncol + kb * kCols + cc) * kBlk + row0;
+            if (kG == 2) rp[lane] = hh ? pmax[kG - 1] : pmax[0];
+            else if (hh == 0) rp[col] = pmax[0];
+          }
+        }
+        if (__ballot(raise) != 0) {
+#pragma unroll
+          for (int g = 0; g < kG; ++g) {
+            const float m_new = fmaxf(m[g], cand[g]);
+            const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m[g] - m_new);
+            m[g] = m_new;
+            l[g] *= alpha;
+#pragma unroll
+            for (int dc = 0; dc < kDC; ++dc) acc[dc][g] *= alpha;
+          }
+        }
+#pragma unroll
+        for (int g = 0; g < kG; ++g) {
+          const float mu = m[g] == -INFINITY ? 0.f : m[g];
+          float sum = 0.f;
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            const float p = __builtin_amdgcn_exp2f(fmaf(S[g][e], a.scale_log2, -mu));  // -inf -> 0
+            S[g][e] = p;
+            sum += p;
+          }
+          l[g] += sum;
+        }
+        // ---- O^T += V^T P^T over the chunk's two 16-key steps.
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          f32_u32x4 P[kG][3];
+#pragma unroll
+          for (int g = 0; g < kG; ++g)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              uint32_t t0, t1, t2;
+              split3(S[g][8 * u + 2 * i], S[g][8 * u + 2 * i + 1], t0, t1, t2);
+              P[g][0][i] = t0;
+              P[g][1][i] = t1;
+              P[g][2][i] = t2;
+            }
+#pragma unroll
+          for (int dp = 0; dp < kDC / 2; ++dp) {
+            const int i = Lay::kKGroups + u * (kDC / 2) + dp;
+            f32_u32x4(&r)[6] = ring[i % kRing];
+#pragma unroll
+            for (int d2 = 0; d2 < 2; ++d2) {
+              const int dc = 2 * dp + d2;
+              const f32_u32x4 vhi = r[3 * d2], vmid = r[3 * d2 + 1], vlo = r[3 * d2 + 2];
+#pragma unroll
+              for (int g = 0; g < kG; ++g) acc[dc][g] = mfma_bf16(vlo, P[g][0], acc[dc][g]);
+#pragma unroll
+              for (int g = 0; g < kG; ++g) acc[dc][g] = mfma_bf16(vmid, P[g][1], acc[dc][g]);
+#pragma unroll
+              for (int g = 0; g < kG; ++g) acc[dc][g] = mfma_bf16(vhi, P[g][2], acc[dc][g]);
+#pragma unroll
+              for (int g = 0; g < kG; ++g) acc[dc][g] = mfma_bf16(vmid, P[g][0], acc[dc][g]);
+#pragma unroll
+              for (int g = 0; g < kG; ++g) acc[dc][g] = mfma_bf16(vhi, P[g][1], acc[dc][g]);
+#pragma unroll
+              for (int g = 0; g < kG; ++g) acc[dc][g] = mfma_bf16(vhi, P[g][0], acc[dc][g]);
+            }
+            const int next = c * kNG + i + kRing;
+            load_group(r, next < 2 * kNG ? off + next * Lay::kGroup : off_next + (next - 2 * kNG) * Lay::kGroup);
+            __builtin_amdgcn_sched_barrier(0x38f);
+          }
+        }
+      }
+      kb = kb_next;
+      off = off_next;
+    }
+    // ---- Epilogue: element 4 q4 + j of acc[dc][g] is d = 32 dc + 8 q4 + 4 hh + j.
+#pragma unroll
+    for (int g = 0; g < kG; ++g) {
+      const float l_tot = half_sum(l[g]);
+      const int lrow = 32 * g + col;
+      if constexpr (kKW == 1) {
+        const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+        const int row = qb * kBlk + row0 + lrow;
+        if constexpr (kPool != 0) {
+          if (hh == 0) a.pool_lse[(int64_t)bh * a.pool_lpad + row] = (m[g] == -INFINITY ? 0.f : m[g]) + log2f(l_tot);
+        }
+        if (row < a.Lq) {
+          float* orow = a.o + b * a.o_sb + h * a.o_sh + (int64_t)row * a.o_sl;
+#pragma unroll
+          for (int dc = 0; dc < kDC; ++dc)
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4) {
+              const sa_f32x16& A = acc[dc][g];
+              *reinterpret_cast<float4*>(orow + 32 * dc + 8 * q4 + 4 * hh) =
+                  make_float4(A[4 * q4] * inv, A[4 * q4 + 1] * inv, A[4 * q4 + 2] * inv, A[4 * q4 + 3] * inv);
+            }
+        }
+      } else {
+#pragma unroll
+        for (int dc = 0; dc < kDC; ++dc)
+#pragma unroll
+          for (int q4 = 0; q4 < 4; ++q4) {
+            const sa_f32x16& A = acc[dc][g];
+            *reinterpret_cast<sa_f32x4*>(part + lrow * kD + 4 * ((8 * dc + 2 * q4 + hh) ^ (lrow & 15))) =
+                sa_f32x4{A[4 * q4], A[4 * q4 + 1], A[4 * q4 + 2], A[4 * q4 + 3]};
+          }
+        if (hh == 0) {
+          ml_lds[wave][0][lrow] = m[g];
+          ml_lds[wave][1][lrow] = l_tot;
+        }
+      }
+    }
+  }
+  if constexpr (kKW == 4) {
+    // Merge in wave order: out = sum_w 2^(m_w - M) acc_w / sum_w 2^(m_w - M) l_w.
+    __syncthreads();
+    constexpr int kChunks = kD / 4;
+    for (int t = threadIdx.x; t < kRows * kChunks; t += 256) {
+      const int lrow = t / kChunks, ch = t % kChunks;
+      float M = -INFINITY;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) M = fmaxf(M, ml_lds[w][0][lrow]);
+      float L = 0.f;
+      sa_f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const float mw = ml_lds[w][0][lrow];
+        const float f = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - M);  // no key of this row: nothing
+        const sa_f32x4 p = *reinterpret_cast<const sa_f32x4*>(
+            reinterpret_cast<const float*>(q_lds[w]) + lrow * kD + 4 * (ch ^ (lrow & 15)));
+        L += f * ml_lds[w][1][lrow];
+        o += f * p;
+      }
+      const float inv = L > 0.f ? 1.f / L : 0.f;
+      const int row = qb * kBlk + row0 + lrow;
+      if constexpr (kPool != 0) {
+        if (ch == 0) a.pool_lse[(int64_t)bh * a.pool_lpad + row] = (M == -INFINITY ? 0.f : M) + log2f(L);
+      }
+      if (row < a.Lq) {
+        float* orow = a.o + b * a.o_sb + h * a.o_sh + (int64_t)row * a.o_sl;
+        *reinterpret_cast<float4*>(orow + 4 * ch) = make_float4(o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv);
       }
     }
   }
@@ -262,11 +826,64 @@ __global__ __launch_bounds__(64 * kWavesF32, kD == 64 ? 2 : 1) void bsa_fwd_f32_
 
 namespace {
 
+int64_t terms_blocks(int B, int Hk, int Lk) { return (int64_t)B * Hk * sa::cdiv(Lk, kBlk); }
+
+template <int kD, int kPool>
+void launch_terms_pool(const F32Args& a, hipStream_t s) {
+  // Up to three rounds of the card's 2 048 waves, four waves share each unit (64 query rows, 32
+  // at head dim 128); measured, one wave against four per unit: 64 units 78 / 43 us, 504 154 / 84,
+  // 2 400 361 / 310, 5 640 717 / 690 (head dim 128: 784 / 771), 7 500 729 / 733, and 16 680 with
+  // few tiles each 1 241 / 1 354.
+  constexpr int64_t kSharedUnits = 6144;
+  constexpr int kHalvesQ = kD == 64 ? 1 : 2;
+  const int64_t groups = (a.n_slots + 3) / 4;
+  const bool shared = (int64_t)a.n_items * kHalvesQ <= kSharedUnits;
+  const int64_t wgs = shared ? 4 * kHalvesQ : kHalvesQ;  // workgroups per dispatch group
+  const dim3 grid((unsigned)((groups + 7) / 8 * 8 * wgs)), blk(256);
+  if (shared) hipLaunchKernelGGL((bsa_fwd_f32_terms_kernel<kD, kPool, 4>), grid, blk, 0, s, a);
+  else hipLaunchKernelGGL((bsa_fwd_f32_terms_kernel<kD, kPool, 1>), grid, blk, 0, s, a);
+}
+
+template <int kD>
+int launch_terms(F32Args& a, int B, void* ws, int pool_cols, void* stream, const char* fn) {
+  const int Hk = a.H / a.kv_rep;
+  const int64_t blocks = terms_blocks(B, Hk, a.Lk);
+  TermArgs t;
+  t.k = a.k; t.v = a.v;
+  t.k_sb = a.k_sb; t.k_sh = a.k_sh; t.k_sl = a.k_sl;
+  t.v_sb = a.v_sb; t.v_sh = a.v_sh; t.v_sl = a.v_sl;
+  t.Hk = Hk; t.Lk = a.Lk; t.nkb = a.nkb;
+  t.kv_cnt = a.list_bh_stride ? a.kv_cnt : nullptr;  // lists shared by the heads are dense
+  t.nqb = a.nqb; t.max_cnt = a.max_cnt;
+  t.planes = static_cast<uint8_t*>(ws);
+  t.flags = reinterpret_cast<uint32_t*>(t.planes + blocks * TermLayout<kD>::kTile);
+  hipStream_t s = sa::as_stream(stream);
+  hipLaunchKernelGGL(f32_terms_kernel<kD>, dim3((unsigned)blocks), dim3(256), 0, s, t);
+  if (int rc = sa::check_launch(fn)) return rc;
+  a.planes = t.planes;
+  a.flags = reinterpret_cast<const uint4*>(t.flags);
+  if (pool_cols == 32) launch_terms_pool<kD, 32>(a, s);
+  else if (pool_cols == 64) launch_terms_pool<kD, 64>(a, s);
+  else launch_terms_pool<kD, 0>(a, s);
+  return sa::check_launch(fn);
+}
+
+// Checks a terms workspace; blocks of one head are addressed with 32-bit offsets.
+int check_terms(int B, int Hk, int Lk, int D, const void* ws, int64_t ws_bytes, const char* fn) {
+  SA_REQUIRE(ws, "%s: null workspace", fn);
+  SA_REQUIRE(reinterpret_cast<uintptr_t>(ws) % 256 == 0, "%s: workspace not 256-byte aligned", fn);
+  const int64_t need = sa::attn_f32_terms_bytes(B, Hk, Lk, D);
+  SA_REQUIRE(ws_bytes >= need, "%s: workspace of %lld bytes < %lld", fn, (long long)ws_bytes, (long long)need);
+  if ((int64_t)sa::cdiv(Lk, kBlk) * 768 * D > 0x7fffffffLL || terms_blocks(B, Hk, Lk) >= (1LL << 31))
+    return sa::fail(SA_ERR_UNSUPPORTED, "%s: Lk=%d too long for the split operands", fn, Lk);
+  return SA_OK;
+}
+
 int launch_f32(const float* q, const int64_t q_strides[3], const float* k, const int64_t k_strides[3],
                const float* v, const int64_t v_strides[3], float* out, const int64_t out_strides[3], int B, int H,
                int Lq, int Lk, int D, const int32_t* kv_idx, const int32_t* kv_cnt, int max_cnt, bool lists_shared,
                float sm_scale, const int32_t* work_order, int64_t n_slots, int kv_rep, bool causal, int pool_cols,
-               float* pool_r, float* pool_lse, void* stream, const char* fn) {
+               float* pool_r, float* pool_lse, void* terms_ws, void* stream, const char* fn) {
   SA_REQUIRE(q && k && v && out && q_strides && k_strides && v_strides && out_strides && kv_idx && kv_cnt,
              "%s: null pointer", fn);
   SA_REQUIRE(B > 0 && H > 0 && Lq > 0 && Lk > 0, "%s: bad shape B=%d H=%d Lq=%d Lk=%d", fn, B, H, Lq, Lk);
@@ -312,6 +929,8 @@ int launch_f32(const float* q, const int64_t q_strides[3], const float* k, const
   a.pool_lse = pool_lse;
   a.pool_lpad = nqb * kBlk;
   SA_REQUIRE(pool_cols == 0 || (pool_r && pool_lse), "%s: pooling needs its buffers", fn);
+  if (terms_ws) return D == 64 ? launch_terms<64>(a, B, terms_ws, pool_cols, stream, fn)
+                               : launch_terms<128>(a, B, terms_ws, pool_cols, stream, fn);
   const dim3 grid((unsigned)(n_slots / kWavesF32)), blk(64 * kWavesF32);
   hipStream_t s = sa::as_stream(stream);
   if (D == 64) {
@@ -329,14 +948,17 @@ int launch_f32(const float* q, const int64_t q_strides[3], const float* k, const
 }  // namespace
 
 namespace sa {
+int64_t attn_f32_terms_bytes(int B, int Hk, int Lk, int D) { return terms_blocks(B, Hk, Lk) * (768LL * D + 16); }
+
 // fp32 attention in pooling mode for the pooled-map entry point (attn_fwd.hip).
 int attn_f32_pooling(const float* q, const int64_t q_strides[3], const float* k, const int64_t k_strides[3],
                      const float* v, const int64_t v_strides[3], float* out, const int64_t out_strides[3], int B,
                      int H, int L, int D, const int32_t* kv_idx, const int32_t* kv_cnt, int max_cnt, int kv_rep,
-                     bool causal, float sm_scale, int pool_cols, float* pool_r, float* pool_lse, void* stream,
-                     const char* fn) {
+                     bool causal, float sm_scale, int pool_cols, float* pool_r, float* pool_lse, void* terms_ws,
+                     void* stream, const char* fn) {
   return launch_f32(q, q_strides, k, k_strides, v, v_strides, out, out_strides, B, H, L, L, D, kv_idx, kv_cnt,
-                    max_cnt, true, sm_scale, nullptr, 0, kv_rep, causal, pool_cols, pool_r, pool_lse, stream, fn);
+                    max_cnt, true, sm_scale, nullptr, 0, kv_rep, causal, pool_cols, pool_r, pool_lse, terms_ws, stream,
+                    fn);
 }
 }  // namespace sa
 
@@ -350,5 +972,28 @@ extern "C" int sa_block_sparse_fwd_f32(const float* q, const int64_t q_strides[3
   (void)bias_strides;
   if (key_bias) return sa::fail(SA_ERR_UNSUPPORTED, "%s: key_bias (bf16 and fp16 only)", fn);
   return launch_f32(q, q_strides, k, k_strides, v, v_strides, out, out_strides, B, H, Lq, Lk, D, kv_idx, kv_cnt,
-                    max_cnt, false, sm_scale, work_order, n_slots, 1, false, 0, nullptr, nullptr, stream, fn);
+                    max_cnt, false, sm_scale, work_order, n_slots, 1, false, 0, nullptr, nullptr, nullptr, stream, fn);
+}
+
+extern "C" int sa_block_sparse_fwd_f32_terms_workspace(int B, int H, int Lk, int D, int64_t* bytes) {
+  const char* fn = "sa_block_sparse_fwd_f32_terms_workspace";
+  SA_REQUIRE(bytes, "%s: null bytes", fn);
+  SA_REQUIRE(B > 0 && H > 0 && Lk > 0, "%s: bad shape B=%d H=%d Lk=%d", fn, B, H, Lk);
+  if (D != 64 && D != 128) return sa::fail(SA_ERR_UNSUPPORTED, "%s: head_dim %d (64 or 128)", fn, D);
+  *bytes = sa::attn_f32_terms_bytes(B, H, Lk, D);
+  return sa::ok();
+}
+
+extern "C" int sa_block_sparse_fwd_f32_terms(const float* q, const int64_t q_strides[3], const float* k,
+                                             const int64_t k_strides[3], const float* v, const int64_t v_strides[3],
+                                             float* out, const int64_t out_strides[3], int B, int H, int Lq, int Lk,
+                                             int D, const int32_t* kv_idx, const int32_t* kv_cnt, int max_cnt,
+                                             float sm_scale, const int32_t* work_order, int64_t n_slots,
+                                             void* workspace, int64_t workspace_bytes, void* stream) {
+  const char* fn = "sa_block_sparse_fwd_f32_terms";
+  SA_REQUIRE(B > 0 && H > 0 && Lk > 0, "%s: bad shape B=%d H=%d Lk=%d", fn, B, H, Lk);
+  if (D != 64 && D != 128) return sa::fail(SA_ERR_UNSUPPORTED, "%s: head_dim %d (64 or 128)", fn, D);
+  if (int rc = check_terms(B, H, Lk, D, workspace, workspace_bytes, fn)) return rc;
+  return launch_f32(q, q_strides, k, k_strides, v, v_strides, out, out_strides, B, H, Lq, Lk, D, kv_idx, kv_cnt,
+                    max_cnt, false, sm_scale, work_order, n_slots, 1, false, 0, nullptr, nullptr, workspace, stream, fn);
 }

@@ -2224,7 +2224,7 @@ int attn_pooling_f32(const float* q, const int64_t q_strides[3], const float* k,
   float* r = reinterpret_cast<float*>(ws + p.r);
   float* lse = reinterpret_cast<float*>(ws + p.lse);
   if (int rc = sa::attn_f32_pooling(q, q_strides, k, k_strides, v, v_strides, out, out_strides, B, H, L, D, la.idx,
-                                    la.cnt, p.nkb, H / H_kv, causal != 0, sm_scale, p.G, r, lse, stream, fn))
+                                    la.cnt, p.nkb, H / H_kv, causal != 0, sm_scale, p.G, r, lse, nullptr, stream, fn))
     return rc;
   return launch_pool_reduce(p, r, lse, B, H, L, block_size, causal, po, po_strides, s, fn);
 }

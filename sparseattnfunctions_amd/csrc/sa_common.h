@@ -59,8 +59,10 @@ inline int64_t k16_ws_bytes_bias(int B, int H, int Lk) { return k16_bias_offset(
 int attn_f32_pooling(const float* q, const int64_t q_strides[3], const float* k, const int64_t k_strides[3],
                      const float* v, const int64_t v_strides[3], float* out, const int64_t out_strides[3], int B,
                      int H, int L, int D, const int32_t* kv_idx, const int32_t* kv_cnt, int max_cnt, int kv_rep,
-                     bool causal, float sm_scale, int pool_cols, float* pool_r, float* pool_lse, void* stream,
-                     const char* fn);
+                     bool causal, float sm_scale, int pool_cols, float* pool_r, float* pool_lse, void* terms_ws,
+                     void* stream, const char* fn);
+// Bytes of the split-operand workspace of the fp32 attention (attn_f32.hip).
+int64_t attn_f32_terms_bytes(int B, int Hk, int Lk, int D);
 
 }  // namespace sa
 

@@ -13,8 +13,9 @@ libsa_hip.so (`sa_mask_to_kv_list` + `sa_block_sparse_fwd`), not Triton.
 
 Inputs are bf16 or fp16 (all three the same), head_dim 64 or 128 as the reference asserts
 (:231); P is rounded to the input dtype before P.V as the reference rounds it to v's (:107).
-fp32 inputs run the fp32 kernel (`sa_block_sparse_fwd_f32`: fp32 MFMA, P kept in fp32, as the
-reference's cast to v's dtype leaves it), head_dim 64 or 128.
+fp32 inputs run the fp32 kernels (P kept in fp32, as the reference's cast to v's dtype leaves
+it), head_dim 64 or 128: `sa_block_sparse_fwd_f32_terms` (each operand split exactly into three
+bf16 terms, fp32 accumulation) or, for a few query blocks, `sa_block_sparse_fwd_f32` (fp32 MFMA).
 
 Differences from the reference, by design:
   * a query block whose mask row is empty yields 0 instead of NaN (:201-203);
@@ -120,6 +121,27 @@ def prepare_fp16_keys(k: torch.Tensor) -> Optional[FP16Keys]:
     return FP16Keys(k_in, ws, stream, event)
 
 
+# fp32 launches of at least this many query blocks run on split bf16 operands. Splitting k and v
+# is one launch more (37 -> 41 us a call where the host bounds it) and pays from two listed tiles
+# per key block, which the library counts per head: 16 blocks of a tenth of the keys each take
+# 66 -> 42 us a call, two heads of 32 blocks with a quarter 159 -> 37 us.
+F32_TERMS_BLOCKS = 8
+
+
+def f32_terms_workspace(B: int, H: int, Lk: int, D: int, device):
+    """Workspace of `sa_block_sparse_fwd_f32_terms`, or None where the fp32 kernel runs without
+    one: keys of one head past its 32-bit offsets, or no memory for it (12 D bytes per key)."""
+    n = ctypes.c_int64(0)
+    _lib.check(_lib.load().sa_block_sparse_fwd_f32_terms_workspace(int(B), int(H), int(Lk), int(D), ctypes.byref(n)),
+               "sa_block_sparse_fwd_f32_terms_workspace")
+    if n.value // (B * H) >= 1 << 31:
+        return None
+    try:
+        return torch.empty(n.value, dtype=torch.uint8, device=device)
+    except torch.cuda.OutOfMemoryError:
+        return None
+
+
 _ORDER_CACHE = {}
 
 
@@ -153,7 +175,7 @@ def block_sparse_attention(q, k, v, kv: KVList, sm_scale: float, key_bias=None, 
     """out = block-sparse softmax(q k^T * sm_scale [+ key_bias]) v over the blocks of `kv`.
 
     q [B,H,Lq,D], k/v [B,H,Lk,D] on the GPU, bf16 or fp16 (one dtype), D = 64 or 128, or fp32
-    (plain lists only: fp32 MFMA, P kept in fp32 as the reference's kernel does);
+    (plain lists only: fp32 arithmetic, P kept in fp32 as the reference's kernel does);
     key_bias optional fp32 [B,H,Lk] (any strides with a contiguous key axis, stride 0 to
     broadcast). `n_text_blocks` only affects scheduling (those block rows are dispatched
     first).
@@ -295,6 +317,17 @@ def block_sparse_attention(q, k, v, kv: KVList, sm_scale: float, key_bias=None, 
                 stream.cuda_stream)
         _lib.check(rc, "sa_block_sparse_fwd_k16")
         return out
+    if fp32 and nqb >= F32_TERMS_BLOCKS:
+        ws = f32_terms_workspace(B, H, Lk, D, q.device)
+        if ws is not None:
+            with torch.cuda.device(q.device):
+                rc = lib.sa_block_sparse_fwd_f32_terms(
+                    q.data_ptr(), _lib.i64(*q.stride()[:3]), k.data_ptr(), _lib.i64(*k.stride()[:3]),
+                    v.data_ptr(), _lib.i64(*v.stride()[:3]), out.data_ptr(), _lib.i64(*out.stride()[:3]),
+                    B, H, Lq, Lk, D, kv.idx.data_ptr(), kv.cnt.data_ptr(), kv.max_cnt, float(sm_scale),
+                    order.data_ptr(), order.numel(), ws.data_ptr(), ws.numel(), _lib.stream_of(q))
+            _lib.check(rc, "sa_block_sparse_fwd_f32_terms")
+            return out
     fn = "sa_block_sparse_fwd_f16" if fp16 else ("sa_block_sparse_fwd_f32" if fp32 else "sa_block_sparse_fwd")
     with torch.cuda.device(q.device):
         rc = getattr(lib, fn)(

@@ -1,0 +1,101 @@
+"""fp32 attention on split bf16 operands (`sa_block_sparse_fwd_f32_terms`): edges of its tiles,
+units and rules, against the fp64 oracle and the fp32 kernel without a workspace."""
+import math
+
+import pytest
+import torch
+
+from oracle.attention import masked_attention
+from sparseattnfunctions_amd._kv import kv_list_from_mask
+from sparseattnfunctions_amd.utils import block_sparse_attn_kernel as bsk
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def dev():
+    return torch.device("cuda:0")
+
+
+def _plain(monkeypatch, *args):
+    """The same call through `sa_block_sparse_fwd_f32`."""
+    with monkeypatch.context() as m:
+        m.setattr(bsk, "F32_TERMS_BLOCKS", 1 << 30)
+        return bsk.block_sparse_attention(*args)
+
+
+def _lists(B, H, Lq, Lk, keep, seed, dev):
+    nqb, nkb = math.ceil(Lq / 64), math.ceil(Lk / 64)
+    mask = torch.rand(B, H, nqb, nkb, generator=torch.Generator().manual_seed(seed)) < keep
+    mask[..., 0] = True
+    return mask, kv_list_from_mask(mask.to(dev), B, H, nqb, nkb)
+
+
+def _rand(seed, *shape):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed))
+
+
+# Units shared by four waves and units of one wave (more than 6 144 of them), partial first and
+# last tiles, lists shorter than the four waves.
+@pytest.mark.parametrize("B,H,Lq,Lk,D,keep", [
+    (1, 1, 512, 512, 64, 1.0), (2, 3, 449, 321, 64, 0.9), (1, 2, 1000, 65, 64, 1.0), (1, 1, 2049, 2047, 64, 0.4),
+    (1, 40, 9900, 700, 64, 0.7), (1, 2, 450, 1001, 128, 0.6), (1, 40, 5000, 450, 128, 0.8),
+])
+def test_errors_no_larger_than_the_fp32_kernels(dev, monkeypatch, B, H, Lq, Lk, D, keep):
+    print(f"case terms {B} {H} {Lq} {Lk} {D} {keep}", flush=True)
+    q, k, v = _rand(1, B, H, Lq, D), _rand(2, B, H, Lk, D), _rand(3, B, H, Lk, D)
+    mask, kv = _lists(B, H, Lq, Lk, keep, Lq + Lk, dev)
+    args = (q.to(dev), k.to(dev), v.to(dev), kv, 1 / math.sqrt(D))
+    heads = [(b, h) for b in range(B) for h in range(0, H, 13)]
+    want = masked_attention(q, k, v, mask, 1 / math.sqrt(D), heads=heads)
+    new, old = (x.cpu().double() for x in (bsk.block_sparse_attention(*args), _plain(monkeypatch, *args)))
+    for b, h in heads:
+        e_new, e_old = (x[b, h] - want[b, h] for x in (new, old))
+        # both round about 1e-6 of a unit-variance v; 5 % covers the spread of so few rows
+        assert e_new.norm() <= 1.05 * e_old.norm(), (e_new.norm().item(), e_old.norm().item())
+        assert e_new.abs().max() <= 2e-5
+    assert (new - old).abs().max() <= 4e-5
+
+
+# Rows, keys and values that the split operands cannot carry run in fp32: the same bits.
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("where,value", [("k", float("inf")), ("k", -2.0 ** 61), ("v", float("nan")),
+                                          ("v", 2.0 ** 100), ("tiny v", 2.0 ** -90), ("q", 2.0 ** 60),
+                                          ("q", float("-inf"))])
+def test_out_of_range_operands(dev, monkeypatch, D, where, value):
+    print(f"case terms out of range {D} {where} {value}", flush=True)
+    # one wave per unit, so that both kernels visit the tiles of a row in the same order
+    B, H, L = 1, 26 if D == 64 else 13, 15360
+    q, k, v = (_rand(i, B, H, L, D).to(dev) for i in (4, 5, 6))
+    t = {"k": k, "v": v, "q": q, "tiny v": v}[where]
+    if where == "tiny v":
+        t[0, 0] *= value
+    else:
+        t[0, 0, 70, 3] = value
+    nb = L // 64
+    mask = torch.zeros(1, 1, nb, nb, dtype=torch.bool)
+    mask[..., :4] = True
+    kv = kv_list_from_mask(mask.to(dev), B, H, nb, nb)
+    args = (q, k, v, kv, 0.125)
+    new, old = bsk.block_sparse_attention(*args), _plain(monkeypatch, *args)
+    # a wave owns 64 query rows (32 at head dim 128) and decides for them
+    rows = slice(64, 128 if D == 64 else 96) if where == "q" else slice(None)
+    assert torch.equal(new[0, 0, rows].isnan(), old[0, 0, rows].isnan())
+    assert torch.equal(new[0, 0, rows].nan_to_num(), old[0, 0, rows].nan_to_num())
+    assert not torch.equal(new[0, 1], old[0, 1])  # the other heads took the split operands
+
+
+def test_short_lists_and_strided_rows(dev, monkeypatch):
+    # head 0: one tile per key block (fp32 bits); head 1: five; BLHD views
+    print("case terms short lists", flush=True)
+    B, L, H = 1, 64 * 3100, 2
+    q, k, v = (_rand(i, B, L, H, 64).to(dev).permute(0, 2, 1, 3) for i in (7, 8, 9))
+    nb = L // 64
+    mask = torch.eye(nb, dtype=torch.bool).repeat(1, H, 1, 1)
+    mask[:, 1, :, :5] = True
+    kv = kv_list_from_mask(mask.to(dev), B, H, nb, nb)
+    args = (q, k, v, kv, 0.125)
+    new, old = bsk.block_sparse_attention(*args), _plain(monkeypatch, *args)
+    assert torch.equal(new[:, 0], old[:, 0])
+    assert not torch.equal(new[:, 1], old[:, 1])
+    assert (new - old).abs().max() <= 4e-5
