@@ -301,8 +301,11 @@ int sa_attn_pooling_fwd(const uint16_t* q, const int64_t q_strides[3], const uin
  * block (causal: up to the diagonal, the diagonal tile masked to keys <= query), grouped key
  * heads as there; the rows' column maxima and log-sum-exps go to the workspace and a reduce
  * kernel forms Po for every block size. D = 64 or 128; same workspace
- * (sa_attn_pooling_workspace), strides in elements, multiples of 4.
+ * (sa_attn_pooling_workspace), strides in elements, multiples of 4. With a workspace of
+ * sa_attn_pooling_workspace_f32's size and L >= 512 the products run on split operands, as
+ * sa_block_sparse_fwd_f32_terms computes them.
  */
+int sa_attn_pooling_workspace_f32(int B, int H, int H_kv, int L, int D, int block_size, int64_t* bytes);
 int sa_attn_pooling_fwd_f32(const float* q, const int64_t q_strides[3], const float* k,
                             const int64_t k_strides[3], const float* v, const int64_t v_strides[3],
                             float* out, const int64_t out_strides[3], int B, int H, int H_kv, int L,

@@ -2129,6 +2129,15 @@ extern "C" int sa_attn_pooling_workspace(int B, int H, int L, int block_size, in
   return sa::ok();
 }
 
+extern "C" int sa_attn_pooling_workspace_f32(int B, int H, int H_kv, int L, int D, int block_size, int64_t* bytes) {
+  const char* fn = "sa_attn_pooling_workspace_f32";
+  SA_REQUIRE(H_kv > 0 && H % H_kv == 0, "%s: H_kv=%d must divide H=%d", fn, H_kv, H);
+  if (D != 64 && D != 128) return sa::fail(SA_ERR_UNSUPPORTED, "%s: head_dim %d (64 or 128)", fn, D);
+  if (int rc = sa_attn_pooling_workspace(B, H, L, block_size, bytes)) return rc;
+  *bytes += sa::attn_f32_terms_bytes(B, H_kv, L, D);
+  return sa::ok();
+}
+
 namespace {
 
 // Po from the stored row maxima and log-sum-exps (pool_reduce_kernel).
@@ -2193,7 +2202,8 @@ int attn_pooling(const uint16_t* q, const int64_t q_strides[3], const uint16_t* 
 
 // fp32 q, k, v (the reference's own arithmetic for attn_with_pooling, which computes in fp32):
 // the fp32 kernel in pooling mode stores the row maxima and log-sum-exps, the reduce kernel
-// forms Po for every block size.
+// forms Po for every block size. A workspace of sa_attn_pooling_workspace_f32's size has room for
+// the split operands of attn_f32.hip, at its end.
 int attn_pooling_f32(const float* q, const int64_t q_strides[3], const float* k, const int64_t k_strides[3],
                      const float* v, const int64_t v_strides[3], float* out, const int64_t out_strides[3], int B,
                      int H, int H_kv, int L, int D, int causal, float sm_scale, int block_size, float* po,
@@ -2223,8 +2233,13 @@ int attn_pooling_f32(const float* q, const int64_t q_strides[3], const float* k,
   if (int rc = sa::check_launch(fn)) return rc;
   float* r = reinterpret_cast<float*>(ws + p.r);
   float* lse = reinterpret_cast<float*>(ws + p.lse);
+  const int64_t plain = (int64_t)p.total;
+  void* terms = nullptr;
+  if (L >= 8 * kBlock && (D == 64 || D == 128) && workspace_bytes - plain >= sa::attn_f32_terms_bytes(B, H_kv, L, D) &&
+      (int64_t)p.nkb * 768 * D <= 0x7fffffffLL)
+    terms = ws + plain;
   if (int rc = sa::attn_f32_pooling(q, q_strides, k, k_strides, v, v_strides, out, out_strides, B, H, L, D, la.idx,
-                                    la.cnt, p.nkb, H / H_kv, causal != 0, sm_scale, p.G, r, lse, nullptr, stream, fn))
+                                    la.cnt, p.nkb, H / H_kv, causal != 0, sm_scale, p.G, r, lse, terms, stream, fn))
     return rc;
   return launch_pool_reduce(p, r, lse, B, H, L, block_size, causal, po, po_strides, s, fn);
 }

@@ -18,13 +18,13 @@ q, k and v are bf16, fp16 or fp32 (one dtype), head_dim 64 or 128. Po is fp32 fo
 fp32 inputs and fp16 for fp16 inputs, the dtypes the reference returns (it computes bf16 inputs
 in fp32 and fp16 inputs in fp16, storing Po in that dtype).
 
-Arithmetic. fp32 inputs run the fp32 kernel (fp32 MFMA, P and row sums in fp32), as the
-reference does. bf16 and fp16 inputs run, by default, the 16-bit kernel: bf16 (fp16) products
-with fp32 accumulation and P rounded to the input dtype before P.V, where the reference casts
-bf16 inputs up to fp32 first (:235-240); `attn_with_pooling(..., precision="fp32")` does what
-the reference does (inputs cast to fp32, the fp32 kernel, the output cast back to the input
-dtype), at the fp32 MFMA rate (1/16 of bf16's). The rows of a last, partial query block that
-lie past L take no part in its maximum; the reference reads them without bounds checks.
+Arithmetic. fp32 inputs run the fp32 kernels (P and row sums in fp32), as the reference does.
+bf16 and fp16 inputs run, by default, the 16-bit kernel: bf16 (fp16) products with fp32
+accumulation and P rounded to the input dtype before P.V, where the reference casts bf16 inputs
+up to fp32 first (:235-240); `attn_with_pooling(..., precision="fp32")` does what the reference
+does (inputs cast to fp32, the fp32 kernels, the output cast back to the input dtype). The rows
+of a last, partial query block that lie past L take no part in its maximum; the reference reads
+them without bounds checks.
 """
 from __future__ import annotations
 
@@ -69,7 +69,18 @@ class _attention_pooling(torch.autograd.Function):
         ws_bytes = ctypes.c_int64(0)
         _lib.check(lib.sa_attn_pooling_workspace(B, H, L, block_size, ctypes.byref(ws_bytes)),
                    "sa_attn_pooling_workspace")
-        ws = torch.empty(ws_bytes.value, dtype=torch.uint8, device=q.device)
+        ws = None
+        if fp32 and L >= 8 * 64 and D in (64, 128):
+            # With room for its split operands the fp32 kernel runs on the bf16 matrix core.
+            more = ctypes.c_int64(0)
+            _lib.check(lib.sa_attn_pooling_workspace_f32(B, H, Hk, L, D, block_size, ctypes.byref(more)),
+                       "sa_attn_pooling_workspace_f32")
+            try:
+                ws = torch.empty(more.value, dtype=torch.uint8, device=q.device)
+            except torch.cuda.OutOfMemoryError:
+                pass
+        if ws is None:
+            ws = torch.empty(ws_bytes.value, dtype=torch.uint8, device=q.device)
         fn = "sa_attn_pooling_fwd_f16" if fp16 else ("sa_attn_pooling_fwd_f32" if fp32 else "sa_attn_pooling_fwd")
         with torch.cuda.device(q.device):
             _lib.check(getattr(lib, fn)(

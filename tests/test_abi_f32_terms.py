@@ -29,3 +29,14 @@ def test_workspace_is_checked(D):
     assert call(p, n.value, q=p + 4) == _lib.SA_ERR_UNSUPPORTED
     assert call(p, n.value, d=96) == _lib.SA_ERR_UNSUPPORTED
     assert call(p, 1 << 62, Lk=1 << 24) == _lib.SA_ERR_UNSUPPORTED  # past the 32-bit offsets of one head
+
+
+def test_pooling_workspace_holds_the_split_operands():
+    lib = _lib.load()
+    n, base = ctypes.c_int64(0), ctypes.c_int64(0)
+    assert lib.sa_attn_pooling_workspace(2, 4, 900, 32, ctypes.byref(base)) == _lib.SA_OK
+    assert lib.sa_attn_pooling_workspace_f32(2, 4, 2, 900, 64, 32, ctypes.byref(n)) == _lib.SA_OK
+    assert base.value % 256 == 0 and n.value == base.value + 2 * 2 * 15 * (768 * 64 + 16)
+    assert lib.sa_attn_pooling_workspace_f32(2, 4, 3, 900, 64, 32, ctypes.byref(n)) == _lib.SA_ERR_INVALID
+    assert lib.sa_attn_pooling_workspace_f32(2, 4, 2, 900, 96, 32, ctypes.byref(n)) == _lib.SA_ERR_UNSUPPORTED
+    assert lib.sa_attn_pooling_workspace_f32(2, 4, 2, 900, 64, 48, ctypes.byref(n)) == _lib.SA_ERR_INVALID

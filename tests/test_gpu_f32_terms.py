@@ -6,8 +6,10 @@ import pytest
 import torch
 
 from oracle.attention import masked_attention
+from oracle.pooling import pooled_attention
 from sparseattnfunctions_amd._kv import kv_list_from_mask
 from sparseattnfunctions_amd.utils import block_sparse_attn_kernel as bsk
+from sparseattnfunctions_amd.utils.attn_pooling_kernel import attn_with_pooling
 
 pytestmark = pytest.mark.gpu
 
@@ -99,3 +101,21 @@ def test_short_lists_and_strided_rows(dev, monkeypatch):
     assert torch.equal(new[:, 0], old[:, 0])
     assert not torch.equal(new[:, 1], old[:, 1])
     assert (new - old).abs().max() <= 4e-5
+
+
+# The pooled map beside one-wave units (more than 6 144) and shared ones, partial last blocks,
+# grouped key heads; bars of the fp32 pooling tests.
+@pytest.mark.parametrize("H,Hk,L,D,bs,causal", [(130, 130, 3077, 64, 64, False), (130, 65, 3077, 64, 32, True),
+                                                 (66, 33, 3077, 128, 128, True), (66, 66, 3077, 128, 32, False),
+                                                 (2, 1, 515, 64, 128, False), (2, 2, 577, 128, 64, True)])
+def test_pooled_map(dev, H, Hk, L, D, bs, causal):
+    print(f"case terms pooled {H} {Hk} {L} {D} {bs} {causal}", flush=True)
+    q, k, v = _rand(1, 1, H, L, D), _rand(2, 1, Hk, L, D), _rand(3, 1, Hk, L, D)
+    o, po = attn_with_pooling(q.to(dev), k.to(dev), v.to(dev), causal, 1 / math.sqrt(D), bs)
+    for h in (0, H - 1):
+        hk = h // (H // Hk)
+        want_o, want_po = pooled_attention(q[:, h:h + 1], k[:, hk:hk + 1], v[:, hk:hk + 1], causal, 1 / math.sqrt(D),
+                                           bs)
+        err = (o[:, h:h + 1].cpu().double() - want_o).abs()
+        assert err.max() <= 2e-5 and err.mean() <= 2e-6
+        assert torch.allclose(po[:, h:h + 1].cpu().double(), want_po, rtol=2e-5, atol=1e-9)
