@@ -575,6 +575,19 @@ int sa_topk_share(const float* P, int64_t p_bh_stride, int64_t p_row_stride, int
                   int n, int K, float* share, void* stream);
 
 /*
+ * The share of sa_topk_share from the query and key rows, without written probabilities: for
+ * each of `rows` queries q_rows [BH][rows_pad][64], the softmax mass (over n keys, scores scaled
+ * by sm_scale) of the K largest probabilities, ties at the K-th counted once each. n <= 16384.
+ * k_ops are the keys in matrix-operand order, as sa_gather_key_operands writes them: rows idx
+ * [n_pad] (int32, outside [0, L): zeros) of x [B, H, L, 64] to out [B*H][n_pad / 32][4][64] chunks
+ * of 16 bytes, chunk (t, s, 32 hh + c) holding columns 16 s + 8 hh .. + 7 of row 32 t + c.
+ */
+int sa_gather_key_operands(const uint16_t* x, const int64_t strides[3], int B, int H, int L, int D,
+                           const int32_t* idx, int n_pad, uint16_t* out, void* stream);
+int sa_topk_mass(const uint16_t* q_rows, const uint16_t* k_ops, int BH, int rows, int rows_pad, int n, int n_pad,
+                 float sm_scale, int K, float* share, void* stream);
+
+/*
  * Gram matrices of the sampled frame-pair attention patterns (judge_similarity,
  * partern_attention.py:502-512): with P the [F*ns x F*ns] video part of the sampled
  * probabilities, G[bh][f2][chunk][pair(f1,f3)] = sum over s1 in the chunk (8 positions)
@@ -595,6 +608,16 @@ int sa_pattern_gram(const float* P, int64_t p_bh_stride, int64_t p_row_stride, i
 int sa_pattern_sim_gram(const uint16_t* q_rows, const uint16_t* k_rows, int BH, int F, int ns,
                         int T, int rows_pad, int keys_pad, float sm_scale, float bias, float* G,
                         void* stream);
+
+/*
+ * sa_pattern_sim_gram in one walk over the keys instead of two: each position's products wait
+ * unnormalised in a caller workspace (sa_pattern_sim_gram_workspace bytes, 16-byte aligned) until
+ * its row sums are known. Same results up to fp32 rounding.
+ */
+int sa_pattern_sim_gram_workspace(int BH, int F, int ns, int64_t* bytes);
+int sa_pattern_sim_gram_ws(const uint16_t* q_rows, const uint16_t* k_rows, int BH, int F, int ns, int T, int rows_pad,
+                           int keys_pad, float sm_scale, float bias, float* G, void* workspace,
+                           int64_t workspace_bytes, void* stream);
 
 /*
  * Routing decision of unified_judge (partern_attention.py:516-521) per head:

@@ -123,6 +123,10 @@ _PROTOTYPES = {
     "sa_topk_share": (_I, [_P, ctypes.c_int64, ctypes.c_int64, _I, _I, _I, _I, _P, _P]),
     "sa_pattern_gram": (_I, [_P, ctypes.c_int64, ctypes.c_int64, _I, _I, _I, _P, _P]),
     "sa_pattern_sim_gram": (_I, [_P, _P, _I, _I, _I, _I, _I, _I, _F, _F, _P, _P]),
+    "sa_gather_key_operands": (_I, [_P, _I64P, _I, _I, _I, _I, _P, _I, _P, _P]),
+    "sa_topk_mass": (_I, [_P, _P, _I, _I, _I, _I, _I, _F, _I, _P, _P]),
+    "sa_pattern_sim_gram_workspace": (_I, [_I, _I, _I, _I64P]),
+    "sa_pattern_sim_gram_ws": (_I, [_P, _P, _I, _I, _I, _I, _I, _I, _F, _F, _P, _P, ctypes.c_int64, _P]),
     "sa_pattern_judge_finish": (_I, [_P, _P, _P, _I, _I, _I, _I, _F, _F, _P, _P, _P, _P, _P]),
     "sa_pattern_plan": (_I, [_P, _I64P, _P, _I, _I, _I, _I, _I, _F, _F, _F, _F, _F, _P, _P, _P, _P, _P, _P]),
     "sa_pattern_combine": (_I, [_P, _I64P, _P, _I64P, _P, _I64P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I,

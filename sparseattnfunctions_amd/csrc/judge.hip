@@ -14,9 +14,15 @@
 //                      G[f1][f3] = sum_{s1,s2} P[f1 s1][f2 s2] * P[f3 s1][f2 s2] of the
 //                      frame-pair patterns (their inner products and norms), as partial sums
 //                      over chunks of s1;
+//   topk_mass_kernel   judge_sparsity as the Python layer runs it: the same masses with the
+//                      scores recomputed by each of a few walks over the keys instead of written;
+//   simgram_kernel     judge_similarity as the Python layer runs it: the Gram partials with
+//                      the probabilities kept on chip;
+//   gather_operands_kernel  sampled keys in matrix-operand order, for topk_mass_kernel;
 //   finish_kernel      per head: mean share > 0.9 (sparse), mean cosine similarity of the
 //                      patterns sharing a key frame > 0.9 (twice), and the routing decision.
 #include <cmath>
+#include <type_traits>
 
 #include "sa_common.h"
 
@@ -340,6 +346,305 @@ __global__ __launch_bounds__(256) void share_kernel(ShareArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------
+// topk_mass_kernel: the share of judge_sparsity without written probabilities. One workgroup of
+// eight waves per (bh, 32 query rows), lane column = row; wave w takes key tiles w, w + 8, ... of
+// every walk over the keys, and each walk recomputes the scores (four MFMAs per 32 x 32 tile from
+// keys in operand order, one coalesced 1 KB load each):
+//   1: row maxima and minima;
+//   2: e = exp2(x - max) and a histogram per row of e's bit pattern above the row's smallest
+//      (linear in log2 e: 256 equal bins, LDS atomics whose bank is the row's), the row sum; the
+//      bin of the K-th largest e follows from the counts. While that bin holds more than kTmCap
+//      entries and spans more than one pattern, it is divided again by another walk;
+//   3: the sum of e above the bin; the bin's entries go to a list, whose K-th largest is then
+//      searched bit by bit by 16 lanes per row.
+// The same selection as share_kernel's, on e instead of e / sum: share = (sum of the entries above
+// the K-th, and it for the ties needed) / row sum. The list arrives in any order, so its sum is
+// taken in fp64, which is exact for the entries of one bin: the result is the same every time.
+// Bound: the scores' exp2, bins and sums, 0.7 G entries for 96 heads of 500 x 15 035, three
+// times (a third walk more where the heads are peaked); writing and re-reading their 2.9 GB in fp32
+// took 1.24 + 1.31 ms, this takes 0.87 (1.09 with a head's workgroups spread over the XCDs).
+constexpr int kTmWaves = 8;
+constexpr int kTmBins = 256;
+constexpr int kTmCap = 256;
+
+struct TopkMassArgs {
+  const uint16_t* qs;   // [BH][rows_pad][64]
+  const jd_u32x4* ks;   // [BH][n_tiles][4][64]: key operands (gather_operands_kernel)
+  int rows, rows_pad, n, n_tiles, K;
+  float scale_log2;
+  float* share;  // [BH][rows]
+  int ng;        // cdiv(rows, 32)
+  int BH;
+};
+
+__global__ __launch_bounds__(64 * kTmWaves, 4) void topk_mass_kernel(TopkMassArgs a) {
+  __shared__ uint32_t hist[kTmBins * 32];  // [bin][row]
+  __shared__ uint32_t list[kTmCap * 32];   // [entry][row]
+  __shared__ float wred[kTmWaves][2][32];  // the waves' partial maxima / minima / sums
+  // Per row: the bin under division is patterns base .. base + width - 1, in kTmBins parts of
+  // 2^shift; above = entries above it, count = entries in it, todo = still to be divided.
+  __shared__ uint32_t base[32], width[32], shift[32], above[32], count[32], fill[32];
+  __shared__ int todo[32];
+  __shared__ int again;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int col = lane & 31, hh = lane >> 5;
+  // A head's workgroups share an XCD, whose L2 then holds the head's keys (workgroups go round
+  // robin over the eight XCDs).
+  const int x8 = blockIdx.x >> 3;
+  const int64_t bh = 8 * (int64_t)(x8 / a.ng) + (blockIdx.x & 7);
+  const int row0 = 32 * (x8 % a.ng);
+  if (bh >= a.BH) return;
+
+  sa_bf16x8 qf[4];
+  {
+    const uint16_t* qp = a.qs + (bh * a.rows_pad + row0 + col) * kD + 8 * hh;  // rows_pad covers row0 + 31
+#pragma unroll
+    for (int s = 0; s < 4; ++s) qf[s] = __builtin_bit_cast(sa_bf16x8, *reinterpret_cast<const jd_u32x4*>(qp + 16 * s));
+  }
+  const jd_u32x4* kbase = a.ks + bh * a.n_tiles * 256 + lane;
+  // f(tag: the whole tile exists, scores of a tile, entries that exist); entry i of a lane is key
+  // 32 kt + 8 (i / 4) + 4 hh + i % 4.
+  auto walk = [&](auto f) __attribute__((always_inline)) {
+    jd_u32x4 kop[4], knext[4];
+    if (wave < a.n_tiles) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) knext[s] = kbase[(int64_t)wave * 256 + 64 * s];
+    }
+    for (int kt = wave; kt < a.n_tiles; kt += kTmWaves) {
+      const int kn = kt + kTmWaves < a.n_tiles ? kt + kTmWaves : kt;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) kop[s] = knext[s];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) knext[s] = kbase[(int64_t)kn * 256 + 64 * s];
+      const int left = a.n - 32 * kt;
+      const sa_f32x16 x = score_tile_k(kop, qf);
+      if (left >= 32) f(std::true_type{}, x, left);
+      else f(std::false_type{}, x, left);
+    }
+  };
+  auto exists = [&](int left, int i) { return 8 * (i >> 2) + 4 * hh + (i & 3) < left; };
+  // max / sum over the two lane halves, then over the waves in order.
+  auto half = [&](float x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return hh ? __uint_as_float(r[0]) : __uint_as_float(r[1]);  // the other half's value
+  };
+
+  // ---- 1: maxima and minima of the raw scores (the scale is positive).
+  float mx = -INFINITY, mn = INFINITY;
+  walk([&](auto whole, const sa_f32x16& x, int left) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      if (whole.value || exists(left, i)) {
+        mx = fmaxf(mx, x[i]);
+        mn = fminf(mn, x[i]);
+      }
+  });
+  mx = fmaxf(mx, half(mx));
+  mn = fminf(mn, half(mn));
+  if (hh == 0) {
+    wred[wave][0][col] = mx;
+    wred[wave][1][col] = mn;
+  }
+  for (int i = t; i < kTmBins * 32; i += 64 * kTmWaves) hist[i] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kTmWaves; ++w) {
+    mx = fmaxf(mx, wred[w][0][col]);
+    mn = fminf(mn, wred[w][1][col]);
+  }
+  const float m = mx * a.scale_log2;
+  auto e_of = [&](float x) { return __builtin_amdgcn_exp2f(fmaf(x, a.scale_log2, -m)); };
+  if (t < 32) {
+    // Patterns from just below the smallest e to just above 1 (exp2 may round either way).
+    const uint32_t lo = min(__float_as_uint(e_of(mn)), 0x3f800000u);
+    const uint32_t b0 = lo > 64u ? lo - 64u : 0u;
+    base[t] = b0;
+    width[t] = row0 + t < a.rows ? 0x3f800040u - b0 : 0u;
+    shift[t] = max(0, 32 - 8 - __clz((int)(0x3f800040u - b0)));
+    above[t] = 0;
+    count[t] = 0;
+    todo[t] = row0 + t < a.rows;
+    fill[t] = 0;
+  }
+  if (t == 0) again = 0;
+  __syncthreads();
+
+  // ---- 2: histograms until the K-th entry's bin fits the list.
+  float l = 0.f;
+  for (int round = 1;; ++round) {
+    const uint32_t b0 = base[col], wd = width[col], sh = shift[col];
+    if (round == 1) {
+      walk([&](auto whole, const sa_f32x16& x, int left) __attribute__((always_inline)) {
+        float sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (whole.value || exists(left, i)) {
+            const float e = e_of(x[i]);
+            sum += e;
+            const uint32_t d = __builtin_elementwise_sub_sat(__float_as_uint(e), b0) >> sh;
+            atomicAdd(&hist[32 * min(d, (uint32_t)kTmBins - 1) + col], 1u);
+          }
+        l += sum;
+      });
+    } else {
+      const bool open = todo[col] != 0;
+      walk([&](auto whole, const sa_f32x16& x, int left) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const uint32_t d = __float_as_uint(e_of(x[i])) - b0;
+          if (open && d < wd && (whole.value || exists(left, i))) atomicAdd(&hist[32 * (d >> sh) + col], 1u);
+        }
+      });
+    }
+    __syncthreads();
+    // 16 lanes per row: lane s sums bins 16 s .. + 15, then the counts from the top.
+    {
+      const int r = t >> 4, s = t & 15;
+      const bool mine = todo[r] != 0;
+      uint32_t h[16], tot = 0;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        h[i] = hist[32 * (16 * s + i) + r];
+        tot += h[i];
+      }
+      uint32_t suffix = tot;  // entries in this lane's bins and above
+#pragma unroll
+      for (int o = 1; o < 16; o <<= 1) {
+        const uint32_t y = (uint32_t)__shfl_down((int)suffix, o, 16);
+        if (s + o < 16) suffix += y;
+      }
+      const uint32_t need = (uint32_t)a.K - above[r];
+      const uint32_t over = suffix - tot;  // entries above this lane's bins
+      __syncthreads();                     // every lane has read above and todo
+      if (mine && over < need && suffix >= need) {  // the K-th is in one of this lane's bins
+        uint32_t run = over;
+        int bin = 15;
+        for (; bin > 0; --bin) {
+          if (run + h[bin] >= need) break;
+          run += h[bin];
+        }
+        above[r] += run;
+        count[r] = h[bin];
+        base[r] += (uint32_t)(16 * s + bin) << shift[r];
+        width[r] = 1u << shift[r];
+        todo[r] = h[bin] > (uint32_t)kTmCap && shift[r] > 0;
+        if (todo[r]) {
+          shift[r] = shift[r] > 8 ? shift[r] - 8 : 0;
+          again = round;
+        }
+      }
+    }
+    for (int i = t; i < kTmBins * 32; i += 64 * kTmWaves) hist[i] = 0;
+    __syncthreads();
+    if (again != round) break;
+  }
+  // ---- 3: the sum above the bin and the bin's entries.
+  const uint32_t b0 = base[col], wd = width[col];
+  const bool listed = count[col] <= (uint32_t)kTmCap;  // else the bin is one pattern
+  float sum_above = 0.f;
+  walk([&](auto whole, const sa_f32x16& x, int left) __attribute__((always_inline)) {
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float e = e_of(x[i]);
+      const uint32_t u = __float_as_uint(e);
+      if (whole.value || exists(left, i)) {
+        sum += u >= b0 + wd ? e : 0.f;
+        if (u - b0 < wd && listed) {
+          const uint32_t at = atomicAdd(&fill[col], 1u);
+          if (at < (uint32_t)kTmCap) list[32 * at + col] = u;
+        }
+      }
+    }
+    sum_above += sum;
+  });
+  l += half(l);
+  sum_above += half(sum_above);
+  if (hh == 0) {
+    wred[wave][0][col] = l;
+    wred[wave][1][col] = sum_above;
+  }
+  __syncthreads();
+  // 16 lanes per row: the K-th largest is the (K - above)-th of the list, or the bin's one pattern.
+  {
+    const int r = t >> 4, s = t & 15;
+    const uint32_t need = (uint32_t)a.K - above[r];
+    const uint32_t nl = min(fill[r], (uint32_t)kTmCap);
+    uint32_t v[kTmCap / 16];
+#pragma unroll
+    for (int i = 0; i < kTmCap / 16; ++i) {
+      const uint32_t at = (uint32_t)(16 * i + s);
+      v[i] = at < nl ? list[32 * at + r] : 0u;
+    }
+    uint32_t thr = base[r];
+    double extra = 0.0;
+    uint32_t gt = 0;
+    if (count[r] <= (uint32_t)kTmCap) {
+      thr = 0;
+      for (int bit = 30; bit >= 0; --bit) {
+        const uint32_t cand = thr | (1u << bit);
+        uint32_t c = 0;
+#pragma unroll
+        for (int i = 0; i < kTmCap / 16; ++i) c += v[i] >= cand;
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) c += (uint32_t)__shfl_xor((int)c, o);
+        if (c >= need) thr = cand;
+      }
+#pragma unroll
+      for (int i = 0; i < kTmCap / 16; ++i)
+        if (v[i] > thr) {
+          extra += (double)__uint_as_float(v[i]);
+          ++gt;
+        }
+#pragma unroll
+      for (int o = 8; o > 0; o >>= 1) {
+        extra += __shfl_xor(extra, o);
+        gt += (uint32_t)__shfl_xor((int)gt, o);
+      }
+    }
+    if (s == 0 && row0 + r < a.rows) {
+      float tot = 0.f, top = 0.f;
+#pragma unroll
+      for (int w = 0; w < kTmWaves; ++w) {
+        tot += wred[w][0][r];
+        top += wred[w][1][r];
+      }
+      const float ties = (float)((int)need - (int)gt) * __uint_as_float(thr);
+      a.share[bh * a.rows + row0 + r] = (top + ((float)extra + ties)) / tot;
+    }
+  }
+}
+
+// Key operands: rows idx of x (zeros for -1) in the order of v_mfma_f32_32x32x16_bf16's A operand,
+// out[bh][row / 32][s][lane (col, hh)] = x[b][h][idx[row]][16 s + 8 hh .. + 7], col = row % 32.
+struct GatherOpsArgs {
+  const uint16_t* x;
+  int64_t sb, sh, sl;
+  int H, L;
+  const int32_t* idx;
+  int n_pad;
+  jd_u32x4* out;
+  int64_t total;  // B * H * n_pad * 8
+};
+
+__global__ __launch_bounds__(256) void gather_operands_kernel(GatherOpsArgs a) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= a.total) return;
+  const int c = (int)(i & 7);  // 16-byte chunk of the row: 8 lanes read one row
+  const int64_t rb = i >> 3;
+  const int64_t bh = rb / a.n_pad;
+  const int row = (int)(rb - bh * a.n_pad);
+  const int64_t b = bh / a.H;
+  const int h = (int)(bh - b * a.H);
+  const int src = a.idx[row];
+  jd_u32x4 v = {0u, 0u, 0u, 0u};
+  if ((unsigned)src < (unsigned)a.L)
+    v = *reinterpret_cast<const jd_u32x4*>(a.x + b * a.sb + h * a.sh + (int64_t)src * a.sl + 8 * c);
+  a.out[((bh * (a.n_pad / 32) + row / 32) * 4 + (c >> 1)) * 64 + (c & 1) * 32 + (row & 31)] = v;
+}
+
+// ---------------------------------------------------------------------------------------
 // gram_kernel: one workgroup per (bh, key frame f2, chunk of kGramChunk sample positions s1).
 // Thread t takes columns s2 = t, t + 256, ... of frame f2 and accumulates, over its s1 chunk,
 // the products of the F values P[f1*ns + s1][f2*ns + s2] (f1 = 0..F-1) of each column.
@@ -401,12 +706,21 @@ __global__ __launch_bounds__(256) void gram_kernel(GramArgs a) {
 // F frames' rows f1*ns + s1 of the 8 positions, 12 columns per position: flat column
 // 32 g + col = 12 j + f1 for position j of the chunk (columns with f1 >= F and positions
 // past ns are zero queries whose results are never used).
-//   pass 1: row max and sum over every key, bias on the T text keys (as probs_kernel);
-//   pass 2, per key frame f2: the probabilities of the frame's ns keys, 32 at a time, go
-//           through LDS ([key][flat column]); lane (key k, half sl) then adds, for each of
-//           its positions 4 sl .. 4 sl + 3, the products P[f1][k] P[f3][k] of the
-//           position's F rows into F(F+1)/2 per-lane sums. After the frame the 64 lanes' sums are added through LDS, in lane
-//           order, into G[bh][f2][chunk][pair].
+// Per key frame f2, e = exp2(x - m) of the frame's ns keys, 32 at a time, goes through LDS
+// ([key][flat column]) and the products e[f1][k] e[f3][k] are summed by v_mfma_f32_4x4x1_16b_f32,
+// in fp32: block b of its 16 is position b % 8 at key 2 i + b / 8, its A and B operands four of
+// the position's 12 columns (lane l: block l / 4, column l % 4), so three LDS reads feed the six
+// column-group pairs u <= w.
+//   kOne: one walk over the keys. m is the row's maximum over the first key tile (text keys carry
+//     the bias, as in probs_kernel), the row sums add up beside the products, and the products,
+//     kept per position, wait in a workspace until the sums are known: G = sum over the positions
+//     of inv[f1] inv[f3] (e e). A row sum above kSgSumMax (or NaN) walks the keys for the exact
+//     maxima first and starts again.
+//   otherwise (no workspace): a first walk for the row sums, then normalised products.
+// Bound: issue of scaling, exp2 and sums (VALU) and of the products, 3 G elements for 96 heads
+// of 5 500 x 5 724, which do not overlap with this MFMA shape. Measured there, per judge: two
+// walks with the products as 66 FMAs per (position, key) 2.2 ms, with MFMA products 1.85,
+// one walk 1.44 (MFMA pipes busy 42 %).
 struct SimGramArgs {
   const uint16_t* qs;  // [BH][rows_pad][64], row f*ns + s
   const uint16_t* ks;  // [BH][keys_pad][64], T text keys then F*ns sampled keys
@@ -415,24 +729,29 @@ struct SimGramArgs {
   float* G;  // [BH][F][n_chunks][NP]
   int n_chunks;
   int64_t total;  // BH * n_chunks
+  float* ws;      // kOne: [total][F][4 kPairs][32] unnormalised products
 };
 
 constexpr int kSgWidth = 12;                            // columns per position (F <= 12)
 constexpr int kSgGroups = kGramChunk * kSgWidth / 32;  // query groups per wave
 static_assert(kGramChunk * kSgWidth == 32 * kSgGroups, "positions fill whole query groups");
-// LDS row stride (floats) of the P tile [key][flat column]: stride / 4 odd, so a b128 read
-// by 16 lanes of consecutive keys covers 16 distinct 4-bank chunks (64 banks).
+// LDS row stride (floats) of the e tile [key][flat column]: the product reads (8 positions x 4
+// columns, 12 apart) of one key cover 32 of the 64 banks once.
 constexpr int kSgStride = 32 * kSgGroups + 4;
+constexpr float kSgSumMax = 0x1p60f;  // a product sum is at most the square of a row sum
+constexpr int sg_pairs(int F) { return ((F + 3) / 4) * ((F + 3) / 4 + 1) / 2; }
 
-template <int F>
+__device__ inline sa_f32x4 mfma4x4(float a, float b, sa_f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 0, 0, 0);
+}
+
+template <int F, bool kOne>
 __global__ __launch_bounds__(256, 2) void simgram_kernel(SimGramArgs a) {
   static_assert(F >= 1 && F <= 12, "frames");
   constexpr int NP = F * (F + 1) / 2;
-  constexpr int kRed = 64 * NP;
-  constexpr int kTile = 32 * kSgStride;
-  constexpr int kLds = kRed > kTile ? kRed : kTile;
-  constexpr int kRead = (F + 3) / 4;  // 16-byte reads per row of F values
-  __shared__ __attribute__((aligned(16))) float lds[4][kLds];
+  constexpr int kQuads = (F + 3) / 4;   // 4-column groups of a position
+  constexpr int kPairs = sg_pairs(F);  // group pairs u <= w
+  __shared__ __attribute__((aligned(16))) float lds[4][32 * kSgStride];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t wid = (int64_t)blockIdx.x * 4 + wave;
   if (wid >= a.total) return;  // no workgroup barriers below
@@ -455,125 +774,233 @@ __global__ __launch_bounds__(256, 2) void simgram_kernel(SimGramArgs a) {
     }
   }
 
-  // ---- pass 1: row statistics over every key
   float m[kSgGroups], l[kSgGroups];
-#pragma unroll
-  for (int g = 0; g < kSgGroups; ++g) {
-    m[g] = -INFINITY;
-    l[g] = 0.f;
-  }
   const uint16_t* kbase = a.ks + (bh * a.keys_pad + col) * kD + 8 * hh;
-  for (int kt = 0; kt < a.keys_pad / 32; ++kt) {
-    jd_u32x4 kop[4];
-    load_k(kbase + (int64_t)kt * 32 * kD, kop);
-    const bool uniform = 32 * kt + 32 <= a.keys && (32 * kt + 32 <= a.T || 32 * kt >= a.T);
-    const float tb = 32 * kt < a.T ? a.bias_log2 : 0.f;
+  // Row sums over key tiles [kt0, kt1) of the whole key list, keys >= end left out. kRunning: the
+  // maxima follow the tiles; else they stay as they are.
+  auto stats = [&](auto running_tag, int kt0, int kt1, int end) __attribute__((always_inline)) {
+    constexpr bool kRunning = decltype(running_tag)::value;
+    if (kt0 >= kt1) return;
+    jd_u32x4 kop[4], knext[4];
+    load_k(kbase + (int64_t)kt0 * 32 * kD, knext);
+    for (int kt = kt0; kt < kt1; ++kt) {
 #pragma unroll
-    for (int g = 0; g < kSgGroups; ++g) {
-      const sa_f32x16 t = score_tile_k(kop, qf[g]);
-      float x[16], tmax = -INFINITY;
-      if (uniform) {
+      for (int s = 0; s < 4; ++s) kop[s] = knext[s];
+      load_k(kbase + (int64_t)min(kt + 1, kt1 - 1) * 32 * kD, knext);  // in flight over this tile
+      const bool uniform = 32 * kt + 32 <= end && (32 * kt + 32 <= a.T || 32 * kt >= a.T);
+      const float tb = 32 * kt < a.T ? a.bias_log2 : 0.f;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) x[i] = fmaf(t[i], a.scale_log2, tb);
-      } else {
+      for (int g = 0; g < kSgGroups; ++g) {
+        const sa_f32x16 t = score_tile_k(kop, qf[g]);
+        if (!kRunning && uniform) {
+          const float off = tb - m[g];
+          float sum = 0.f;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) sum += __builtin_amdgcn_exp2f(fmaf(t[i], a.scale_log2, off));
+          l[g] += sum;
+          continue;
+        }
+        float x[16], tmax = -INFINITY;
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
           const int key = 32 * kt + 8 * (i >> 2) + 4 * hh + (i & 3);
-          x[i] = key >= a.keys ? -INFINITY : fmaf(t[i], a.scale_log2, key < a.T ? a.bias_log2 : 0.f);
+          x[i] = key >= end ? -INFINITY : fmaf(t[i], a.scale_log2, key < a.T ? a.bias_log2 : 0.f);
+        }
+        if (kRunning) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) tmax = fmaxf(tmax, x[i]);
+          const float mn = fmaxf(m[g], tmax);
+          l[g] *= m[g] == mn ? 1.f : __builtin_amdgcn_exp2f(m[g] - mn);
+          m[g] = mn;
+        }
+        if (m[g] != -INFINITY) {
+          float sum = 0.f;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) sum += __builtin_amdgcn_exp2f(x[i] - m[g]);
+          l[g] += sum;
         }
       }
-#pragma unroll
-      for (int i = 0; i < 16; ++i) tmax = fmaxf(tmax, x[i]);
-      const float mn = fmaxf(m[g], tmax);
-      if (mn != -INFINITY) {
-        float sum = 0.f;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) sum += __builtin_amdgcn_exp2f(x[i] - mn);
-        l[g] = l[g] * __builtin_amdgcn_exp2f(m[g] - mn) + sum;
-        m[g] = mn;
-      }
     }
-  }
+  };
+  // Both halves of a row's keys take one maximum, so that their sums add up directly.
+  auto merge_max = [&]() {
+#pragma unroll
+    for (int g = 0; g < kSgGroups; ++g) {
+      const auto mo = __builtin_amdgcn_permlane32_swap(__float_as_uint(m[g]), __float_as_uint(m[g]), false, false);
+      const float M = fmaxf(__uint_as_float(mo[0]), __uint_as_float(mo[1]));
+      if (m[g] != M) l[g] *= __builtin_amdgcn_exp2f(m[g] - M);
+      m[g] = M;
+    }
+  };
+  auto reset = [&]() {
+#pragma unroll
+    for (int g = 0; g < kSgGroups; ++g) {
+      m[g] = -INFINITY;
+      l[g] = 0.f;
+    }
+  };
   float inv[kSgGroups];
+  auto finish = [&]() {  // inv = 1 / row sum; true when a sum left the range (it is at least 1: the row's maximum of a tile)
+    bool bad = false;
 #pragma unroll
-  for (int g = 0; g < kSgGroups; ++g) {
-    const auto mo = __builtin_amdgcn_permlane32_swap(__float_as_uint(m[g]), __float_as_uint(m[g]), false, false);
-    const auto lo = __builtin_amdgcn_permlane32_swap(__float_as_uint(l[g]), __float_as_uint(l[g]), false, false);
-    const float m0 = __uint_as_float(mo[0]), m1 = __uint_as_float(mo[1]);
-    const float M = fmaxf(m0, m1);
-    const float lt = __uint_as_float(lo[0]) * __builtin_amdgcn_exp2f(m0 - M) +
-                     __uint_as_float(lo[1]) * __builtin_amdgcn_exp2f(m1 - M);
-    m[g] = M;
-    inv[g] = 1.f / lt;
-  }
+    for (int g = 0; g < kSgGroups; ++g) {
+      const auto lo = __builtin_amdgcn_permlane32_swap(__float_as_uint(l[g]), __float_as_uint(l[g]), false, false);
+      const float lt = __uint_as_float(lo[0]) + __uint_as_float(lo[1]);
+      bad |= !(lt <= kSgSumMax);
+      inv[g] = 1.f / lt;
+    }
+    return __ballot(bad) != 0;
+  };
+  const int n_tiles = a.keys_pad / 32;
 
-  // ---- pass 2: per key frame, probabilities through LDS and the pair products. Columns of
-  // positions past ns (zero queries, whose uniform rows are not samples) write zeros.
-  bool pos_ok[kSgGroups];
-#pragma unroll
-  for (int g = 0; g < kSgGroups; ++g) {
-    const int flat = 32 * g + col;
-    pos_ok[g] = chunk * kGramChunk + flat / kSgWidth < a.ns && flat % kSgWidth < F;
-  }
-  const int my_key = lane & 31, sl = lane >> 5;
+  // Lane l reads column 4 u + l % 4 of position (l / 4) % 8 at key 2 i + l / 32.
+  float* wp = L + 4 * hh * kSgStride + col;
+  const float* rp = L + hh * kSgStride + kSgWidth * ((lane >> 2) & 7) + (lane & 3);
   const int n_kt = (a.ns + 31) / 32;
-  float acc[NP];
-#pragma unroll
-  for (int p = 0; p < NP; ++p) acc[p] = 0.f;
-  for (int f2 = 0; f2 < F; ++f2) {
+  // Products of key frame f2 (kOne: unnormalised, and the frame's part of the row sums).
+  auto frame = [&](int f2, sa_f32x4 (&acc)[kPairs]) __attribute__((always_inline)) {
     const int frame0 = a.T + f2 * a.ns;
+#pragma unroll
+    for (int p = 0; p < kPairs; ++p) acc[p] = sa_f32x4{0.f, 0.f, 0.f, 0.f};
+    auto load_frame = [&](int t, jd_u32x4 (&k4)[4]) {
+      load_k(a.ks + (bh * a.keys_pad + min(frame0 + 32 * t + col, a.keys_pad - 1)) * kD + 8 * hh, k4);
+    };
+    jd_u32x4 kop[4], knext[4];
+    load_frame(0, knext);
     for (int t = 0; t < n_kt; ++t) {
-      jd_u32x4 kop[4];
-      load_k(a.ks + (bh * a.keys_pad + min(frame0 + 32 * t + col, a.keys_pad - 1)) * kD + 8 * hh, kop);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) kop[s] = knext[s];
+      load_frame(min(t + 1, n_kt - 1), knext);  // in flight over this tile
+      const int left = a.ns - 32 * t;  // keys of the frame from this tile on
 #pragma unroll
       for (int g = 0; g < kSgGroups; ++g) {
-        const sa_f32x16 tt = score_tile_k(kop, qf[g]);
+        sa_f32x16 e = score_tile_k(kop, qf[g]);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) e[i] = __builtin_amdgcn_exp2f(fmaf(e[i], a.scale_log2, -m[g]));
+        if (left < 32) {  // keys past the frame count for nothing
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            if (8 * (i >> 2) + 4 * hh + (i & 3) >= left) e[i] = 0.f;
+        }
+        float sum = 0.f;
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          const int kr = 8 * (i >> 2) + 4 * hh + (i & 3);
-          const float pv = (pos_ok[g] && 32 * t + kr < a.ns)
-                               ? __builtin_amdgcn_exp2f(fmaf(tt[i], a.scale_log2, -m[g])) * inv[g] : 0.f;
-          L[kr * kSgStride + 32 * g + col] = pv;
+          if (kOne) sum += e[i];
+          else e[i] *= inv[g];
+          wp[(8 * (i >> 2) + (i & 3)) * kSgStride + 32 * g] = e[i];
         }
+        if (kOne) l[g] += sum;
       }
       __builtin_amdgcn_wave_barrier();
+      // Operands of four steps are read while the previous four's products run.
+      float x[2][4][kQuads];
+      auto read4 = [&](int blk, float (&y)[4][kQuads]) __attribute__((always_inline)) {
 #pragma unroll
-      for (int j = 0; j < kGramChunk / 2; ++j) {
-        float x[4 * kRead];
-        const float* rp = L + my_key * kSgStride + kSgWidth * (kGramChunk / 2 * sl + j);
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int u = 0; u < kRead; ++u) {
-          const float4 v4 = *reinterpret_cast<const float4*>(rp + 4 * u);
-          x[4 * u] = v4.x;
-          x[4 * u + 1] = v4.y;
-          x[4 * u + 2] = v4.z;
-          x[4 * u + 3] = v4.w;
+          for (int u = 0; u < kQuads; ++u) y[i][u] = rp[2 * (4 * blk + i) * kSgStride + 4 * u];
+      };
+      read4(0, x[0]);
+#pragma unroll
+      for (int blk = 0; blk < 4; ++blk) {
+        if (blk < 3) read4(blk + 1, x[(blk + 1) & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          int p = 0;
+#pragma unroll
+          for (int u = 0; u < kQuads; ++u)
+#pragma unroll
+            for (int w = u; w < kQuads; ++w) {
+              acc[p] = mfma4x4(x[blk & 1][i][u], x[blk & 1][i][w], acc[p]);
+              ++p;
+            }
         }
-        int p = 0;
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+  };
+  // G of key frame f2 from v(p, i): the product sum of column 4 u + i and column 4 w + lane % 4 of
+  // the lane's position (p = the pair u <= w), added over the 8 positions.
+  auto write_g = [&](int f2, auto v) __attribute__((always_inline)) {
+    float* out = a.G + ((bh * F + f2) * a.n_chunks + chunk) * NP;
+    int p = 0;
 #pragma unroll
-        for (int f1 = 0; f1 < F; ++f1)
+    for (int u = 0; u < kQuads; ++u)
 #pragma unroll
-          for (int f3 = f1; f3 < F; ++f3) {
-            acc[p] = fmaf(x[f1], x[f3], acc[p]);
-            ++p;
+      for (int w = u; w < kQuads; ++w) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float sum = v(p, u, w, i);
+#pragma unroll
+          for (int o = 4; o < 32; o <<= 1) sum += __shfl_xor(sum, o);
+          const int f1 = 4 * u + i, f3 = 4 * w + (lane & 3);
+          if (lane < 4 && f1 <= f3 && f3 < F) out[f1 * F - f1 * (f1 - 1) / 2 + (f3 - f1)] = sum;
+        }
+        ++p;
+      }
+  };
+  // Columns that are no sample (f1 >= F, positions past ns) weigh nothing.
+  auto drop_unused = [&]() {
+#pragma unroll
+    for (int g = 0; g < kSgGroups; ++g) {
+      const int flat = 32 * g + col;
+      if (!(chunk * kGramChunk + flat / kSgWidth < a.ns && flat % kSgWidth < F)) inv[g] = 0.f;
+    }
+  };
+  sa_f32x4 acc[kPairs];
+  if constexpr (!kOne) {
+    reset();
+    stats(std::true_type{}, 0, n_tiles, a.keys);
+    merge_max();
+    finish();
+    drop_unused();
+    for (int f2 = 0; f2 < F; ++f2) {
+      frame(f2, acc);
+      write_g(f2, [&](int p, int, int, int i) { return acc[p][i] + __shfl_xor(acc[p][i], 32); });
+    }
+  } else {
+    float* ws = a.ws + wid * (F * 4 * kPairs * 32);
+    // Maxima over the first tile (after a failed walk: over every key), then the text keys' part of
+    // the sums, then every frame's products to ws and its sums to l.
+    for (int tiles = 1;; tiles = n_tiles) {
+      reset();
+      stats(std::true_type{}, 0, tiles, a.keys);
+      merge_max();
+#pragma unroll
+      for (int g = 0; g < kSgGroups; ++g) l[g] = 0.f;
+      stats(std::false_type{}, 0, (a.T + 31) / 32, a.T);
+      for (int f2 = 0; f2 < F; ++f2) {
+        frame(f2, acc);
+#pragma unroll
+        for (int p = 0; p < kPairs; ++p)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float sum = acc[p][i] + __shfl_xor(acc[p][i], 32);
+            if (lane < 32) ws[(f2 * 4 * kPairs + 4 * p + i) * 32 + lane] = sum;
           }
       }
-      __builtin_amdgcn_wave_barrier();
+      if (!finish() || tiles == n_tiles) break;
     }
-    // lanes' sums -> LDS [lane][pair] -> lane p adds pair p over the 64 lanes in order
+    drop_unused();
+    // The rows' factors by flat column; the lane's own stores to ws come back in order.
 #pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      L[lane * NP + p] = acc[p];
-      acc[p] = 0.f;
-    }
+    for (int g = 0; g < kSgGroups; ++g)
+      if (hh == 0) L[32 * g + col] = inv[g];
     __builtin_amdgcn_wave_barrier();
-    float* out = a.G + ((bh * F + f2) * a.n_chunks + chunk) * NP;
-    for (int p = lane; p < NP; p += 64) {
-      float sum = 0.f;
-      for (int q = 0; q < 64; ++q) sum += L[q * NP + p];
-      out[p] = sum;
+    const float* fp = L + kSgWidth * ((lane >> 2) & 7);
+    float fa[kQuads * 4], fb[kQuads];  // factors of the position's columns and of 4 w + lane % 4
+#pragma unroll
+    for (int c = 0; c < 4 * kQuads; ++c) fa[c] = fp[c];
+#pragma unroll
+    for (int w = 0; w < kQuads; ++w) fb[w] = fp[4 * w + (lane & 3)];
+    for (int f2 = 0; f2 < F; ++f2) {
+      float e[4 * kPairs];
+#pragma unroll
+      for (int p = 0; p < 4 * kPairs; ++p) e[p] = ws[(f2 * 4 * kPairs + p) * 32 + (lane & 31)];
+      write_g(f2, [&](int p, int u, int w, int i) { return e[4 * p + i] * fa[4 * u + i] * fb[w]; });
     }
-    __builtin_amdgcn_wave_barrier();
   }
 }
 
@@ -608,8 +1035,18 @@ __device__ float col_sim(const float* Gp, int F, int n_chunks, float* gs /* LDS 
   __syncthreads();
   for (int e = t; e < F * NP; e += 256) {
     const int f2 = e / NP, p = e - f2 * NP;
+    // Added in chunk order, eight loads at a time.
+    const float* gp = Gp + (int64_t)f2 * n_chunks * NP + p;
     float s = 0.f;
-    for (int c = 0; c < n_chunks; ++c) s += Gp[((int64_t)f2 * n_chunks + c) * NP + p];
+    int c = 0;
+    for (; c + 8 <= n_chunks; c += 8) {
+      float y[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) y[i] = gp[(int64_t)(c + i) * NP];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) s += y[i];
+    }
+    for (; c < n_chunks; ++c) s += gp[(int64_t)c * NP];
     gs[e] = s;
   }
   __syncthreads();
@@ -694,6 +1131,48 @@ extern "C" int sa_topk_share(const float* P, int64_t p_bh_stride, int64_t p_row_
   return sa::check_launch(fn);
 }
 
+extern "C" int sa_gather_key_operands(const uint16_t* x, const int64_t strides[3], int B, int H, int L, int D,
+                                      const int32_t* idx, int n_pad, uint16_t* out, void* stream) {
+  const char* fn = "sa_gather_key_operands";
+  SA_REQUIRE(x && strides && idx && out, "%s: null pointer", fn);
+  SA_REQUIRE(B > 0 && H > 0 && L > 0 && n_pad > 0 && n_pad % 32 == 0, "%s: bad shape (n_pad a multiple of 32)", fn);
+  if (D != kD) return sa::fail(SA_ERR_UNSUPPORTED, "%s: head_dim %d (64)", fn, D);
+  SA_REQUIRE(reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0,
+             "%s: x/out must be 16-byte aligned", fn);
+  for (int i = 0; i < 3; ++i)
+    if (strides[i] % 8 != 0) return sa::fail(SA_ERR_UNSUPPORTED, "%s: strides must be multiples of 8 elements", fn);
+  GatherOpsArgs a;
+  a.x = x; a.sb = strides[0]; a.sh = strides[1]; a.sl = strides[2]; a.H = H; a.L = L; a.idx = idx; a.n_pad = n_pad;
+  a.out = reinterpret_cast<jd_u32x4*>(out);
+  a.total = (int64_t)B * H * n_pad * 8;
+  SA_REQUIRE((a.total + 255) / 256 < (1LL << 31), "%s: grid too large", fn);
+  hipLaunchKernelGGL(gather_operands_kernel, dim3((unsigned)((a.total + 255) / 256)), dim3(256), 0,
+                     sa::as_stream(stream), a);
+  return sa::check_launch(fn);
+}
+
+extern "C" int sa_topk_mass(const uint16_t* q_rows, const uint16_t* k_ops, int BH, int rows, int rows_pad, int n,
+                            int n_pad, float sm_scale, int K, float* share, void* stream) {
+  const char* fn = "sa_topk_mass";
+  SA_REQUIRE(q_rows && k_ops && share, "%s: null pointer", fn);
+  SA_REQUIRE(reinterpret_cast<uintptr_t>(q_rows) % 16 == 0 && reinterpret_cast<uintptr_t>(k_ops) % 16 == 0,
+             "%s: q_rows/k_ops must be 16-byte aligned", fn);
+  SA_REQUIRE(BH > 0 && rows > 0 && n > 0 && K >= 1 && K <= n, "%s: bad shape (1 <= K <= n)", fn);
+  SA_REQUIRE(rows_pad % 32 == 0 && rows_pad >= rows && n_pad % 32 == 0 && n_pad >= n,
+             "%s: rows_pad/n_pad must be multiples of 32 covering rows/n", fn);
+  SA_REQUIRE(std::isfinite(sm_scale) && sm_scale > 0.f, "%s: bad sm_scale", fn);
+  if (n > 16384) return sa::fail(SA_ERR_UNSUPPORTED, "%s: n=%d > 16384", fn, n);
+  TopkMassArgs a;
+  a.qs = q_rows; a.ks = reinterpret_cast<const jd_u32x4*>(k_ops); a.rows = rows; a.rows_pad = rows_pad;
+  a.n = n; a.n_tiles = n_pad / 32; a.K = K; a.scale_log2 = sm_scale * kLog2e; a.share = share;
+  a.ng = (rows + 31) / 32;
+  a.BH = BH;
+  const int64_t grid = ((int64_t)BH + 7) / 8 * 8 * a.ng;
+  SA_REQUIRE(grid < (1LL << 31), "%s: grid too large", fn);
+  hipLaunchKernelGGL(topk_mass_kernel, dim3((unsigned)grid), dim3(64 * kTmWaves), 0, sa::as_stream(stream), a);
+  return sa::check_launch(fn);
+}
+
 extern "C" int sa_pattern_gram(const float* P, int64_t p_bh_stride, int64_t p_row_stride, int BH, int F, int ns,
                                float* G, void* stream) {
   const char* fn = "sa_pattern_gram";
@@ -732,9 +1211,10 @@ extern "C" int sa_pattern_judge_finish(const float* share, const float* G1, cons
   return sa::check_launch(fn);
 }
 
-extern "C" int sa_pattern_sim_gram(const uint16_t* q_rows, const uint16_t* k_rows, int BH, int F, int ns, int T,
-                                   int rows_pad, int keys_pad, float sm_scale, float bias, float* G, void* stream) {
-  const char* fn = "sa_pattern_sim_gram";
+namespace {
+
+int launch_sim_gram(const uint16_t* q_rows, const uint16_t* k_rows, int BH, int F, int ns, int T, int rows_pad,
+                    int keys_pad, float sm_scale, float bias, float* G, float* ws, void* stream, const char* fn) {
   SA_REQUIRE(q_rows && k_rows && G, "%s: null pointer", fn);
   SA_REQUIRE(reinterpret_cast<uintptr_t>(q_rows) % 16 == 0 && reinterpret_cast<uintptr_t>(k_rows) % 16 == 0,
              "%s: q_rows/k_rows must be 16-byte aligned", fn);
@@ -747,14 +1227,48 @@ extern "C" int sa_pattern_sim_gram(const uint16_t* q_rows, const uint16_t* k_row
   a.scale_log2 = sm_scale * kLog2e; a.bias_log2 = bias * kLog2e; a.G = G;
   a.n_chunks = (ns + kGramChunk - 1) / kGramChunk;
   a.total = (int64_t)BH * a.n_chunks;
+  a.ws = ws;
   const dim3 grid((unsigned)((a.total + 3) / 4)), blk(256);
   hipStream_t s = sa::as_stream(stream);
   switch (F) {
-#define SA_SG_CASE(n) \
-  case n: hipLaunchKernelGGL(simgram_kernel<n>, grid, blk, 0, s, a); break;
+#define SA_SG_CASE(n)                                                              \
+  case n:                                                                          \
+    if (ws) hipLaunchKernelGGL((simgram_kernel<n, true>), grid, blk, 0, s, a);     \
+    else hipLaunchKernelGGL((simgram_kernel<n, false>), grid, blk, 0, s, a);       \
+    break;
     SA_SG_CASE(1) SA_SG_CASE(2) SA_SG_CASE(3) SA_SG_CASE(4) SA_SG_CASE(5) SA_SG_CASE(6)
     SA_SG_CASE(7) SA_SG_CASE(8) SA_SG_CASE(9) SA_SG_CASE(10) SA_SG_CASE(11) SA_SG_CASE(12)
 #undef SA_SG_CASE
   }
   return sa::check_launch(fn);
+}
+
+}  // namespace
+
+extern "C" int sa_pattern_sim_gram(const uint16_t* q_rows, const uint16_t* k_rows, int BH, int F, int ns, int T,
+                                   int rows_pad, int keys_pad, float sm_scale, float bias, float* G, void* stream) {
+  return launch_sim_gram(q_rows, k_rows, BH, F, ns, T, rows_pad, keys_pad, sm_scale, bias, G, nullptr, stream,
+                         "sa_pattern_sim_gram");
+}
+
+extern "C" int sa_pattern_sim_gram_workspace(int BH, int F, int ns, int64_t* bytes) {
+  const char* fn = "sa_pattern_sim_gram_workspace";
+  SA_REQUIRE(bytes, "%s: null bytes", fn);
+  SA_REQUIRE(BH > 0 && F >= 1 && F <= 12 && ns > 0, "%s: bad shape (1 <= F <= 12)", fn);
+  *bytes = (int64_t)BH * ((ns + kGramChunk - 1) / kGramChunk) * F * 4 * sg_pairs(F) * 32 * 4;
+  return sa::ok();
+}
+
+extern "C" int sa_pattern_sim_gram_ws(const uint16_t* q_rows, const uint16_t* k_rows, int BH, int F, int ns, int T,
+                                      int rows_pad, int keys_pad, float sm_scale, float bias, float* G,
+                                      void* workspace, int64_t workspace_bytes, void* stream) {
+  const char* fn = "sa_pattern_sim_gram_ws";
+  int64_t need = 0;
+  if (int rc = sa_pattern_sim_gram_workspace(BH, F, ns, &need)) return rc;
+  SA_REQUIRE(workspace && reinterpret_cast<uintptr_t>(workspace) % 16 == 0, "%s: workspace null or not 16-byte aligned",
+             fn);
+  SA_REQUIRE(workspace_bytes >= need, "%s: workspace of %lld bytes < %lld", fn, (long long)workspace_bytes,
+             (long long)need);
+  return launch_sim_gram(q_rows, k_rows, BH, F, ns, T, rows_pad, keys_pad, sm_scale, bias, G,
+                         static_cast<float*>(workspace), stream, fn);
 }

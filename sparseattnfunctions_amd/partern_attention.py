@@ -23,6 +23,7 @@ keeps bf16 scores and softmax throughout); `ParternAttentionRowVersion` and the 
 """
 from __future__ import annotations
 
+import ctypes
 import math
 from dataclasses import dataclass
 
@@ -302,6 +303,21 @@ def _compact(x, idx, n_pad):
     return gather_tokens(x, full.to(x.device)).reshape(B * H, n_pad, 64)
 
 
+def _key_operands(x, idx, n_pad):
+    """Rows idx of x (bf16 [B,H,L,64]) in matrix-operand order (`sa_gather_key_operands`), zero
+    padded: as many bytes as [B*H, n_pad, 64]."""
+    full = torch.full((n_pad,), -1, dtype=torch.int32)
+    full[: idx.numel()] = idx.to(torch.int32)
+    full = full.to(x.device)
+    B, H, L, D = x.shape
+    out = torch.empty(B * H, n_pad, 64, dtype=x.dtype, device=x.device)
+    with torch.cuda.device(x.device):
+        _lib.check(_lib.load().sa_gather_key_operands(x.data_ptr(), _lib.i64(*x.stride()[:3]), B, H, L, D,
+                                                      full.data_ptr(), n_pad, out.data_ptr(), _lib.stream_of(x)),
+                   "sa_gather_key_operands")
+    return out
+
+
 def _probs(qs, ks, rows, keys, n_bias, bias, c_lo, c_hi, P, sm_scale: float = scale_factor):
     BH = qs.shape[0]
     with torch.cuda.device(qs.device):
@@ -321,16 +337,12 @@ def _sparsity_rows(q, k, g: PatternGeometry, idx_q):
     ns = idx_q.numel()
     keys = torch.arange(0, g.L, 3)
     n = keys.numel()
-    qs, ks = _compact(q, idx_q + g.text_length, _pad32(ns)), _compact(k, keys, _pad32(n))
-    K = int(n * SPARSE_KEEP)
+    qs, ks = _compact(q, idx_q + g.text_length, _pad32(ns)), _key_operands(k, keys, _pad32(n))
     share = torch.empty(B * H, ns, dtype=torch.float32, device=q.device)
-    # rows padded to whole 128-byte lines
-    for h0, h1 in _chunks(B * H, ns * _pad32(n) * 4):
-        P = torch.empty(h1 - h0, ns, _pad32(n), dtype=torch.float32, device=q.device)
-        _probs(qs[h0:h1], ks[h0:h1], ns, n, 0, 0.0, 0, n, P)
-        with torch.cuda.device(q.device):
-            _lib.check(_lib.load().sa_topk_share(P.data_ptr(), P.stride(0), P.stride(1), h1 - h0, ns, n, K,
-                                                 share[h0:h1].data_ptr(), _lib.stream_of(q)), "sa_topk_share")
+    with torch.cuda.device(q.device):
+        _lib.check(_lib.load().sa_topk_mass(qs.data_ptr(), ks.data_ptr(), B * H, ns, qs.shape[1], n, _pad32(n),
+                                            scale_factor, int(n * SPARSE_KEEP), share.data_ptr(),
+                                            _lib.stream_of(q)), "sa_topk_mass")
     return share
 
 
@@ -349,10 +361,14 @@ def _similarity_gram(q, k, g: PatternGeometry, index_k):
     computed without writing the probabilities (one fused kernel)."""
     T, F, ns = g.text_length, g.frames, g.sample_num
     qs, ks, G = _similarity_inputs(q, k, g, index_k)
+    n = ctypes.c_int64(0)
+    lib = _lib.load()
+    _lib.check(lib.sa_pattern_sim_gram_workspace(qs.shape[0], F, ns, ctypes.byref(n)), "sa_pattern_sim_gram_workspace")
+    ws = torch.empty(n.value, dtype=torch.uint8, device=q.device)  # each position's products, until its sums are known
     with torch.cuda.device(q.device):
-        _lib.check(_lib.load().sa_pattern_sim_gram(
+        _lib.check(lib.sa_pattern_sim_gram_ws(
             qs.data_ptr(), ks.data_ptr(), qs.shape[0], F, ns, T, qs.shape[1], ks.shape[1], scale_factor,
-            composition_bias(g), G.data_ptr(), _lib.stream_of(q)), "sa_pattern_sim_gram")
+            composition_bias(g), G.data_ptr(), ws.data_ptr(), ws.numel(), _lib.stream_of(q)), "sa_pattern_sim_gram_ws")
     return G
 
 
