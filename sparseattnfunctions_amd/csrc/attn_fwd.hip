@@ -79,8 +79,9 @@ struct FwdArgs {
   int64_t o_sb, o_sh, o_sl;
   int H, Lq, Lk, nqb, nkb;
   int n_items;             // B*H*nqb
-  const int32_t* order;    // dispatch slot -> item (bh*nqb + qb), -1 = idle; may be null
+  const int32_t* order;    // dispatch slot -> item (bh*nqb + qb), -1 = idle; may be null: xcd_item
   int n_slots;
+  int longest_last;        // without an order: each XCD's items in descending order
   // Key-range split (n_parts > 1; plain lists only): slot (bh * n_parts + p) * nqb + qb
   // computes list positions [cnt * p / n_parts, cnt * (p + 1) / n_parts) of item bh * nqb + qb
   // and stores its unnormalised partial to ws[item * n_parts + p] (kSplitFloats each: acc
@@ -88,6 +89,7 @@ struct FwdArgs {
   // forms the output. `order` is not read.
   int n_parts;
   float* ws;
+  int shared_from;  // kShare: the first dispatch group whose items are shared by four waves each
   const int32_t* kv_idx;
   const int32_t* kv_cnt;
   int max_cnt;
@@ -124,6 +126,16 @@ struct FwdArgs {
   const uint16_t* k16;
   const uint32_t* k16_norm2;
 };
+
+// Item of a dispatch slot without a work order: as sa_attn_work_order places them, each XCD (group
+// w of four slots runs on XCD w % 8) a contiguous range of items; -1 = idle.
+__device__ inline int xcd_item(const FwdArgs& a, int slot) {
+  const int w = slot / kWaves, x = w & 7;
+  const int lo = (int)(((int64_t)a.n_items * x) >> 3), hi = (int)(((int64_t)a.n_items * (x + 1)) >> 3);
+  const int i = (w >> 3) * kWaves + slot % kWaves;
+  if (i >= hi - lo) return -1;
+  return a.longest_last ? hi - 1 - i : lo + i;
+}
 
 __device__ inline sa_bf16x8 as_bf16x8(uint4 x) { return __builtin_bit_cast(sa_bf16x8, x); }
 __device__ inline sa_bf16x8 as_bf16x8(sa_u32x4v x) { return __builtin_bit_cast(sa_bf16x8, x); }
@@ -284,7 +296,11 @@ constexpr int kWaitLgkm0 = 0xC07F;
 // launches.)
 // kDV: value columns that enter P.V and the output, kD or 32 (head dim 64: v tiles are
 // copied as usual and only their first 32 columns are read; out has 32 columns).
-template <bool kBias, bool kMask, int kPool, typename T = __bf16, int kD = 64, int kDV = kD, bool kK16 = false>
+// kShare (head dim 64): the items of dispatch groups from shared_from on are each
+// shared by the four waves of a workgroup, wave p taking list positions [cnt p / 4, cnt (p + 1) / 4)
+// and all merging their partials through the LDS of their tiles; see shared_groups for when.
+template <bool kBias, bool kMask, int kPool, typename T = __bf16, int kD = 64, int kDV = kD, bool kK16 = false,
+          bool kShare = false>
 __global__ __launch_bounds__(256, kD == 64 ? 2 : 1) void bsa_fwd_kernel(FwdArgs a) {
   static_assert(!kK16 || (!kMask && kPool == 0 && std::is_same<T, __bf16>::value && kD == 64 && kDV == 64),
                 "fp16 scores: plain or key-bias bf16 lists at head dim 64");
@@ -293,6 +309,8 @@ __global__ __launch_bounds__(256, kD == 64 ? 2 : 1) void bsa_fwd_kernel(FwdArgs 
   static_assert(kPool == 0 || ((kPool == 32 || kPool == 64) && !kBias), "pooling: 32- or 64-key columns, no bias");
   static_assert(kD == 64 || kD == 128, "head dim 64 or 128");
   static_assert(kDV == kD || (kDV == 32 && kD == 64 && kPool == 0 && !kMask), "32 value columns: head dim 64");
+  static_assert(!kShare || (kD == 64 && !(kMask && kPool != 0)),
+                "shared items: head dim 64; the causal pooling loop runs 4 % slower with them");
   typedef Elem<T> E;
   constexpr int kDS = kD / 16;     // 16-wide d steps of S = K Q^T
   constexpr int kDC = kDV / 32;    // 32-row d chunks of O^T
@@ -319,10 +337,16 @@ __global__ __launch_bounds__(256, kD == 64 ? 2 : 1) void bsa_fwd_kernel(FwdArgs 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 31;  // query column within a 32-row group (MFMA n index)
   const int hh = lane >> 5;   // lane half (MFMA k group)
-  const int slot = blockIdx.x * kWaves + wave;
+  __shared__ float ml_lds[kShare ? kWaves : 1][2][kBlock];  // row maxima and sums of the partials
+  const bool shared = kShare && (int)blockIdx.x >= a.shared_from;
+  int slot = blockIdx.x * kWaves + wave;
+  if (shared) {  // a shared group is four workgroups, on the group's XCD
+    const int y = blockIdx.x - a.shared_from;
+    slot = 4 * (a.shared_from + 8 * (y >> 5) + (y & 7)) + ((y >> 3) & 3);
+  }
   if (slot >= a.n_slots) return;
   // Key-range parts exist for plain lists only; the other variants compile without them.
-  constexpr bool kSplit = !kBias && !kMask && kPool == 0 && kDV == kD && !kK16;
+  constexpr bool kSplit = !kBias && !kMask && kPool == 0 && kDV == kD && !kK16 && !kShare;
   const bool split = kSplit && a.n_parts > 1;
   int item, part = 0;
   if (split) {
@@ -332,9 +356,10 @@ __global__ __launch_bounds__(256, kD == 64 ? 2 : 1) void bsa_fwd_kernel(FwdArgs 
     part = rem / a.nqb;
     item = bh_s * a.nqb + (rem - part * a.nqb);
   } else {
-    item = __builtin_amdgcn_readfirstlane(a.order ? a.order[slot] : slot);
+    item = __builtin_amdgcn_readfirstlane(a.order ? a.order[slot] : xcd_item(a, slot));
   }
-  if (item < 0 || item >= a.n_items) return;  // idle slot (no workgroup barriers below)
+  // Idle slot. (The only barriers below are a shared item's, whose waves all take the same branch.)
+  if (item < 0 || item >= a.n_items) return;
   const int bh = item / a.nqb;
   const int qb = item - bh * a.nqb;
   const int b = bh / a.H;
@@ -347,6 +372,10 @@ __global__ __launch_bounds__(256, kD == 64 ? 2 : 1) void bsa_fwd_kernel(FwdArgs 
   if (split) {
     beg = cnt * part / a.n_parts;
     cnt = cnt * (part + 1) / a.n_parts;
+  }
+  if (shared) {
+    beg = (cnt * wave) >> 2;
+    cnt = (cnt * (wave + 1)) >> 2;
   }
   __builtin_assume(beg >= 0);
   // Constant address space: the compiler may use scalar loads (nothing here writes them).
@@ -875,10 +904,83 @@ __global__ __launch_bounds__(256, kD == 64 ? 2 : 1) void bsa_fwd_kernel(FwdArgs 
     if (__ballot(bad) != 0) run_item(std::true_type{}, false);
   }
 
+  if (shared) {
+    // ---- Partials to LDS: rows 0 .. 31 over the wave's K tile, rows 32 .. 63 over its V tile
+    // (both read out, and no copy is in flight), 16-byte chunks XOR-swizzled by the row.
+    constexpr int kCh = kDV / 4;  // chunks per row
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      float* w = reinterpret_cast<float*>(g ? v_lds + wave * kTileBytes : k_lds + wave * kTileBytes);
+      const float l_tot = xhalf_sum(l[g]);
+#pragma unroll
+      for (int dc = 0; dc < kDC; ++dc)
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4) {
+          const sa_f32x16& A = acc[dc][g];
+          *reinterpret_cast<float4*>(w + col * kDV + 4 * ((8 * dc + 2 * q4 + hh) ^ (col & (kCh - 1)))) =
+              make_float4(A[4 * q4], A[4 * q4 + 1], A[4 * q4 + 2], A[4 * q4 + 3]);
+        }
+      if (hh == 0) {
+        // Offset 0 of a fast pass; a wave without a key of the row has nothing to weigh.
+        ml_lds[kShare ? wave : 0][0][32 * g + col] = l_tot == 0.f ? -INFINITY : (m[g] == -INFINITY ? 0.f : m[g]);
+        ml_lds[kShare ? wave : 0][1][32 * g + col] = l_tot;
+      }
+    }
+    __syncthreads();
+    // ---- out = sum_p 2^(m_p - M) acc_p / sum_p 2^(m_p - M) l_p, in list order; each wave takes
+    // 16 rows, kCh lanes per row.
+    const int ch = lane % kCh;
+    constexpr int kStep = 64 / kCh;  // rows per pass
+    for (int r = 16 * wave + lane / kCh; r < 16 * (wave + 1); r += kStep) {
+      float M = -INFINITY;
+#pragma unroll
+      for (int p = 0; p < 4; ++p) M = fmaxf(M, ml_lds[p % (kShare ? 4 : 1)][0][r]);
+      float lsum = 0.f;
+      float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const int wv = p % (kShare ? 4 : 1);
+        const float mp = ml_lds[wv][0][r];
+        const float f = mp == -INFINITY ? 0.f : fast_exp2(mp - M);
+        const float* w = reinterpret_cast<const float*>((r >= 32 ? v_lds : k_lds) + p * kTileBytes);
+        const float4 x = *reinterpret_cast<const float4*>(w + (r & 31) * kDV + 4 * (ch ^ (r & (kCh - 1))));
+        lsum = fmaf(f, ml_lds[wv][1][r], lsum);
+        o.x = fmaf(f, x.x, o.x);
+        o.y = fmaf(f, x.y, o.y);
+        o.z = fmaf(f, x.z, o.z);
+        o.w = fmaf(f, x.w, o.w);
+      }
+      const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
+      int row = qb * kBlock + r;
+      bool store = row < a.Lq;
+      if (store && a.o_rows) {
+        row = a.o_rows[row];
+        store = (unsigned)row < (unsigned)a.o_dst_rows;
+      }
+      if (store)
+        *reinterpret_cast<uint2*>(obase + (int64_t)row * a.o_sl + 4 * ch) =
+            make_uint2(E::pack(o.x * inv, o.y * inv), E::pack(o.z * inv, o.w * inv));
+    }
+    if constexpr (kPool == 0) return;
+  }
+
   // ---- Epilogue: out = acc / l (each lane half holds a partial l of its keys).
   float row_lse = 0.f;  // pooling: log2-sum-exp2 of row qb * 64 + lane
+  if (shared) {  // pooling: the row's merged log2-sum-exp2, in every wave
+    float M = -INFINITY, lsum = 0.f;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) M = fmaxf(M, ml_lds[p % (kShare ? 4 : 1)][0][lane]);
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const float mp = ml_lds[p % (kShare ? 4 : 1)][0][lane];
+      lsum = fmaf(mp == -INFINITY ? 0.f : fast_exp2(mp - M), ml_lds[p % (kShare ? 4 : 1)][1][lane], lsum);
+    }
+    row_lse = (M == -INFINITY ? 0.f : M) + log2f(lsum);
+    if (kPool != 0 && a.pool_lse && wave == 0) a.pool_lse[(int64_t)bh * a.pool_lpad + qb * kBlock + lane] = row_lse;
+  }
 #pragma unroll
   for (int g = 0; g < 2; ++g) {
+    if (shared) break;
     const float l_tot = xhalf_sum(l[g]);
     if (split) {  // partial of a key-range part: acc, row sum, row max (0 in the fast pass)
       float* w = a.ws + ((int64_t)item * a.n_parts + part) * kSplitFloats<kD>;
@@ -949,7 +1051,9 @@ __global__ __launch_bounds__(256, kD == 64 ? 2 : 1) void bsa_fwd_kernel(FwdArgs 
       float* po = a.pool_po + b * a.po_sb + h * a.po_sh + (int64_t)min(pr, a.pool_nd - 1) * a.po_si;
       const int j_lane = lane & 31;
       float tot = 0.f;  // this lane's columns, then summed over the 32 lanes
-      for (int c0 = 0; c0 < ncol; c0 += 32) {
+      // The waves of a shared item take the column chunks in turn (every wave's maxima are in
+      // memory since the barrier above).
+      for (int c0 = shared ? 32 * wave : 0; c0 < ncol; c0 += shared ? 128 : 32) {
         // Every load is issued (at a computed column, clamped) before any is used.
         float x[32];
 #pragma unroll
@@ -974,8 +1078,15 @@ __global__ __launch_bounds__(256, kD == 64 ? 2 : 1) void bsa_fwd_kernel(FwdArgs 
       }
 #pragma unroll
       for (int o = 16; o >= 1; o >>= 1) tot += __shfl_xor(tot, o);
+      if (shared) {
+        float* tp = &ml_lds[0][0][0];  // read out by every wave before the barrier
+        __syncthreads();
+        if (j_lane == 0) tp[2 * wave + hh] = tot;
+        __syncthreads();
+        tot = ((tp[hh] + tp[2 + hh]) + tp[4 + hh]) + tp[6 + hh];
+      }
       if (writer) {
-        for (int c = j_lane; c < ncol; c += 32) po[c] = po[c] / tot;
+        for (int c = j_lane + (shared ? 32 * wave : 0); c < ncol; c += shared ? 128 : 32) po[c] = po[c] / tot;
       }
     }
   }
@@ -1020,7 +1131,7 @@ __global__ __launch_bounds__(128, 2) void bsa_fwd_pair_kernel(FwdArgs a) {
   const int x = blockIdx.x;
   const int slot = 4 * (8 * (x >> 5) + (x & 7)) + ((x >> 3) & 3);
   int item = -1;
-  if (slot < a.n_slots) item = __builtin_amdgcn_readfirstlane(a.order ? a.order[slot] : slot);
+  if (slot < a.n_slots) item = __builtin_amdgcn_readfirstlane(a.order ? a.order[slot] : xcd_item(a, slot));
   // Both waves take the same branch: no barrier is left unmatched.
   if (item < 0 || item >= a.n_items) return;
   const int bh = item / a.nqb;
@@ -1472,11 +1583,56 @@ size_t split_workspace_bytes(int64_t n_items, int D, int parts) {
   return (size_t)n_items * parts * (D == 64 ? kSplitFloats<64> : kSplitFloats<128>) * sizeof(float);
 }
 
+// The first dispatch group (of four slots) whose items four waves share (none: the number of
+// groups). The card holds 2 048 of these waves, two per SIMD; a last round of less than one wave
+// per SIMD runs for a whole item's time at a fraction of the card. So the whole multiples of 1 024
+// slots run one wave per item and a remainder of up to kShareMax slots is shared, four short waves
+// per item. Measured at head dim 64, one wave per item against the remainder shared (us; dense
+// lists of 40 tiles, in brackets a fifth of them): remainder 16 of 1 040 slots 79 / 56, 112 of 2 160
+// 128 / 99 (47 / 40), 352 of 2 400 129 / 113 (50 / 43), 592 of 2 640 131 / 123 (49 / 48), 832 of
+// 2 880 134 / 135 (51 / 51), 976 of 2 000 94 / 96 (41 / 42); [2, 30, 13776, 64] merged-token
+// attention 3.60 / 3.49 ms. Two waves per item, or every item shared: slower than one from 8 tiles
+// per item down (316 -> 339 us, [2, 30, 12000, 64] with a tenth of the blocks).
+constexpr int64_t kShareRound = 1024;
+constexpr int64_t kShareMax = 704;
+
+int shared_from(int64_t n_slots) {
+  const int64_t left = n_slots % kShareRound;
+  return (int)((left > 0 && left <= kShareMax ? n_slots - left : n_slots) / kWaves);
+}
+
+template <bool kBias, bool kMask, typename T, int kDV, bool kK16, int kPool = 0>
+void launch_shared(FwdArgs a, int from, hipStream_t s) {
+  a.shared_from = from;
+  const int64_t left = a.n_slots / kWaves - from;
+  const dim3 g((unsigned)(from + (left + 7) / 8 * 32)), blk(64 * kWaves);
+  hipLaunchKernelGGL((bsa_fwd_kernel<kBias, kMask, kPool, T, 64, kDV, kK16, true>), g, blk, 0, s, a);
+}
+
 // One kernel variant per (tile masks, key bias, pooling columns): the caller has rejected
 // the combinations of tile masks or pooling with a key bias.
 template <typename T, int kD>
 void launch_variant(const FwdArgs& a, dim3 g, dim3 blk, hipStream_t s, bool mask, bool bias, int pool_cols,
                     bool v32 = false) {
+  if constexpr (kD == 64) {
+    const bool may_share = a.n_parts == 1 && !(mask && pool_cols);
+    const int from = may_share ? shared_from(a.n_slots) : a.n_slots / kWaves;
+    if (from < a.n_slots / kWaves) {
+      if (pool_cols == 32) return launch_shared<false, false, T, 64, false, 32>(a, from, s);
+      if (pool_cols == 64) return launch_shared<false, false, T, 64, false, 64>(a, from, s);
+      if constexpr (std::is_same<T, __bf16>::value) {
+        if (a.k16)
+          return bias ? launch_shared<true, false, T, 64, true>(a, from, s)
+                      : launch_shared<false, false, T, 64, true>(a, from, s);
+        if (v32)
+          return bias ? launch_shared<true, false, T, 32, false>(a, from, s)
+                      : launch_shared<false, false, T, 32, false>(a, from, s);
+      }
+      if (mask) return launch_shared<false, true, T, 64, false>(a, from, s);
+      return bias ? launch_shared<true, false, T, 64, false>(a, from, s)
+                  : launch_shared<false, false, T, 64, false>(a, from, s);
+    }
+  }
   if constexpr (kD == 64 && std::is_same<T, __bf16>::value) {
     if (a.k16) {  // fp16 scores (the caller has rejected every mode but the key bias)
       if (bias) hipLaunchKernelGGL((bsa_fwd_kernel<true, false, 0, T, kD, kD, true>), g, blk, 0, s, a);
@@ -1543,8 +1699,8 @@ int launch_fwd(const uint16_t* q, const int64_t q_strides[3], const uint16_t* k,
   SA_REQUIRE(n_items < (1LL << 30), "%s: too many query blocks", fn);
   if (work_order) {
     SA_REQUIRE(n_slots > 0 && n_slots % kWaves == 0, "%s: n_slots must be a positive multiple of 4", fn);
-  } else {
-    n_slots = (n_items + kWaves - 1) / kWaves * kWaves;
+  } else {  // xcd_item: each of the eight XCDs' ranges in whole groups
+    n_slots = ((n_items + 7) / 8 + kWaves - 1) / kWaves * 8 * kWaves;
   }
   // 16-byte vector accesses: base pointers 16-byte aligned, row strides multiples of 8 elements.
   const void* ptrs[4] = {q, k, v, out};
@@ -1576,6 +1732,9 @@ int launch_fwd(const uint16_t* q, const int64_t q_strides[3], const uint16_t* k,
   a.n_items = (int)n_items;
   a.order = work_order;
   a.n_slots = (int)n_slots;
+  // Causal lists grow with the query block: the longest start first (and each XCD keeps to its
+  // heads: [2, 30, 17776, 64] pooled 3.29 -> 3.06 ms, in ascending order 3.25).
+  a.longest_last = pool_cols && kv_slot ? 1 : 0;
   a.n_parts = 1;
   a.ws = nullptr;
   a.k16 = k16;
