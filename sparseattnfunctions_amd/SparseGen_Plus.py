@@ -119,7 +119,11 @@ class BlockSparseAttention:
     def _calculate_sparsity(self, kv: KVList):
         """Fraction of skipped blocks; with B == 1 the reference scores the layer as if the
         other 96 - H heads were 90 % sparse (:126-132)."""
-        kept = kv.cnt.sum().item() / (kv.rows * kv.nkb)
+        return self._sparsity_of(kv, kv.cnt.sum().item())
+
+    @staticmethod
+    def _sparsity_of(kv: KVList, kept_blocks: int):
+        kept = kept_blocks / (kv.rows * kv.nkb)
         if kv.B == 1:
             return ((1 - kept) * kv.H + 0.9 * (96 - kv.H)) / 96
         return 1 - kept
@@ -150,8 +154,14 @@ class BlockSparseAttention:
         kv = transfer_attn_to_kv_list(pool, mode="energy", init_k=cur_k, max_retain_ratio=max_r,
                                       min_retain_ratio=min_r, energy_threshold=thr)
         self.mask[layer] = kv
+        # The record's block count is copied out before the attention is launched, so that the wait
+        # for it ends while the attention runs and the next layer's launches are not held up.
+        kept = kv.cnt.sum().to("cpu", non_blocking=True)
+        counted = torch.cuda.Event()
+        counted.record(torch.cuda.current_stream(q.device))
         out = block_sparse_attention(q, k, v, kv, self.sm_scale, n_text_blocks=N_TEXT_BLOCKS)
-        sparsity = self._calculate_sparsity(kv)
+        counted.synchronize()
+        sparsity = self._sparsity_of(kv, kept.item())
         self._record_sparsity(self.counter // (self.layernum * self.timestep), self.counter // self.layernum,
                               self.counter % self.layernum, sparsity)
         return out

@@ -16,7 +16,7 @@ def gather_tokens(x: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
     idx = idx.to(torch.int32).contiguous()
     B, H, L, D = x.shape
     out = torch.empty(B, H, idx.numel(), D, dtype=x.dtype, device=x.device)
-    with torch.cuda.device(x.device):
+    with _lib.on(x.device):
         rc = _lib.load().sa_gather_tokens(x.data_ptr(), _lib.i64(*x.stride()[:3]), B, H, L, D, idx.data_ptr(),
                                           idx.numel(), out.data_ptr(), _lib.i64(*out.stride()[:3]), _lib.stream_of(x))
     _lib.check(rc, "sa_gather_tokens")

@@ -80,7 +80,7 @@ def kv_list_from_mask(mask: torch.Tensor, B: int, H: int, nqb: int, nkb: int) ->
     m8 = m8.expand(B, H, m8.shape[2], m8.shape[3])
     kv = KVList.empty(B, H, nqb, nkb, mask.device)
     lib = _lib.load()
-    with torch.cuda.device(mask.device):
+    with _lib.on(mask.device):
         rc = lib.sa_mask_to_kv_list(
             m8.data_ptr(), _lib.i64(*m8.stride()), B, H, nqb, nkb,
             kv.idx.data_ptr(), kv.max_cnt, kv.cnt.data_ptr(), _lib.stream_of(mask),

@@ -198,8 +198,12 @@ def check(rc: int, what: str) -> None:
     raise SAError(msg)
 
 
+_I64_ARRAYS = {n: ctypes.c_int64 * n for n in range(1, 10)}
+
+
 def i64(*vals: int):
-    return (ctypes.c_int64 * len(vals))(*[int(x) for x in vals])
+    n = len(vals)
+    return (_I64_ARRAYS[n] if n in _I64_ARRAYS else ctypes.c_int64 * n)(*vals)
 
 
 def ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -221,7 +225,24 @@ def side_stream(device) -> "torch.cuda.Stream":
 
 def stream_of(t: torch.Tensor) -> int:
     """The current HIP stream of the tensor's device (hipStream_t as an integer)."""
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
+
+
+class _Here:
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        return False
+
+
+_HERE_CONTEXT = _Here()
+
+
+def on(device: torch.device):
+    """`torch.cuda.device(device)` for a GPU tensor's device; nothing to enter or leave when it is
+    the current one already (a launch's host path is some tens of microseconds, the switch 2-3)."""
+    return _HERE_CONTEXT if device.index == torch._C._cuda_getDevice() else torch.cuda.device(device)
 
 
 def require_gpu(*tensors: torch.Tensor) -> None:

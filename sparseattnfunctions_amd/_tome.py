@@ -67,7 +67,7 @@ def metric_from_qkv(k, v=None, text_len: int = 226, mode: int = 0) -> torch.Tens
     B, H, L, D = k.shape
     N = L - text_len
     out = torch.empty((B, N, 64) if mode == 0 else (B * H, N, 130), dtype=torch.float32, device=k.device)
-    with torch.cuda.device(k.device):
+    with _lib.on(k.device):
         rc = _lib.load().sa_tome_metric(k.data_ptr(), _lib.i64(*k.stride()[:3]), _lib.ptr(v),
                                         _lib.i64(*v.stride()[:3]) if v is not None else None, B, H, L, D, text_len,
                                         mode, out.data_ptr(), _lib.stream_of(k))
@@ -81,7 +81,7 @@ def normalize(metric: torch.Tensor) -> torch.Tensor:
     x = metric.to(torch.float32).contiguous()
     out = torch.empty_like(x)
     rows = x.numel() // x.shape[-1]
-    with torch.cuda.device(x.device):
+    with _lib.on(x.device):
         rc = _lib.load().sa_tome_normalize(x.data_ptr(), rows, x.shape[-1], out.data_ptr(), _lib.stream_of(x))
     _lib.check(rc, "sa_tome_normalize")
     return out
@@ -132,7 +132,7 @@ def match(metric: torch.Tensor, a_idx: torch.Tensor, b_idx: torch.Tensor, r: int
                "sa_tome_match_workspace")
     ws = torch.empty(max(ws_bytes.value, 1), dtype=torch.uint8, device=metric.device)
     metric = metric.contiguous()
-    with torch.cuda.device(metric.device):
+    with _lib.on(metric.device):
         rc = lib.sa_tome_match(metric.data_ptr(), C, ctypes.byref(maps.struct), ws.data_ptr(), ws.numel(),
                                _lib.stream_of(metric))
     _lib.check(rc, "sa_tome_match")
@@ -165,7 +165,7 @@ def match_noalloc(metric: torch.Tensor, a_idx: torch.Tensor, b_idx: torch.Tensor
     prev = _NOALLOC_LAST.get(key)
     if prev is not None and not capturing:
         stream.wait_event(prev)
-    with torch.cuda.device(dev):
+    with _lib.on(dev):
         rc = _lib.load().sa_tome_match_noalloc(metric.data_ptr(), C, ctypes.byref(maps.struct), stream.cuda_stream)
     _lib.check(rc, "sa_tome_match_noalloc")
     if not capturing:
@@ -181,7 +181,7 @@ def _apply(fn_name, x, maps: TomeMaps, heads_per_group: int, rows_out: int, out:
     B, H, _, D = x.shape
     if out is None:
         out = torch.empty(B, H, rows_out, D, dtype=x.dtype, device=x.device)
-    with torch.cuda.device(x.device):
+    with _lib.on(x.device):
         rc = getattr(_lib.load(), fn_name)(x.data_ptr(), _lib.i64(*x.stride()[:3]), B, H, D, heads_per_group,
                                            ctypes.byref(maps.struct), out.data_ptr(), _lib.i64(*out.stride()[:3]),
                                            _lib.stream_of(x))
@@ -215,7 +215,7 @@ def merge_many(xs, maps: TomeMaps, heads_per_group: int):
     op = (ctypes.c_void_p * n)(*[o.data_ptr() for o in outs])
     xst = _lib.i64(*[s for x in xs for s in x.stride()[:3]])
     ost = _lib.i64(*[s for o in outs for s in o.stride()[:3]])
-    with torch.cuda.device(xs[0].device):
+    with _lib.on(xs[0].device):
         rc = _lib.load().sa_tome_merge_multi(n, xp, xst, B, H, D, heads_per_group, ctypes.byref(maps.struct), op, ost,
                                              _lib.stream_of(xs[0]))
     _lib.check(rc, "sa_tome_merge_multi")

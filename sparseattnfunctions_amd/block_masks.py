@@ -48,13 +48,13 @@ def pool_blocks(q: torch.Tensor, k: Optional[torch.Tensor] = None, block: int = 
     if k16_ws is not None:
         if k is None or block != 64:
             raise ValueError("pool_blocks: k16_ws needs k and 64-token blocks")
-        with torch.cuda.device(q.device):
+        with _lib.on(q.device):
             rc = lib.sa_block_pool_k16(q.data_ptr(), _lib.i64(*q.stride()[:3]), k.data_ptr(), _lib.i64(*k.stride()[:3]),
                                        B, H, L, D, qp.data_ptr(), kp.data_ptr(), k16_ws.data_ptr(), k16_ws.numel(),
                                        _lib.stream_of(q))
         _lib.check(rc, "sa_block_pool_k16")
         return qp, kp
-    with torch.cuda.device(q.device):
+    with _lib.on(q.device):
         rc = lib.sa_block_pool(
             q.data_ptr(), _lib.i64(*q.stride()[:3]),
             _lib.ptr(k), _lib.i64(*k.stride()[:3]) if k is not None else None,
@@ -89,7 +89,7 @@ def topk_kv_list(q_pooled, k_pooled, B: int, H: int, topk: int, n_text_blocks: i
             raise ValueError(f"local bitmap {tuple(local_bitmap.shape)} != ({nqb}, {nkb})")
         loc = local_bitmap.to(device=dev, dtype=torch.uint8).contiguous()
     lib = _lib.load()
-    with torch.cuda.device(dev):
+    with _lib.on(dev):
         rc = lib.sa_block_topk_kv_list(
             _lib.ptr(q_pooled), _lib.ptr(k_pooled), _lib.ptr(scores_in), B * H, nqb, nkb, D,
             int(topk), int(n_text_blocks), _lib.ptr(loc), kv.idx.data_ptr(), kv.max_cnt,

@@ -68,7 +68,7 @@ def sample_block_tokens(q: torch.Tensor, k: Optional[torch.Tensor] = None, num_k
     if k is not None:
         ks = torch.empty_like(qs)
         tk = torch.empty_like(tq)
-    with torch.cuda.device(q.device):
+    with _lib.on(q.device):
         rc = _lib.load().sa_sample_block_tokens(
             rand_q.data_ptr(), q.data_ptr(), _lib.i64(*q.stride()[:3]),
             _lib.ptr(rand_k), _lib.ptr(k), _lib.i64(*k.stride()[:3]) if k is not None else None,
@@ -87,7 +87,7 @@ def sampled_block_scores(q: torch.Tensor, k: torch.Tensor, num_keep: int = 16,
     nb = math.ceil(L / BLOCK)
     qs, ks, _, _ = sample_block_tokens(q, k, num_keep, rand_q, rand_k, generator)
     pooled = torch.empty(B, H, nb, nb, dtype=torch.float32, device=q.device)
-    with torch.cuda.device(q.device):
+    with _lib.on(q.device):
         rc = _lib.load().sa_sampled_block_scores(qs.data_ptr(), ks.data_ptr(), B * H, nb, int(num_keep),
                                                  qs.shape[1], pooled.data_ptr(), _lib.stream_of(q))
     _lib.check(rc, "sa_sampled_block_scores")
@@ -127,7 +127,7 @@ def energy_kv_list(scores: torch.Tensor, mode: str = "energy", init_k=None, max_
     s = scores.to(torch.float32).contiguous()
     kv = KVList.empty(B, H, nqb, nkb, s.device)
     mask = torch.empty(B, H, nqb, nkb, dtype=torch.uint8, device=s.device) if return_mask else None
-    with torch.cuda.device(s.device):
+    with _lib.on(s.device):
         rc = _lib.load().sa_energy_kv_list(
             s.data_ptr(), B * H, nqb, nkb, MODES[mode], float(energy_threshold), min_keep, max_keep, k0,
             int(n_text_blocks), kv.idx.data_ptr(), kv.max_cnt, kv.cnt.data_ptr(), _lib.ptr(mask),
@@ -150,7 +150,7 @@ def energy_mask(scores: torch.Tensor, mode: str, threshold: float) -> torch.Tens
     s = scores.to(torch.float32).contiguous()
     kv = KVList.empty(G, 1, rows, n, s.device)
     mask = torch.empty(G, rows, n, dtype=torch.uint8, device=s.device)
-    with torch.cuda.device(s.device):
+    with _lib.on(s.device):
         rc = _lib.load().sa_energy_kv_list(
             s.data_ptr(), G, rows, n, CUT_MODES[mode], float(threshold), 0, n, 1, 0, kv.idx.data_ptr(), kv.max_cnt,
             kv.cnt.data_ptr(), mask.data_ptr(), _lib.stream_of(s))

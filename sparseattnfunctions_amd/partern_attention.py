@@ -195,7 +195,7 @@ class ParternAttentionColVersion_V2:
         q_idx = torch.empty(BH, F * S, dtype=torch.int32, device=dev)
         lib = _lib.load()
         stream = _lib.stream_of(q)
-        with torch.cuda.device(dev):
+        with _lib.on(dev):
             _lib.check(lib.sa_pattern_plan(
                 ff_mass.data_ptr(), _lib.i64(*ff_mass.stride()[:3]), i2i.data_ptr(), B, H, F, S, T,
                 0.01, 100.0, 0.05, 100.0, 0.1, stats.data_ptr(), fac.data_ptr(), case.data_ptr(), inv0.data_ptr(),
@@ -222,7 +222,7 @@ class ParternAttentionColVersion_V2:
                                        out=o_frames[:, :, rows])
         main.wait_stream(side)
         o_text.record_stream(main)
-        with torch.cuda.device(dev):
+        with _lib.on(dev):
             _lib.check(lib.sa_pattern_combine(
                 o_frames.data_ptr(), _lib.i64(*o_frames.stride()[:3]), o_text.data_ptr(),
                 _lib.i64(*o_text.stride()[:3]), ff_mass.data_ptr(), _lib.i64(*ff_mass.stride()[:3]),
@@ -237,7 +237,7 @@ class ParternAttentionColVersion_V2:
         B, H = mass.shape[:2]
         i2t = torch.empty(B, H, g.frames, 1, dtype=torch.float32, device=mass.device)
         i2i = torch.empty(B, H, g.frames, g.frames, dtype=torch.float32, device=mass.device)
-        with torch.cuda.device(mass.device):
+        with _lib.on(mass.device):
             _lib.check(_lib.load().sa_pattern_maps(mass.data_ptr(), _lib.i64(*mass.stride()[:3]), B, H, g.frames,
                                                    g.sample_num, i2t.data_ptr(), i2i.data_ptr(),
                                                    _lib.stream_of(mass)), "sa_pattern_maps")
@@ -269,7 +269,7 @@ def constrained_mod_factor(modify_factor, min_threshold=0.01, max_threshold=50.0
     x = modify_factor.to(torch.float32).contiguous()
     out = torch.empty_like(x)
     stats = torch.empty(B * H, 3, dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
+    with _lib.on(x.device):
         _lib.check(_lib.load().sa_constrained_mod_factor(x.data_ptr(), B * H, L, float(min_threshold),
                                                          float(max_threshold), stats.data_ptr(), out.data_ptr(),
                                                          _lib.stream_of(x)), "sa_constrained_mod_factor")
@@ -311,7 +311,7 @@ def _key_operands(x, idx, n_pad):
     full = full.to(x.device)
     B, H, L, D = x.shape
     out = torch.empty(B * H, n_pad, 64, dtype=x.dtype, device=x.device)
-    with torch.cuda.device(x.device):
+    with _lib.on(x.device):
         _lib.check(_lib.load().sa_gather_key_operands(x.data_ptr(), _lib.i64(*x.stride()[:3]), B, H, L, D,
                                                       full.data_ptr(), n_pad, out.data_ptr(), _lib.stream_of(x)),
                    "sa_gather_key_operands")
@@ -320,7 +320,7 @@ def _key_operands(x, idx, n_pad):
 
 def _probs(qs, ks, rows, keys, n_bias, bias, c_lo, c_hi, P, sm_scale: float = scale_factor):
     BH = qs.shape[0]
-    with torch.cuda.device(qs.device):
+    with _lib.on(qs.device):
         _lib.check(_lib.load().sa_sampled_probs(
             qs.data_ptr(), ks.data_ptr(), BH, rows, qs.shape[1], keys, ks.shape[1], sm_scale, n_bias, bias,
             c_lo, c_hi, P.data_ptr(), P.stride(0), P.stride(1), _lib.stream_of(qs)), "sa_sampled_probs")
@@ -339,7 +339,7 @@ def _sparsity_rows(q, k, g: PatternGeometry, idx_q):
     n = keys.numel()
     qs, ks = _compact(q, idx_q + g.text_length, _pad32(ns)), _key_operands(k, keys, _pad32(n))
     share = torch.empty(B * H, ns, dtype=torch.float32, device=q.device)
-    with torch.cuda.device(q.device):
+    with _lib.on(q.device):
         _lib.check(_lib.load().sa_topk_mass(qs.data_ptr(), ks.data_ptr(), B * H, ns, qs.shape[1], n, _pad32(n),
                                             scale_factor, int(n * SPARSE_KEEP), share.data_ptr(),
                                             _lib.stream_of(q)), "sa_topk_mass")
@@ -365,7 +365,7 @@ def _similarity_gram(q, k, g: PatternGeometry, index_k):
     lib = _lib.load()
     _lib.check(lib.sa_pattern_sim_gram_workspace(qs.shape[0], F, ns, ctypes.byref(n)), "sa_pattern_sim_gram_workspace")
     ws = torch.empty(n.value, dtype=torch.uint8, device=q.device)  # each position's products, until its sums are known
-    with torch.cuda.device(q.device):
+    with _lib.on(q.device):
         _lib.check(lib.sa_pattern_sim_gram_ws(
             qs.data_ptr(), ks.data_ptr(), qs.shape[0], F, ns, T, qs.shape[1], ks.shape[1], scale_factor,
             composition_bias(g), G.data_ptr(), ws.data_ptr(), ws.numel(), _lib.stream_of(q)), "sa_pattern_sim_gram_ws")
@@ -381,7 +381,7 @@ def _similarity_gram_via_probs(q, k, g: PatternGeometry, index_k):
     for h0, h1 in _chunks(BH, nv * _pad32(nv) * 4):
         P = torch.empty(h1 - h0, nv, _pad32(nv), dtype=torch.float32, device=q.device)
         _probs(qs[h0:h1], ks[h0:h1], nv, T + nv, T, composition_bias(g), T, T + nv, P)
-        with torch.cuda.device(q.device):
+        with _lib.on(q.device):
             _lib.check(_lib.load().sa_pattern_gram(P.data_ptr(), P.stride(0), P.stride(1), h1 - h0, F, ns,
                                                    G[h0:h1].data_ptr(), _lib.stream_of(q)), "sa_pattern_gram")
     return G
@@ -391,7 +391,7 @@ def _finish(share, G1, G2, BH, rows, F, ns, device):
     f32 = dict(dtype=torch.float32, device=device)
     sm, c1, c2 = torch.empty(BH, **f32), torch.empty(BH, **f32), torch.empty(BH, **f32)
     use = torch.empty(BH, dtype=torch.int32, device=device)
-    with torch.cuda.device(device):
+    with _lib.on(device):
         _lib.check(_lib.load().sa_pattern_judge_finish(
             _lib.ptr(share), _lib.ptr(G1), _lib.ptr(G2), BH, rows, F, ns, SPARSE_THR, SIM_THR, sm.data_ptr(),
             c1.data_ptr(), c2.data_ptr(), use.data_ptr(), torch.cuda.current_stream(device).cuda_stream),

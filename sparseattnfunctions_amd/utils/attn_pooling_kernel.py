@@ -82,7 +82,7 @@ class _attention_pooling(torch.autograd.Function):
         if ws is None:
             ws = torch.empty(ws_bytes.value, dtype=torch.uint8, device=q.device)
         fn = "sa_attn_pooling_fwd_f16" if fp16 else ("sa_attn_pooling_fwd_f32" if fp32 else "sa_attn_pooling_fwd")
-        with torch.cuda.device(q.device):
+        with _lib.on(q.device):
             _lib.check(getattr(lib, fn)(
                 q.data_ptr(), _lib.i64(*q.stride()[:3]), k.data_ptr(), _lib.i64(*k.stride()[:3]),
                 v.data_ptr(), _lib.i64(*v.stride()[:3]), o.data_ptr(), _lib.i64(*o.stride()[:3]),

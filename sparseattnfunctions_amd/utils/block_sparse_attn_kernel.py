@@ -24,6 +24,7 @@ Differences from the reference, by design:
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 from typing import Optional
 
@@ -52,6 +53,7 @@ N_XCD = 8  # MI355X: workgroups are dealt round-robin to 8 XCDs, each with its o
 N_CU = 256
 
 
+@functools.lru_cache(maxsize=1024)
 def split_parts(n_items: int, max_cnt: int, D: int) -> int:
     """Key-range parts per query block (`sa_attn_split_parts`) for a plain launch of n_items
     query blocks over lists of width max_cnt: 1 means one wave per block."""
@@ -112,7 +114,7 @@ def prepare_fp16_keys(k: torch.Tensor) -> Optional[FP16Keys]:
     B, H, Lk, D = k.shape
     ws = torch.empty(k16_workspace_bytes(B, H, Lk, D), dtype=torch.uint8, device=k.device)
     stream = torch.cuda.current_stream(k.device)
-    with torch.cuda.device(k.device):
+    with _lib.on(k.device):
         rc = _lib.load().sa_block_sparse_fwd_k16_prepare(k.data_ptr(), _lib.i64(*k.stride()[:3]), B, H, Lk, D,
                                                           ws.data_ptr(), ws.numel(), stream.cuda_stream)
     _lib.check(rc, "sa_block_sparse_fwd_k16_prepare")
@@ -128,16 +130,22 @@ def prepare_fp16_keys(k: torch.Tensor) -> Optional[FP16Keys]:
 F32_TERMS_BLOCKS = 8
 
 
+@functools.lru_cache(maxsize=1024)
+def f32_terms_workspace_bytes(B: int, H: int, Lk: int, D: int) -> int:
+    n = ctypes.c_int64(0)
+    _lib.check(_lib.load().sa_block_sparse_fwd_f32_terms_workspace(B, H, Lk, D, ctypes.byref(n)),
+               "sa_block_sparse_fwd_f32_terms_workspace")
+    return n.value
+
+
 def f32_terms_workspace(B: int, H: int, Lk: int, D: int, device):
     """Workspace of `sa_block_sparse_fwd_f32_terms`, or None where the fp32 kernel runs without
     one: keys of one head past its 32-bit offsets, or no memory for it (12 D bytes per key)."""
-    n = ctypes.c_int64(0)
-    _lib.check(_lib.load().sa_block_sparse_fwd_f32_terms_workspace(int(B), int(H), int(Lk), int(D), ctypes.byref(n)),
-               "sa_block_sparse_fwd_f32_terms_workspace")
-    if n.value // (B * H) >= 1 << 31:
+    n = f32_terms_workspace_bytes(B, H, Lk, D)
+    if n // (B * H) >= 1 << 31:
         return None
     try:
-        return torch.empty(n.value, dtype=torch.uint8, device=device)
+        return torch.empty(n, dtype=torch.uint8, device=device)
     except torch.cuda.OutOfMemoryError:
         return None
 
@@ -147,7 +155,7 @@ _ORDER_CACHE = {}
 
 def work_order(B: int, H: int, nqb: int, n_text_blocks: int, device) -> torch.Tensor:
     """Device copy of the attention dispatch order (`sa_attn_work_order`), cached per shape."""
-    key = (B, H, nqb, n_text_blocks, str(device))
+    key = (B, H, nqb, n_text_blocks, device)
     order = _ORDER_CACHE.get(key)
     if order is None:
         lib = _lib.load()
@@ -255,7 +263,7 @@ def block_sparse_attention(q, k, v, kv: KVList, sm_scale: float, key_bias=None, 
         # from the caching allocator on this stream (the kernels use it in stream order).
         ws = torch.empty(split_workspace_bytes(B * H * nqb, D, parts), dtype=torch.uint8, device=q.device)
         fn = "sa_block_sparse_fwd_split_f16" if fp16 else "sa_block_sparse_fwd_split"
-        with torch.cuda.device(q.device):
+        with _lib.on(q.device):
             rc = getattr(lib, fn)(
                 q.data_ptr(), _lib.i64(*q.stride()[:3]), k.data_ptr(), _lib.i64(*k.stride()[:3]),
                 v.data_ptr(), _lib.i64(*v.stride()[:3]), out.data_ptr(), _lib.i64(*out.stride()[:3]),
@@ -268,7 +276,7 @@ def block_sparse_attention(q, k, v, kv: KVList, sm_scale: float, key_bias=None, 
     if q_rows is not None or o_rows is not None or tile_masks is not None:
         kv_slot, masks = (tile_masks[0], tile_masks[1]) if tile_masks is not None else (None, None)
         fn = "sa_block_sparse_fwd_mapped_f16" if fp16 else "sa_block_sparse_fwd_mapped"
-        with torch.cuda.device(q.device):
+        with _lib.on(q.device):
             rc = getattr(lib, fn)(
                 q.data_ptr(), _lib.i64(*q.stride()[:3]), k.data_ptr(), _lib.i64(*k.stride()[:3]),
                 v.data_ptr(), _lib.i64(*v.stride()[:3]), out.data_ptr(), _lib.i64(*out.stride()[:3]),
@@ -279,7 +287,7 @@ def block_sparse_attention(q, k, v, kv: KVList, sm_scale: float, key_bias=None, 
         _lib.check(rc, fn)
         return out
     if Dout == 32 and D == 64:
-        with torch.cuda.device(q.device):
+        with _lib.on(q.device):
             rc = lib.sa_block_sparse_fwd_v32(
                 q.data_ptr(), _lib.i64(*q.stride()[:3]), k.data_ptr(), _lib.i64(*k.stride()[:3]),
                 v.data_ptr(), _lib.i64(*v.stride()[:3]), out.data_ptr(), _lib.i64(*out.stride()[:3]),
@@ -308,7 +316,7 @@ def block_sparse_attention(q, k, v, kv: KVList, sm_scale: float, key_bias=None, 
             ws = torch.empty(k16_workspace_bytes(B, H, Lk, D, with_bias=key_bias is not None), dtype=torch.uint8,
                              device=q.device)
             prepared = 0
-        with torch.cuda.device(q.device):
+        with _lib.on(q.device):
             rc = lib.sa_block_sparse_fwd_k16(
                 q.data_ptr(), _lib.i64(*q.stride()[:3]), k.data_ptr(), _lib.i64(*k.stride()[:3]),
                 v.data_ptr(), _lib.i64(*v.stride()[:3]), out.data_ptr(), _lib.i64(*out.stride()[:3]),
@@ -320,7 +328,7 @@ def block_sparse_attention(q, k, v, kv: KVList, sm_scale: float, key_bias=None, 
     if fp32 and nqb >= F32_TERMS_BLOCKS:
         ws = f32_terms_workspace(B, H, Lk, D, q.device)
         if ws is not None:
-            with torch.cuda.device(q.device):
+            with _lib.on(q.device):
                 rc = lib.sa_block_sparse_fwd_f32_terms(
                     q.data_ptr(), _lib.i64(*q.stride()[:3]), k.data_ptr(), _lib.i64(*k.stride()[:3]),
                     v.data_ptr(), _lib.i64(*v.stride()[:3]), out.data_ptr(), _lib.i64(*out.stride()[:3]),
@@ -329,7 +337,7 @@ def block_sparse_attention(q, k, v, kv: KVList, sm_scale: float, key_bias=None, 
             _lib.check(rc, "sa_block_sparse_fwd_f32_terms")
             return out
     fn = "sa_block_sparse_fwd_f16" if fp16 else ("sa_block_sparse_fwd_f32" if fp32 else "sa_block_sparse_fwd")
-    with torch.cuda.device(q.device):
+    with _lib.on(q.device):
         rc = getattr(lib, fn)(
             q.data_ptr(), _lib.i64(*q.stride()[:3]),
             k.data_ptr(), _lib.i64(*k.stride()[:3]),
@@ -374,7 +382,7 @@ def cell_kv_list(mask: torch.Tensor, B: int, H: int, Lq: int, Lk: int, block_m: 
     nqb, nkb = math.ceil(Lq / BLOCK), math.ceil(Lk / BLOCK)
     kv = KVList.empty(B, H, nqb, nkb, mask.device)
     slot = None if (block_m >= BLOCK and block_n >= BLOCK) else torch.empty_like(kv.idx)
-    with torch.cuda.device(mask.device):
+    with _lib.on(mask.device):
         _lib.check(_lib.load().sa_mask_cells_to_kv_list(
             m.data_ptr(), _lib.i64(*m.stride()), B, H, Lq, Lk, block_m, block_n, kv.idx.data_ptr(), _lib.ptr(slot),
             kv.max_cnt, kv.cnt.data_ptr(), _lib.stream_of(m)), "sa_mask_cells_to_kv_list")

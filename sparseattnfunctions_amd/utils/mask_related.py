@@ -222,7 +222,7 @@ def inner_frame_cell_sums(q, k, original_length=FRAME_LENGTH, stride=64):
     mass = block_sparse_attention(q[:, :, :q_len], k[:, :, :k_len], ind, dense_kv_list(B, H, Qr, Kr, q.device),
                                   1 / 8, v_cols=32 if Kr <= 32 and q.dtype == torch.bfloat16 else None)
     out = torch.empty(B, H, Qr, Kr, dtype=torch.float32, device=q.device)
-    with torch.cuda.device(q.device):
+    with _lib.on(q.device):
         rc = _lib.load().sa_row_group_sums(mass.data_ptr(), _lib.i64(*mass.stride()[:3]), B, H, q_len, stride, 0, Kr,
                                            out.data_ptr(), _lib.stream_of(mass))
     _lib.check(rc, "sa_row_group_sums")
@@ -263,7 +263,7 @@ def get_block_mask(inner_frame_mask, frame_mask, padding=4):
     fm = (frame_mask != 0).to(torch.uint8).contiguous()
     im = (inner_frame_mask != 0).to(torch.uint8).contiguous()
     out = torch.empty(B, H, F * Ri + padding, F * Ci + padding, dtype=torch.float32, device=fm.device)
-    with torch.cuda.device(fm.device):
+    with _lib.on(fm.device):
         rc = _lib.load().sa_kron_block_mask(fm.data_ptr(), im.data_ptr(), B * H, F, Ri, Ci, int(padding),
                                             out.data_ptr(), _lib.stream_of(fm))
     _lib.check(rc, "sa_kron_block_mask")
