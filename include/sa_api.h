@@ -338,6 +338,15 @@ int sa_attn_work_order(int B, int H, int nqb, int n_text_blocks, int n_xcd, int3
                        int64_t* n_slots);
 
 /*
+ * (host) The same order with every text row's item in a dispatch group of its own, whose four
+ * waves share it: for 16-bit launches at head dim 64 in which one wave over a text row's list
+ * would outlast the other rows. The group's four slots hold the item + 2^30; launches at head
+ * dim 128 or in fp32 take sa_attn_work_order.
+ */
+int sa_attn_work_order_long(int B, int H, int nqb, int n_text_blocks, int n_xcd, int32_t* order,
+                            int64_t* n_slots);
+
+/*
  * Host. Suggested key-range parts per query block for sa_block_sparse_fwd_split: a launch of
  * n_items = B*H*ceil(Lq/64) query blocks with lists of width max_cnt, head dim D, on a device
  * of n_cus compute units (MI355X: 256). *parts = 1: no split. Parts are chosen to fill the

@@ -86,6 +86,8 @@ class StaLayout:
                                           kv_slot.data_ptr(), masks.data_ptr(), ctypes.byref(n_slots)),
                    "sa_sta_block_masks")
         self.n_partial = n_slots.value
+        video_cnt = kv_cnt[self.text_blocks:].float()
+        self.row_blocks = video_cnt.mean().item() if video_cnt.numel() else None
         self.perm = perm.to(device)
         self.inv = torch.empty_like(perm).scatter_(0, perm.long(), torch.arange(self.L, dtype=torch.int32)).to(device)
         self.kv_idx, self.kv_cnt, self.kv_slot, self.masks = (t.to(device) for t in (kv_idx, kv_cnt, kv_slot, masks))
@@ -138,7 +140,7 @@ class SildingTileAttention:
         if L != lay.L or k.shape != q.shape or v.shape != q.shape:
             raise ValueError(f"expected q, k, v of {lay.L} tokens for this configuration, got {tuple(q.shape)}")
         scale = sm_scale if sm_scale is not None else 1.0 / math.sqrt(D)
-        kv = KVList(lay.kv_idx, lay.kv_cnt, 1, 1, lay.nb, lay.nb)
+        kv = KVList(lay.kv_idx, lay.kv_cnt, 1, 1, lay.nb, lay.nb, row_blocks=lay.row_blocks)
         return block_sparse_attention(q, k, v, kv, scale, n_text_blocks=lay.text_blocks,
                                       tile_masks=(lay.kv_slot, lay.masks, True))
 
@@ -151,7 +153,7 @@ class SildingTileAttention:
         if L != lay.L or k.shape != q.shape or v.shape != q.shape:
             raise ValueError(f"expected q, k, v of {lay.L} tokens for this configuration, got {tuple(q.shape)}")
         kt, vt = _gather(k, lay.perm), _gather(v, lay.perm)
-        kv = KVList(lay.kv_idx, lay.kv_cnt, 1, 1, lay.nb, lay.nb)
+        kv = KVList(lay.kv_idx, lay.kv_cnt, 1, 1, lay.nb, lay.nb, row_blocks=lay.row_blocks)
         return block_sparse_attention(q, kt, vt, kv, 1.0 / math.sqrt(D), n_text_blocks=lay.text_blocks,
                                       q_rows=lay.perm, o_rows=lay.perm,
                                       tile_masks=(lay.kv_slot, lay.masks, True))

@@ -9,6 +9,7 @@ program re-reading the whole mask row.
 from __future__ import annotations
 
 from dataclasses import dataclass
+from typing import Optional
 
 import torch
 
@@ -24,6 +25,7 @@ class KVList:
     nqb: int
     nkb: int
     dense: bool = False  # every row lists every key block (set by the dense-list builders)
+    row_blocks: Optional[float] = None  # about how many blocks a row without text lists, where the host knows
 
     @property
     def rows(self) -> int:

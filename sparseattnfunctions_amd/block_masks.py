@@ -81,6 +81,8 @@ def topk_kv_list(q_pooled, k_pooled, B: int, H: int, topk: int, n_text_blocks: i
         nkb = k_pooled.shape[1]
         dev = q_pooled.device
     kv = KVList.empty(B, H, nqb, nkb, dev)
+    if local_bitmap is None:
+        kv.row_blocks = min(nkb, int(topk) + int(n_text_blocks))
     mask = torch.empty(B, H, nqb, nkb, dtype=torch.uint8, device=dev) if return_mask else None
     scores = torch.empty(B, H, nqb, nkb, dtype=torch.float32, device=dev) if return_scores else None
     loc = None

@@ -114,9 +114,15 @@ class CombinedAttn:
         if L != self.geometry.L:
             raise ValueError(f"sequence length {L} does not match the geometry (L={self.geometry.L})")
         nb = math.ceil(L / 64)
-        local = local_window_bitmap(self.geometry, self.window, q.device)
-        return meanpool_topk_kv_list(q, k, topk_count(self.global_ratio, nb), self.n_text_blocks(),
-                                     local_bitmap=local, with_fp16_keys=with_fp16_keys)
+        g = self.geometry
+        local = local_window_bitmap(g, self.window, q.device)
+        topk = topk_count(self.global_ratio, nb)
+        out = meanpool_topk_kv_list(q, k, topk, self.n_text_blocks(), local_bitmap=local,
+                                    with_fp16_keys=with_fp16_keys)
+        kv = out[0] if with_fp16_keys else out
+        window = math.prod(min(2 * w + 1, n) for w, n in zip(self.window, (g.T, g.Hp, g.Wp)))
+        kv.row_blocks = min(nb, topk + self.n_text_blocks() + window / 64)
+        return out
 
     @staticmethod
     def rearranger(q, k, v):

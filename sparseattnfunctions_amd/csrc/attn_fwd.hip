@@ -127,6 +127,9 @@ struct FwdArgs {
   const uint32_t* k16_norm2;
 };
 
+// Added to the item in the four slots of a group that share it (sa_attn_work_order_long).
+constexpr int kSharedItem = 1 << 30;
+
 // Item of a dispatch slot without a work order: as sa_attn_work_order places them, each XCD (group
 // w of four slots runs on XCD w % 8) a contiguous range of items; -1 = idle.
 __device__ inline int xcd_item(const FwdArgs& a, int slot) {
@@ -298,7 +301,10 @@ constexpr int kWaitLgkm0 = 0xC07F;
 // copied as usual and only their first 32 columns are read; out has 32 columns).
 // kShare (head dim 64): the items of dispatch groups from shared_from on are each
 // shared by the four waves of a workgroup, wave p taking list positions [cnt p / 4, cnt (p + 1) / 4)
-// and all merging their partials through the LDS of their tiles; see shared_groups for when.
+// and all merging their partials through the LDS of their tiles; see shared_from for when. So are
+// the groups of a work order that hold one item four times (sa_attn_work_order_long): a text row
+// over nkb blocks is a serial chain of 1.2 us per block, the whole launch where the other rows are
+// short or few ([1, 6, 17776, 64] with a fifth of the blocks 348 -> 171 us, [1, 24, 2944, 64] 81 -> 58).
 template <bool kBias, bool kMask, int kPool, typename T = __bf16, int kD = 64, int kDV = kD, bool kK16 = false,
           bool kShare = false>
 __global__ __launch_bounds__(256, kD == 64 ? 2 : 1) void bsa_fwd_kernel(FwdArgs a) {
@@ -338,7 +344,7 @@ __global__ __launch_bounds__(256, kD == 64 ? 2 : 1) void bsa_fwd_kernel(FwdArgs 
   const int col = lane & 31;  // query column within a 32-row group (MFMA n index)
   const int hh = lane >> 5;   // lane half (MFMA k group)
   __shared__ float ml_lds[kShare ? kWaves : 1][2][kBlock];  // row maxima and sums of the partials
-  const bool shared = kShare && (int)blockIdx.x >= a.shared_from;
+  bool shared = kShare && (int)blockIdx.x >= a.shared_from;
   int slot = blockIdx.x * kWaves + wave;
   if (shared) {  // a shared group is four workgroups, on the group's XCD
     const int y = blockIdx.x - a.shared_from;
@@ -357,6 +363,11 @@ __global__ __launch_bounds__(256, kD == 64 ? 2 : 1) void bsa_fwd_kernel(FwdArgs 
     item = bh_s * a.nqb + (rem - part * a.nqb);
   } else {
     item = __builtin_amdgcn_readfirstlane(a.order ? a.order[slot] : xcd_item(a, slot));
+    if (kShare && a.order && item >= kSharedItem) {  // the group's four slots hold one item
+      if (shared && (slot & (kWaves - 1)) != 0) return;  // (the same for the whole workgroup)
+      shared = true;
+      item -= kSharedItem;
+    }
   }
   // Idle slot. (The only barriers below are a shared item's, whose waves all take the same branch.)
   if (item < 0 || item >= a.n_items) return;
@@ -1466,19 +1477,28 @@ __global__ __launch_bounds__(128, 2) void bsa_fwd_pair_kernel(FwdArgs a) {
 }  // namespace
 
 
-extern "C" int sa_attn_work_order(int B, int H, int nqb, int n_text_blocks, int n_xcd, int32_t* order,
-                                  int64_t* n_slots) {
-  SA_REQUIRE(n_slots, "sa_attn_work_order: null n_slots");
+namespace {
+
+// The work order; with share_text a text row's item takes a whole group of four slots, each
+// holding item + kSharedItem.
+int build_work_order(const char* fn, int B, int H, int nqb, int n_text_blocks, int n_xcd, bool share_text,
+                     int32_t* order, int64_t* n_slots) {
+  SA_REQUIRE(n_slots, "%s: null n_slots", fn);
   SA_REQUIRE(B > 0 && H > 0 && nqb > 0 && n_text_blocks >= 0 && n_xcd > 0,
-             "sa_attn_work_order: bad arguments B=%d H=%d nqb=%d n_text=%d n_xcd=%d", B, H, nqb, n_text_blocks, n_xcd);
+             "%s: bad arguments B=%d H=%d nqb=%d n_text=%d n_xcd=%d", fn, B, H, nqb, n_text_blocks, n_xcd);
   const int64_t n_items = (int64_t)B * H * nqb;
-  SA_REQUIRE(n_items < (1LL << 30), "sa_attn_work_order: too many items");
+  SA_REQUIRE(n_items < (1LL << 30), "%s: too many items", fn);
   // Contiguous bh-major chunks of (nearly) equal size, one per XCD.
   std::vector<int64_t> lo(n_xcd + 1);
   for (int x = 0; x <= n_xcd; ++x) lo[x] = n_items * x / n_xcd;
-  int64_t max_chunk = 0;
-  for (int x = 0; x < n_xcd; ++x) max_chunk = std::max<int64_t>(max_chunk, lo[x + 1] - lo[x]);
-  const int64_t wg_per_xcd = (max_chunk + kWaves - 1) / kWaves;
+  const int64_t nt = share_text ? std::min(n_text_blocks, nqb) : 0;
+  // Items before `it` that take a group each.
+  auto texts = [&](int64_t it) { return it / nqb * nt + std::min<int64_t>(it % nqb, nt); };
+  int64_t wg_per_xcd = 0;
+  for (int x = 0; x < n_xcd; ++x) {
+    const int64_t n = lo[x + 1] - lo[x], shared = texts(lo[x + 1]) - texts(lo[x]);
+    wg_per_xcd = std::max(wg_per_xcd, shared + (n - shared + kWaves - 1) / kWaves);
+  }
   const int64_t total = wg_per_xcd * n_xcd * kWaves;
   *n_slots = total;
   if (!order) return sa::ok();
@@ -1490,7 +1510,11 @@ extern "C" int sa_attn_work_order(int B, int H, int nqb, int n_text_blocks, int 
     for (int pass = 0; pass < 2; ++pass)
       for (int64_t it = lo[x]; it < lo[x + 1]; ++it) {
         const bool text = (it % nqb) < n_text_blocks;
-        if (text == (pass == 0)) chunk.push_back((int32_t)it);
+        if (text != (pass == 0)) continue;
+        if (text && share_text)
+          chunk.insert(chunk.end(), kWaves, (int32_t)it + kSharedItem);
+        else
+          chunk.push_back((int32_t)it);
       }
     // Workgroup w of this XCD is dispatch index w*n_xcd + x (round-robin dispatch).
     for (size_t p = 0; p < chunk.size(); ++p) {
@@ -1499,6 +1523,18 @@ extern "C" int sa_attn_work_order(int B, int H, int nqb, int n_text_blocks, int 
     }
   }
   return sa::ok();
+}
+
+}  // namespace
+
+extern "C" int sa_attn_work_order(int B, int H, int nqb, int n_text_blocks, int n_xcd, int32_t* order,
+                                  int64_t* n_slots) {
+  return build_work_order("sa_attn_work_order", B, H, nqb, n_text_blocks, n_xcd, false, order, n_slots);
+}
+
+extern "C" int sa_attn_work_order_long(int B, int H, int nqb, int n_text_blocks, int n_xcd, int32_t* order,
+                                       int64_t* n_slots) {
+  return build_work_order("sa_attn_work_order_long", B, H, nqb, n_text_blocks, n_xcd, true, order, n_slots);
 }
 
 namespace {
@@ -1596,8 +1632,12 @@ size_t split_workspace_bytes(int64_t n_items, int D, int parts) {
 constexpr int64_t kShareRound = 1024;
 constexpr int64_t kShareMax = 704;
 
-int shared_from(int64_t n_slots) {
-  const int64_t left = n_slots % kShareRound;
+// Slots that n_items take with one item each (in xcd_item's and sa_attn_work_order's layout).
+int64_t plain_slots(int64_t n_items) { return ((n_items + 7) / 8 + kWaves - 1) / kWaves * 8 * kWaves; }
+
+// extra: slots past plain_slots, three for each item that already has a group of its own.
+int shared_from(int64_t n_slots, int64_t extra) {
+  const int64_t left = (n_slots - extra / 24 * 32) % kShareRound;
   return (int)((left > 0 && left <= kShareMax ? n_slots - left : n_slots) / kWaves);
 }
 
@@ -1616,8 +1656,9 @@ void launch_variant(const FwdArgs& a, dim3 g, dim3 blk, hipStream_t s, bool mask
                     bool v32 = false) {
   if constexpr (kD == 64) {
     const bool may_share = a.n_parts == 1 && !(mask && pool_cols);
-    const int from = may_share ? shared_from(a.n_slots) : a.n_slots / kWaves;
-    if (from < a.n_slots / kWaves) {
+    const int64_t extra = a.order ? std::max<int64_t>(a.n_slots - plain_slots(a.n_items), 0) : 0;
+    const int from = may_share ? shared_from(a.n_slots, extra) : a.n_slots / kWaves;
+    if (from < a.n_slots / kWaves || (may_share && extra > 0)) {
       if (pool_cols == 32) return launch_shared<false, false, T, 64, false, 32>(a, from, s);
       if (pool_cols == 64) return launch_shared<false, false, T, 64, false, 64>(a, from, s);
       if constexpr (std::is_same<T, __bf16>::value) {
@@ -1700,7 +1741,7 @@ int launch_fwd(const uint16_t* q, const int64_t q_strides[3], const uint16_t* k,
   if (work_order) {
     SA_REQUIRE(n_slots > 0 && n_slots % kWaves == 0, "%s: n_slots must be a positive multiple of 4", fn);
   } else {  // xcd_item: each of the eight XCDs' ranges in whole groups
-    n_slots = ((n_items + 7) / 8 + kWaves - 1) / kWaves * 8 * kWaves;
+    n_slots = plain_slots(n_items);
   }
   // 16-byte vector accesses: base pointers 16-byte aligned, row strides multiples of 8 elements.
   const void* ptrs[4] = {q, k, v, out};

@@ -153,17 +153,42 @@ def f32_terms_workspace(B: int, H: int, Lk: int, D: int, device):
 _ORDER_CACHE = {}
 
 
-def work_order(B: int, H: int, nqb: int, n_text_blocks: int, device) -> torch.Tensor:
-    """Device copy of the attention dispatch order (`sa_attn_work_order`), cached per shape."""
-    key = (B, H, nqb, n_text_blocks, device)
+# Text rows list every key block, and one wave over nkb blocks (1.2 us each) can outlast everything
+# else in a launch of few heads or short lists: there each text row is shared by the four waves of a
+# workgroup. The lines: the other rows' blocks per wave slot against nkb (first), and a row's own
+# blocks, which take up to twice as long beside the added workgroups, against nkb (second). Without /
+# with, us, at a first ratio of 0.17: top-k [1, 6, 17776, 64] 348 / 171; 0.24: sliding tiles [1, 20,
+# 10054, 64] 262 / 177; 0.34: top-k on it 245 / 186. Past the first line long rows beside short ones keep
+# the matrix core busy while those start and end: top-k 170 / 172 at 0.60 and 522 / 529 at 1.1, sliding
+# tiles [2, 30, 3106, 64] 105 / 115 at 0.44, with wide windows 192 / 251 at 0.95. Past the second:
+# sliding tiles [1, 26, 2459, 64] 73 / 79 at half of nkb. Launches that share every row
+# (`shared_from` in csrc/attn_fwd.hip) take the plain order.
+WAVE_SLOTS = 2048  # of these kernels at head dim 64: two per SIMD
+SHARE_TEXT_BELOW = 0.35
+SHARE_TEXT_ROW_BELOW = 0.4
+ALL_SHARED_ITEMS = 704
+
+
+def shares_text_rows(n_items: int, nkb: int, n_text_blocks: int, row_blocks: Optional[float], D: int) -> bool:
+    """Whether a launch's text rows take a workgroup each (`sa_attn_work_order_long`)."""
+    return (n_text_blocks > 0 and D == 64 and row_blocks is not None and n_items > ALL_SHARED_ITEMS
+            and n_items * row_blocks <= SHARE_TEXT_BELOW * WAVE_SLOTS * nkb
+            and row_blocks <= SHARE_TEXT_ROW_BELOW * nkb)
+
+
+def work_order(B: int, H: int, nqb: int, n_text_blocks: int, device, share_text: bool = False) -> torch.Tensor:
+    """Device copy of the attention dispatch order (`sa_attn_work_order`; with share_text
+    `sa_attn_work_order_long`), cached per shape."""
+    key = (B, H, nqb, n_text_blocks, device, share_text)
     order = _ORDER_CACHE.get(key)
     if order is None:
         lib = _lib.load()
         n = ctypes.c_int64(0)
-        _lib.check(lib.sa_attn_work_order(B, H, nqb, n_text_blocks, N_XCD, None, ctypes.byref(n)), "sa_attn_work_order")
+        name = "sa_attn_work_order_long" if share_text else "sa_attn_work_order"
+        build = getattr(lib, name)
+        _lib.check(build(B, H, nqb, n_text_blocks, N_XCD, None, ctypes.byref(n)), name)
         host = torch.empty(n.value, dtype=torch.int32)
-        _lib.check(lib.sa_attn_work_order(B, H, nqb, n_text_blocks, N_XCD, host.data_ptr(), ctypes.byref(n)),
-                   "sa_attn_work_order")
+        _lib.check(build(B, H, nqb, n_text_blocks, N_XCD, host.data_ptr(), ctypes.byref(n)), name)
         order = host.to(device)
         _ORDER_CACHE[key] = order
     return order
@@ -272,7 +297,8 @@ def block_sparse_attention(q, k, v, kv: KVList, sm_scale: float, key_bias=None, 
                 _lib.stream_of(q))
         _lib.check(rc, fn)
         return out
-    order = work_order(B, H, nqb, n_text_blocks, q.device)
+    share_text = not fp32 and shares_text_rows(B * H * nqb, kv.nkb, n_text_blocks, kv.row_blocks, D)
+    order = work_order(B, H, nqb, n_text_blocks, q.device, share_text)
     if q_rows is not None or o_rows is not None or tile_masks is not None:
         kv_slot, masks = (tile_masks[0], tile_masks[1]) if tile_masks is not None else (None, None)
         fn = "sa_block_sparse_fwd_mapped_f16" if fp16 else "sa_block_sparse_fwd_mapped"

@@ -94,6 +94,33 @@ def test_work_order_is_a_permutation(lib):
                 assert text.nonzero().max() < (~text).nonzero().min()
 
 
+def test_long_work_order_gives_each_text_row_a_group(lib):
+    import torch
+    for B, H, nqb, nt in [(2, 30, 278, 4), (1, 1, 1, 0), (1, 3, 5, 2), (1, 3, 5, 9), (2, 5, 41, 3)]:
+        n, plain = ctypes.c_int64(0), ctypes.c_int64(0)
+        assert lib.sa_attn_work_order(B, H, nqb, nt, 8, None, ctypes.byref(plain)) == 0
+        assert lib.sa_attn_work_order_long(B, H, nqb, nt, 8, None, ctypes.byref(n)) == 0
+        assert n.value % 32 == 0 and n.value >= plain.value
+        order = torch.full((n.value + 4,), 7, dtype=torch.int32)
+        assert lib.sa_attn_work_order_long(B, H, nqb, nt, 8, order.data_ptr(), ctypes.byref(n)) == 0
+        assert (order[n.value:] == 7).all()
+        groups = order[:n.value].view(-1, 4)
+        own = (groups >= 1 << 30).any(1)
+        shared = groups[own] - (1 << 30)
+        assert (shared == shared[:, :1]).all()
+        rest = groups[~own].flatten()
+        items = torch.cat([shared[:, 0], rest[rest >= 0]])
+        assert torch.equal(items.sort().values, torch.arange(B * H * nqb, dtype=torch.int32))
+        assert ((shared[:, 0] % nqb) < nt).all() and ((rest[rest >= 0] % nqb) >= nt).all()
+        for x in range(8):  # each XCD's text rows come first, on the heads of its plain order
+            mine = own[torch.arange(own.numel()) % 8 == x]
+            assert not (mine[1:] & ~mine[:-1]).any()
+        if not own.any():
+            assert n.value == plain.value
+    assert lib.sa_attn_work_order_long(0, 1, 1, 0, 8, None, ctypes.byref(n)) == _lib.SA_ERR_INVALID
+    assert lib.sa_attn_work_order_long(1, 1, 1, 0, 8, None, None) == _lib.SA_ERR_INVALID
+
+
 def test_split_parts_query(lib):
     parts = ctypes.c_int(-1)
     assert lib.sa_attn_split_parts(0, 128, 64, 256, ctypes.byref(parts)) == _lib.SA_ERR_INVALID
