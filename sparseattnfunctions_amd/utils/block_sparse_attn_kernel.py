@@ -158,21 +158,25 @@ _ORDER_CACHE = {}
 # workgroup. The lines: the other rows' blocks per wave slot against nkb (first), and a row's own
 # blocks, which take up to twice as long beside the added workgroups, against nkb (second). Without /
 # with, us, at a first ratio of 0.17: top-k [1, 6, 17776, 64] 348 / 171; 0.24: sliding tiles [1, 20,
-# 10054, 64] 262 / 177; 0.34: top-k on it 245 / 186. Past the first line long rows beside short ones keep
-# the matrix core busy while those start and end: top-k 170 / 172 at 0.60 and 522 / 529 at 1.1, sliding
-# tiles [2, 30, 3106, 64] 105 / 115 at 0.44, with wide windows 192 / 251 at 0.95. Past the second:
-# sliding tiles [1, 26, 2459, 64] 73 / 79 at half of nkb. Launches that share every row
-# (`shared_from` in csrc/attn_fwd.hip) take the plain order.
+# 10054, 64] 262 / 177; 0.34: top-k on it 245 / 186; 0.36: combined [1, 30, 4546, 64] 116 / 94;
+# 0.42 and 0.45: top-k [2, 7, 11581, 64] 284 / 237, [2, 21, 3461, 64] 109 / 100. Past the first line, lower
+# with tile masks, long rows beside short ones keep the matrix core busy while those start and end:
+# top-k [2, 25, 3696, 64] 116 / 119 at 0.51, 170 / 172 at 0.60 and 522 / 529 at 1.1, sliding tiles
+# [2, 30, 3106, 64] 105 / 115 at 0.44, with wide windows 192 / 251 at 0.95. Past the second: sliding
+# tiles [1, 26, 2459, 64] 73 / 79 at half of nkb. Launches that share every row (`shared_from` in
+# csrc/attn_fwd.hip) take the plain order.
 WAVE_SLOTS = 2048  # of these kernels at head dim 64: two per SIMD
-SHARE_TEXT_BELOW = 0.35
+SHARE_TEXT_BELOW = 0.5
+SHARE_TEXT_BELOW_MASKED = 0.35
 SHARE_TEXT_ROW_BELOW = 0.4
 ALL_SHARED_ITEMS = 704
 
 
-def shares_text_rows(n_items: int, nkb: int, n_text_blocks: int, row_blocks: Optional[float], D: int) -> bool:
+def shares_text_rows(n_items: int, nkb: int, n_text_blocks: int, row_blocks: Optional[float], D: int,
+                     masked: bool = False) -> bool:
     """Whether a launch's text rows take a workgroup each (`sa_attn_work_order_long`)."""
     return (n_text_blocks > 0 and D == 64 and row_blocks is not None and n_items > ALL_SHARED_ITEMS
-            and n_items * row_blocks <= SHARE_TEXT_BELOW * WAVE_SLOTS * nkb
+            and n_items * row_blocks <= (SHARE_TEXT_BELOW_MASKED if masked else SHARE_TEXT_BELOW) * WAVE_SLOTS * nkb
             and row_blocks <= SHARE_TEXT_ROW_BELOW * nkb)
 
 
@@ -297,7 +301,8 @@ def block_sparse_attention(q, k, v, kv: KVList, sm_scale: float, key_bias=None, 
                 _lib.stream_of(q))
         _lib.check(rc, fn)
         return out
-    share_text = not fp32 and shares_text_rows(B * H * nqb, kv.nkb, n_text_blocks, kv.row_blocks, D)
+    share_text = not fp32 and shares_text_rows(B * H * nqb, kv.nkb, n_text_blocks, kv.row_blocks, D,
+                                               tile_masks is not None)
     order = work_order(B, H, nqb, n_text_blocks, q.device, share_text)
     if q_rows is not None or o_rows is not None or tile_masks is not None:
         kv_slot, masks = (tile_masks[0], tile_masks[1]) if tile_masks is not None else (None, None)
