@@ -340,8 +340,9 @@ int sa_attn_work_order(int B, int H, int nqb, int n_text_blocks, int n_xcd, int3
 /*
  * (host) The same order with every text row's item in a dispatch group of its own, whose four
  * waves share it: for 16-bit launches at head dim 64 in which one wave over a text row's list
- * would outlast the other rows. The group's four slots hold the item + 2^30; launches at head
- * dim 128 or in fp32 take sa_attn_work_order.
+ * would outlast the other rows. The group's four slots hold the item + 2^30, and with any such
+ * item the order has more slots than sa_attn_work_order's for 8 XCDs, by which a launch knows it.
+ * Launches at head dim 128 or in fp32 run such an item in the group's first slot.
  */
 int sa_attn_work_order_long(int B, int H, int nqb, int n_text_blocks, int n_xcd, int32_t* order,
                             int64_t* n_slots);

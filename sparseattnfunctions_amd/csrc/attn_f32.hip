@@ -279,7 +279,7 @@ __global__ __launch_bounds__(64 * kWavesF32, kD == 64 ? 2 : 1) void bsa_fwd_f32_
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int slot = blockIdx.x * kWavesF32 + wave;
   if (slot >= a.n_slots) return;
-  const int item = __builtin_amdgcn_readfirstlane(a.order ? a.order[slot] : slot);
+  const int item = __builtin_amdgcn_readfirstlane(a.order ? order_item(a.order, slot) : slot);
   if (item < 0 || item >= a.n_items) return;
   const int bh = item / a.nqb;
   const int qb = item - bh * a.nqb;
@@ -495,7 +495,7 @@ __global__ __launch_bounds__(256, 2) void bsa_fwd_f32_terms_kernel(F32Args a) {
   const int unit = 4 * kHalvesQ * w8 + ((x >> 3) % kWgs) * kUnitsWg + (kKW == 1 ? wave : 0);
   const int slot = unit / kHalvesQ;
   if (slot >= a.n_slots) return;  // kKW = 4: the same for every wave of the workgroup
-  const int item = __builtin_amdgcn_readfirstlane(a.order ? a.order[slot] : slot);
+  const int item = __builtin_amdgcn_readfirstlane(a.order ? order_item(a.order, slot) : slot);
   if (item < 0 || item >= a.n_items) return;
   const int row0 = (unit % kHalvesQ) * kRows;
   const int bh = item / a.nqb;

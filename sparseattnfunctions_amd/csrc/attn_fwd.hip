@@ -127,9 +127,6 @@ struct FwdArgs {
   const uint32_t* k16_norm2;
 };
 
-// Added to the item in the four slots of a group that share it (sa_attn_work_order_long).
-constexpr int kSharedItem = 1 << 30;
-
 // Item of a dispatch slot without a work order: as sa_attn_work_order places them, each XCD (group
 // w of four slots runs on XCD w % 8) a contiguous range of items; -1 = idle.
 __device__ inline int xcd_item(const FwdArgs& a, int slot) {
@@ -362,7 +359,9 @@ __global__ __launch_bounds__(256, kD == 64 ? 2 : 1) void bsa_fwd_kernel(FwdArgs 
     part = rem / a.nqb;
     item = bh_s * a.nqb + (rem - part * a.nqb);
   } else {
-    item = __builtin_amdgcn_readfirstlane(a.order ? a.order[slot] : xcd_item(a, slot));
+    if (!a.order) item = xcd_item(a, slot);
+    else item = kShare ? a.order[slot] : order_item(a.order, slot);
+    item = __builtin_amdgcn_readfirstlane(item);
     if (kShare && a.order && item >= kSharedItem) {  // the group's four slots hold one item
       if (shared && (slot & (kWaves - 1)) != 0) return;  // (the same for the whole workgroup)
       shared = true;
@@ -1142,7 +1141,7 @@ __global__ __launch_bounds__(128, 2) void bsa_fwd_pair_kernel(FwdArgs a) {
   const int x = blockIdx.x;
   const int slot = 4 * (8 * (x >> 5) + (x & 7)) + ((x >> 3) & 3);
   int item = -1;
-  if (slot < a.n_slots) item = __builtin_amdgcn_readfirstlane(a.order ? a.order[slot] : xcd_item(a, slot));
+  if (slot < a.n_slots) item = __builtin_amdgcn_readfirstlane(a.order ? order_item(a.order, slot) : xcd_item(a, slot));
   // Both waves take the same branch: no barrier is left unmatched.
   if (item < 0 || item >= a.n_items) return;
   const int bh = item / a.nqb;
@@ -1479,6 +1478,9 @@ __global__ __launch_bounds__(128, 2) void bsa_fwd_pair_kernel(FwdArgs a) {
 
 namespace {
 
+// Slots that n_items take with one item each (in xcd_item's and sa_attn_work_order's layout).
+int64_t plain_slots(int64_t n_items) { return ((n_items + 7) / 8 + kWaves - 1) / kWaves * 8 * kWaves; }
+
 // The work order; with share_text a text row's item takes a whole group of four slots, each
 // holding item + kSharedItem.
 int build_work_order(const char* fn, int B, int H, int nqb, int n_text_blocks, int n_xcd, bool share_text,
@@ -1499,6 +1501,10 @@ int build_work_order(const char* fn, int B, int H, int nqb, int n_text_blocks, i
     const int64_t n = lo[x + 1] - lo[x], shared = texts(lo[x + 1]) - texts(lo[x]);
     wg_per_xcd = std::max(wg_per_xcd, shared + (n - shared + kWaves - 1) / kWaves);
   }
+  // A launch tells a long order from a plain one by its slots (launch_variant): one shared item among
+  // n = 1 mod 4 of an XCD would fit the plain order's.
+  if (texts(n_items) > 0)
+    while (wg_per_xcd * n_xcd * kWaves <= plain_slots(n_items)) ++wg_per_xcd;
   const int64_t total = wg_per_xcd * n_xcd * kWaves;
   *n_slots = total;
   if (!order) return sa::ok();
@@ -1632,10 +1638,8 @@ size_t split_workspace_bytes(int64_t n_items, int D, int parts) {
 constexpr int64_t kShareRound = 1024;
 constexpr int64_t kShareMax = 704;
 
-// Slots that n_items take with one item each (in xcd_item's and sa_attn_work_order's layout).
-int64_t plain_slots(int64_t n_items) { return ((n_items + 7) / 8 + kWaves - 1) / kWaves * 8 * kWaves; }
-
-// extra: slots past plain_slots, three for each item that already has a group of its own.
+// extra: slots past plain_slots, three for each item that already has a group of its own. Only a long
+// order has any (build_work_order), and it is then run by a kernel that shares its items.
 int shared_from(int64_t n_slots, int64_t extra) {
   const int64_t left = (n_slots - extra / 24 * 32) % kShareRound;
   return (int)((left > 0 && left <= kShareMax ? n_slots - left : n_slots) / kWaves);

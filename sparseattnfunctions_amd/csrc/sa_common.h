@@ -71,6 +71,16 @@ int64_t attn_f32_terms_bytes(int B, int Hk, int Lk, int D);
     if (!(cond)) return ::sa::fail(SA_ERR_INVALID, __VA_ARGS__); \
   } while (0)
 
+// Added to the item in the four slots of a group that share it (sa_attn_work_order_long).
+constexpr int kSharedItem = 1 << 30;
+
+// Item of a work order's slot for a kernel that runs one wave (or pair) per item: a shared item
+// runs in the first slot of its group and leaves the others idle (-1).
+__device__ inline int order_item(const int32_t* order, int slot) {
+  const int item = order[slot];
+  return item < kSharedItem ? item : (slot & 3) ? -1 : item - kSharedItem;
+}
+
 typedef __bf16 sa_bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 sa_bf16x4 __attribute__((ext_vector_type(4)));
 typedef float sa_f32x16 __attribute__((ext_vector_type(16)));

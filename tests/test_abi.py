@@ -121,6 +121,33 @@ def test_long_work_order_gives_each_text_row_a_group(lib):
     assert lib.sa_attn_work_order_long(1, 1, 1, 0, 8, None, None) == _lib.SA_ERR_INVALID
 
 
+def test_long_work_order_is_told_from_a_plain_one(lib):
+    """A launch shares the items of a long order exactly when it has more slots than the plain order
+    for eight XCDs: so it has, with one shared item or many, for any number of XCDs, and each item
+    is there once."""
+    import torch
+    n, plain, other = ctypes.c_int64(0), ctypes.c_int64(0), ctypes.c_int64(0)
+    for BH in range(1, 61):
+        for nqb in range(2, 301):
+            assert lib.sa_attn_work_order(1, BH, nqb, 0, 8, None, ctypes.byref(plain)) == 0
+            for nt in range(5):
+                assert lib.sa_attn_work_order_long(1, BH, nqb, nt, 8, None, ctypes.byref(n)) == 0
+                assert (n.value > plain.value) if nt else (n.value == plain.value), (BH, nqb, nt)
+            assert lib.sa_attn_work_order_long(1, BH, nqb, 1, 1 + nqb % 7, None, ctypes.byref(other)) == 0
+            assert other.value > plain.value, (BH, nqb)
+    # one text item in each XCD's range of 1 mod 4 items: it fits the plain order's slots
+    for BH, nqb, n_xcd in [(8, 217, 8), (8, 221, 8), (7, 247, 8), (1, 5, 1), (8, 5, 8), (1, 13, 3)]:
+        assert lib.sa_attn_work_order_long(1, BH, nqb, 1, n_xcd, None, ctypes.byref(n)) == 0
+        order = torch.full((n.value + 4,), 7, dtype=torch.int32)
+        assert lib.sa_attn_work_order_long(1, BH, nqb, 1, n_xcd, order.data_ptr(), ctypes.byref(n)) == 0
+        assert (order[n.value:] == 7).all()
+        order = order[:n.value]
+        shared = order[order >= 1 << 30].view(-1, 4) - (1 << 30)
+        assert (shared == shared[:, :1]).all() and shared.shape[0] == BH
+        items = torch.cat([shared[:, 0], order[(order >= 0) & (order < 1 << 30)]])
+        assert torch.equal(items.sort().values, torch.arange(BH * nqb, dtype=torch.int32))
+
+
 def test_split_parts_query(lib):
     parts = ctypes.c_int(-1)
     assert lib.sa_attn_split_parts(0, 128, 64, 256, ctypes.byref(parts)) == _lib.SA_ERR_INVALID

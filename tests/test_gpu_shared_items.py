@@ -1,5 +1,6 @@
 """Query blocks left over after whole rounds of the card are shared by four waves each
 (`shared_from` in csrc/attn_fwd.hip): launches on both sides of the rule's lines."""
+import ctypes
 import math
 
 import pytest
@@ -7,6 +8,7 @@ import torch
 
 from oracle.attention import masked_attention
 from oracle.pooling import pooled_attention
+from sparseattnfunctions_amd import _lib
 from sparseattnfunctions_amd._kv import kv_list_from_mask
 from sparseattnfunctions_amd.utils.attn_pooling_kernel import attn_with_pooling
 from sparseattnfunctions_amd.utils.block_sparse_attn_kernel import block_sparse_attention, shares_text_rows
@@ -88,3 +90,126 @@ def test_shared_text_rows(H, text, mode):
         err = (out[b, h].cpu().double() - want[b, h]).abs()
         assert err.max() <= 2e-2 and err.mean() <= 2e-3, (h, err.max().item())
     assert torch.all(out[0, H - 1, :64] == 0)  # an empty list
+
+
+def _text_rows_everywhere(dev, H, nb, text, tail, dtype=torch.bfloat16, D=64):
+    """q, k, v of nb blocks, the last of `tail` tokens; lists of the text blocks, one block of the
+    row's own and every block for text rows, and those lists' mask."""
+    L = 64 * (nb - 1) + tail
+    g = torch.Generator(dev).manual_seed(H * nb)
+    q, k, v = (torch.randn(1, H, L, D, device=dev, generator=g).to(dtype) for _ in range(3))
+    mask = torch.eye(nb, dtype=torch.bool, device=dev).repeat(1, H, 1, 1)
+    mask[:, :, :text] = True
+    mask[:, :, :, :text] = True
+    kv = kv_list_from_mask(mask, 1, H, nb, nb)
+    kv.row_blocks = text + 1
+    return q, k, v, kv, mask
+
+
+def _rows_in_64_bits(q, k, v, mask, rows, bias=None):
+    """Outputs of query blocks `rows` of every head, [H, 64 len(rows), D]."""
+    out = []
+    for h in range(q.shape[1]):
+        idx = torch.cat([torch.arange(64 * r, min(64 * r + 64, q.shape[2]), device=q.device) for r in rows])
+        s = q[0, h, idx].double() @ k[0, h].double().T.contiguous() * 0.125
+        if bias is not None:
+            s += bias[0, h].double()
+        keep = mask[0, h, idx // 64].repeat_interleave(64, dim=1)[:, :k.shape[2]]
+        out.append(torch.softmax(s.masked_fill(~keep, -math.inf), dim=-1) @ v[0, h].double())
+    return torch.stack(out), idx
+
+
+# One text block per head, one or no head starting in each XCD's range of 1 mod 4 items: the text
+# rows' groups would fit the slots of the order without them (1 760, 1 792, 1 760; with a bias,
+# which never takes key-range parts, 1 024), of which no remainder is shared.
+@pytest.mark.parametrize("H,nb,biased", [(8, 217, False), (8, 221, False), (7, 247, False), (8, 125, True)])
+def test_one_text_row_per_range(H, nb, biased):
+    print(f"case shared items one text row per range H={H} nb={nb} biased={biased}", flush=True)
+    dev = torch.device("cuda:0")
+    q, k, v, kv, mask = _text_rows_everywhere(dev, H, nb, 1, 2)
+    assert shares_text_rows(H * nb, nb, 1, kv.row_blocks, 64)
+    bias = torch.randn(1, H, q.shape[2], device=dev) if biased else None
+    out = torch.full_like(q, math.nan)
+    block_sparse_attention(q, k, v, kv, 0.125, key_bias=bias, n_text_blocks=1, out=out)
+    assert torch.isfinite(out).all()
+    want, idx = _rows_in_64_bits(q, k, v, mask, (0, 1, nb - 1), bias)
+    err = (out[0][:, idx].double() - want).abs()
+    assert err.max() <= 2e-2 and err.mean() <= 2e-3, err.max().item()
+    kv.row_blocks = None  # the same lists without shared text rows
+    plain = block_sparse_attention(q, k, v, kv, 0.125, key_bias=bias, n_text_blocks=1)
+    assert (out - plain).abs().max() <= 2e-2
+
+
+# Token masks with text rows in groups of their own: one text block that would fit the plain order's
+# 736, 960 and 1 024 slots, and two.
+@pytest.mark.parametrize("config,H", [
+    (dict(kernel_size=(1, 3, 3), tile_size=(12, 3, 3), img_size=(12, 21, 36), text_length=51), 5),
+    (dict(kernel_size=(1, 5, 5), tile_size=(11, 3, 3), img_size=(11, 27, 33), text_length=58), 6),
+    (dict(kernel_size=(1, 5, 5), tile_size=(11, 3, 3), img_size=(11, 24, 30), text_length=49), 8),
+    (dict(kernel_size=(1, 3, 3), tile_size=(12, 3, 3), img_size=(12, 21, 36), text_length=100), 5),
+])
+def test_text_rows_beside_token_masks(config, H):
+    print(f"case shared items sliding {config} H={H}", flush=True)
+    from sparseattnfunctions_amd._kv import KVList
+    from sparseattnfunctions_amd.SildingTileAttention import SildingTileAttention
+
+    dev, text = torch.device("cuda:0"), config["text_length"]
+    layer = SildingTileAttention(config)
+    T, Hp, Wp = config["img_size"]
+    L = text + T * Hp * Wp
+    g = torch.Generator(dev).manual_seed(H)
+    q, k, v = (torch.randn(1, H, L, 64, device=dev, generator=g).bfloat16() for _ in range(3))
+    lay = layer._get_layout(dev)
+    assert shares_text_rows(H * lay.nb, lay.nb, lay.text_blocks, lay.row_blocks, 64, True)
+    out = torch.full_like(q, math.nan)
+    kv = KVList(lay.kv_idx, lay.kv_cnt, 1, 1, lay.nb, lay.nb, row_blocks=lay.row_blocks)
+    opts = dict(n_text_blocks=lay.text_blocks, tile_masks=(lay.kv_slot, lay.masks, True))
+    block_sparse_attention(q, k, v, kv, 0.125, out=out, **opts)
+    assert torch.isfinite(out).all()
+    kv.row_blocks = None
+    plain = block_sparse_attention(q, k, v, kv, 0.125, **opts)
+    assert (out - plain).abs().max() <= 2e-2
+    want = torch.stack([torch.softmax(q[0, h, :text].double() @ k[0, h].double().T.contiguous() / 8, dim=-1)
+                        @ v[0, h].double() for h in range(H)])
+    err = (layer(q, k, v)[0, :, :text].double() - want).abs()
+    assert err.max() <= 2e-2 and err.mean() <= 2e-3, err.max().item()
+
+
+# Kernels that never share an item run a long order's in the group's first slot: the plain order's
+# bits.
+@pytest.mark.parametrize("dtype,D,terms", [(torch.bfloat16, 128, False), (torch.float16, 128, False),
+                                           (torch.float32, 64, False), (torch.float32, 128, False),
+                                           (torch.float32, 64, True), (torch.float32, 128, True)])
+@pytest.mark.parametrize("H,nb", [(3, 9), (8, 13)])
+def test_long_order_in_kernels_that_do_not_share(dtype, D, terms, H, nb):
+    print(f"case long order unshared {dtype} D={D} terms={terms} H={H} nb={nb}", flush=True)
+    dev, lib = torch.device("cuda:0"), _lib.load()
+    q, k, v, kv, _ = _text_rows_everywhere(dev, H, nb, 2, 33, dtype, D)
+    L, st = q.shape[2], _lib.i64(*q.stride()[:3])
+    ws = None
+    if terms:
+        n = ctypes.c_int64(0)
+        _lib.check(lib.sa_block_sparse_fwd_f32_terms_workspace(1, H, L, D, ctypes.byref(n)), "workspace")
+        ws = torch.empty(n.value, dtype=torch.uint8, device=dev)
+    outs = []
+    for name in ("sa_attn_work_order", "sa_attn_work_order_long"):
+        n = ctypes.c_int64(0)
+        build = getattr(lib, name)
+        _lib.check(build(1, H, nb, 2, 8, None, ctypes.byref(n)), name)
+        order = torch.empty(n.value, dtype=torch.int32)
+        _lib.check(build(1, H, nb, 2, 8, order.data_ptr(), ctypes.byref(n)), name)
+        order = order.to(dev)
+        out = torch.full_like(q, math.nan)
+        args = [q.data_ptr(), st, k.data_ptr(), st, v.data_ptr(), st, out.data_ptr(), st, 1, H, L, L, D,
+                kv.idx.data_ptr(), kv.cnt.data_ptr(), kv.max_cnt]
+        if terms:
+            rc = lib.sa_block_sparse_fwd_f32_terms(*args, 0.125, order.data_ptr(), order.numel(), ws.data_ptr(),
+                                                   ws.numel(), _lib.stream_of(q))
+        else:
+            fn = {torch.bfloat16: "sa_block_sparse_fwd", torch.float16: "sa_block_sparse_fwd_f16",
+                  torch.float32: "sa_block_sparse_fwd_f32"}[dtype]
+            rc = getattr(lib, fn)(*args, None, None, 0.125, order.data_ptr(), order.numel(), _lib.stream_of(q))
+        _lib.check(rc, name)
+        outs.append(out)
+    torch.cuda.synchronize()
+    assert torch.isfinite(outs[0]).all() and torch.equal(outs[0], outs[1])
