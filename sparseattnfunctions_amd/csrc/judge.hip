@@ -453,8 +453,10 @@ __global__ __launch_bounds__(64 * kTmWaves, 4) void topk_mass_kernel(TopkMassArg
     mx = fmaxf(mx, wred[w][0][col]);
     mn = fminf(mn, wred[w][1][col]);
   }
-  const float m = mx * a.scale_log2;
-  auto e_of = [&](float x) { return __builtin_amdgcn_exp2f(fmaf(x, a.scale_log2, -m)); };
+  // The difference is formed before the scaling: it is exactly 0 at the row's maximum, so e <= 1, the
+  // bins' top, whatever the scores' size (mx * scale rounded first is off by 2^-14 at 1 024, and the
+  // largest e by 344 patterns).
+  auto e_of = [&](float x) { return __builtin_amdgcn_exp2f((x - mx) * a.scale_log2); };
   if (t < 32) {
     // Patterns from just below the smallest e to just above 1 (exp2 may round either way).
     const uint32_t lo = min(__float_as_uint(e_of(mn)), 0x3f800000u);

@@ -49,6 +49,22 @@ def test_topk_mass(dev, kind, n, K, rows):
     assert torch.equal(share, again)  # whatever the order of the lists
 
 
+# Rows of equal scores so large that their scaled maximum, rounded, leaves a remainder: every entry is
+# the row's largest, so the K largest hold K / n of the mass.
+@pytest.mark.parametrize("n,K", [(100, 20), (1000, 200), (16384, 3276)])
+@pytest.mark.parametrize("x,y", [(10, 9), (300, 70), (-3, 1000), (2.0 ** 20, 2.0 ** 19 + 4096)])
+def test_topk_mass_of_large_equal_scores(dev, n, K, x, y):
+    print(f"case topk_mass equal scores {x} * {y} n={n} K={K}", flush=True)
+    q = torch.full((1, 3, 33, 64), float(x)).bfloat16().to(dev)
+    k = torch.full((1, 3, n, 64), float(y)).bfloat16().to(dev)
+    qs = pa._compact(q, torch.arange(33), 64)
+    ks = pa._key_operands(k, torch.arange(n), pa._pad32(n))
+    share = torch.full((3, 33), -1.0, device=dev)
+    _lib.check(_lib.load().sa_topk_mass(qs.data_ptr(), ks.data_ptr(), 3, 33, 64, n, pa._pad32(n), 0.125, K,
+                                        share.data_ptr(), _lib.stream_of(q)), "sa_topk_mass")
+    assert torch.allclose(share.double(), torch.full_like(share, K / n, dtype=torch.float64), rtol=2e-6, atol=0)
+
+
 # Frames of one tile, of a tile and a remainder, and of many; text shorter than a tile, of many
 # tiles and absent; scores whose sums leave the first walk's range (a second walk).
 @pytest.mark.parametrize("F,ns,T,amp", [(1, 5, 0, 1.0), (4, 32, 7, 1.0), (11, 37, 224, 1.0), (12, 9, 33, 1.0),
