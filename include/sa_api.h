@@ -201,10 +201,10 @@ int sa_block_sparse_fwd_f32(const float* q, const int64_t q_strides[3], const fl
  * (and P) split exactly into three bf16 terms and each product into the six term products down
  * to 2^-18 of the largest, accumulated in fp32; errors against a 64-bit softmax are no larger
  * than sa_block_sparse_fwd_f32's. The call first writes the split k and v to the workspace
- * (`sa_block_sparse_fwd_f32_terms_workspace` bytes, 256-byte aligned). Heads whose |k| or |v|
- * reach 2^60 (inf and NaN included) or whose |v| all lie below 2^-80, query blocks whose |q|
- * reach 2^60, and heads with fewer than 3/2 listed tiles per key block are computed as
- * sa_block_sparse_fwd_f32 does.
+ * (`sa_block_sparse_fwd_f32_terms_workspace` bytes, 256-byte aligned). Heads in which a |k| or |v|
+ * reaches 2^60 (inf and NaN included) or, other than 0, lies below 2^-80, query blocks (halves at
+ * D = 128) with such a |q|, and heads with fewer than 3/2 listed tiles per key block are computed
+ * as sa_block_sparse_fwd_f32 does.
  */
 int sa_block_sparse_fwd_f32_terms_workspace(int B, int H, int Lk, int D, int64_t* bytes);
 int sa_block_sparse_fwd_f32_terms(const float* q, const int64_t q_strides[3], const float* k,

@@ -300,15 +300,18 @@ __global__ __launch_bounds__(64 * kWavesF32, kD == 64 ? 2 : 1) void bsa_fwd_f32_
 //     3 (dc % 2) + term, lane (col, hh) holds V[32 c + 16 u + 8 (j / 4) + 4 hh + j % 4]
 //     [32 dc + col], j < 8: the A operand of O^T = V^T P^T for the key slots in which S^T leaves P.
 // Rows past Lk are zero. flags[head * nkb + block] = the largest |k| of the block's two chunks
-// and the largest |v| of its two chunks (fp32 bits): the attention takes the split operands only
-// where all are below kTermMax (no inf or NaN, no product near overflow) and the values not all
-// below kTermMin (their low terms would leave bf16's normal range); other heads run in fp32.
+// and the largest |v| of its two chunks (fp32 bits), or kTermMax where one of a chunk's values is
+// not 0 but below kTermMin. The attention takes the split operands only where all are below
+// kTermMax: no inf or NaN, no product near overflow, and every value's low term (2^-16 of it) and
+// its products with probabilities far enough above 2^-126. Other heads run in fp32. (One value
+// decides for its head: a column or block of small values beside ordinary ones would lose its
+// low terms however large the head's maximum is.)
 // A head whose lists hold fewer than 3/2 tiles per key block is not worth the pass: its blocks
 // are only flagged (kTermSkip) and it runs in fp32. Measured on [2, 30, 17776, 64] (fp32 kernel
 // against this path, us): 2.1 tiles per block 586 / 609, 2.7 695 / 659, 4.3 993 / 801; with one
 // tile per block of [2, 30, 3000, 64] 49 / 92.
 constexpr uint32_t kTermMax = 0x5d800000u;  // 2^60
-constexpr uint32_t kTermMin = 0x17800000u;  // 2^-80
+constexpr uint32_t kTermMin = 0x17800000u;  // 2^-80: 2^18 products that lose 2^-126 lose 2^-28 of a value
 constexpr uint32_t kTermSkip = 0xffffffffu;  // no |x| has these bits
 
 template <int kD>
@@ -337,6 +340,17 @@ __device__ inline void split3(float x0, float x1, uint32_t& hi, uint32_t& mid, u
 }
 
 __device__ inline uint32_t abs_bits(float x) { return __float_as_uint(x) & 0x7fffffffu; }
+
+// Largest and, 0 apart, smallest |x| of a wave's operands.
+struct TermRange {
+  uint32_t hi = 0u, lo1 = 0xffffffffu;  // lo1: the smallest less one, so that 0 counts as the largest
+  __device__ void add(float x) {
+    const uint32_t b = abs_bits(x);
+    hi = max(hi, b);
+    lo1 = min(lo1, b - 1u);
+  }
+  __device__ uint32_t flag() const { return lo1 < kTermMin - 1u ? max(hi, kTermMax) : hi; }
+};
 
 __device__ inline uint32_t wave_max_u(uint32_t x) {
 #pragma unroll
@@ -384,7 +398,7 @@ __global__ __launch_bounds__(256) void f32_terms_kernel(TermArgs a) {
   const int c = wave & 1;
   const int key0 = kb * kBlk + 32 * c;
   uint8_t* dst = a.planes + blk * Lay::kTile + c * Lay::kGroups * Lay::kGroup + 16 * lane;
-  uint32_t amax = 0u;
+  TermRange range;
   auto put = [&](int group, int operand, const float (&x)[8]) {
     f32_u32x4 t[3];
 #pragma unroll
@@ -394,7 +408,8 @@ __global__ __launch_bounds__(256) void f32_terms_kernel(TermArgs a) {
       t[0][i] = hi;
       t[1][i] = mid;
       t[2][i] = lo;
-      amax = max(amax, max(abs_bits(x[2 * i]), abs_bits(x[2 * i + 1])));
+      range.add(x[2 * i]);
+      range.add(x[2 * i + 1]);
     }
 #pragma unroll
     for (int p = 0; p < 3; ++p)
@@ -428,8 +443,8 @@ __global__ __launch_bounds__(256) void f32_terms_kernel(TermArgs a) {
         put(Lay::kKGroups + u * (kD / 64) + (dc >> 1), 3 * (dc & 1), x);
       }
   }
-  amax = wave_max_u(amax);
-  if (lane == 0) a.flags[blk * 4 + wave] = amax;
+  const uint32_t flag = wave_max_u(range.flag());
+  if (lane == 0) a.flags[blk * 4 + wave] = flag;
 }
 
 __device__ inline sa_f32x16 mfma_bf16(f32_u32x4 x, f32_u32x4 y, sa_f32x16 c) {
@@ -517,12 +532,12 @@ __global__ __launch_bounds__(256, 2) void bsa_fwd_f32_terms_kernel(F32Args a) {
   f32_u32x4* ql = q_lds[wave];
   bool use_terms = (uint32_t)__builtin_amdgcn_readfirstlane((int)fl[0].x) != kTermSkip;
   if (use_terms) {
-    // The head's largest |k| and |v| and this wave's largest |q|.
-    uint32_t kmax = 0u, vmax = 0u;
+    // The flags of the head's blocks and of this wave's query rows.
+    uint32_t worst = 0u;
+    TermRange range;
     for (int j = 0; j < a.nkb; j += 64) {
       const uint4 f = fl[min(j + lane, a.nkb - 1)];
-      kmax = max(kmax, max(f.x, f.y));
-      vmax = max(vmax, max(f.z, f.w));
+      worst = max(worst, max(max(f.x, f.y), max(f.z, f.w)));
     }
 #pragma unroll
     for (int g = 0; g < kG; ++g) {
@@ -541,16 +556,14 @@ __global__ __launch_bounds__(256, 2) void bsa_fwd_f32_terms_kernel(F32Args a) {
           qhi[g][s][i] = t0;
           mid[i] = t1;
           lo[i] = t2;
-          kmax = max(kmax, max(abs_bits(y[2 * i]), abs_bits(y[2 * i + 1])));
+          range.add(y[2 * i]);
+          range.add(y[2 * i + 1]);
         }
         ql[(g * kDS + s) * 64 + lane] = mid;
         ql[((kG + g) * kDS + s) * 64 + lane] = lo;
       }
     }
-    kmax = wave_max_u(kmax);
-    vmax = wave_max_u(vmax);
-    use_terms = __builtin_amdgcn_readfirstlane(kmax < kTermMax && vmax < kTermMax &&
-                                               (vmax >= kTermMin || vmax == 0u));
+    use_terms = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_max_u(max(worst, range.flag()))) < kTermMax;
   }
 
   float* part = reinterpret_cast<float*>(q_lds[wave]);  // kKW = 4: [row][16-byte chunk ^ row % 16]

@@ -87,6 +87,41 @@ def test_out_of_range_operands(dev, monkeypatch, D, where, value):
     assert not torch.equal(new[0, 1], old[0, 1])  # the other heads took the split operands
 
 
+# A block, column or element of small values inside an ordinary head: their low terms would leave
+# bf16's range (and a query row's its own), so the head (or row group) runs in fp32: the same bits.
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("where,value", [("v block", 2.0 ** -115), ("v column", 2.0 ** -110), ("v", 2.0 ** -140),
+                                          ("k", -2.0 ** -100), ("q", 2.0 ** -90)])
+def test_small_values_in_an_ordinary_head(dev, monkeypatch, D, where, value):
+    print(f"case terms small values {D} {where} {value}", flush=True)
+    # one wave per unit, so that both kernels visit the tiles of a row in the same order
+    B, H, L = 1, 26 if D == 64 else 13, 15360
+    q, k, v = (_rand(i, B, H, L, D).to(dev) for i in (4, 5, 6))
+    v[0, 1, 128:192] = 0  # zeros are no small values
+    if where == "v block":
+        v[0, 0, 64:128] *= value
+    elif where == "v column":
+        v[0, 0, :, 5] *= value
+    else:
+        {"v": v, "k": k, "q": q}[where][0, 0, 70, 3] = value
+    nb = L // 64
+    mask = torch.zeros(1, 1, nb, nb, dtype=torch.bool)
+    mask[..., :4] = True
+    mask[..., 7, :] = torch.arange(nb) == 1  # a row of the small block alone
+    kv = kv_list_from_mask(mask.to(dev), B, H, nb, nb)
+    args = (q, k, v, kv, 0.125)
+    new, old = bsk.block_sparse_attention(*args), _plain(monkeypatch, *args)
+    rows = slice(64, 128 if D == 64 else 96) if where == "q" else slice(None)
+    assert torch.equal(new[0, 0, rows], old[0, 0, rows])
+    assert not torch.equal(new[0, 1], old[0, 1])  # the other heads took the split operands
+    if where.startswith("v "):
+        s = q[0, 0, 448:512].double() @ k[0, 0, 64:128].double().T.contiguous() * 0.125
+        want = torch.softmax(s, dim=-1) @ v[0, 0, 64:128].double()
+        cols = slice(5, 6) if where == "v column" else slice(None)
+        got, want = new[0, 0, 448:512, cols].double(), want[:, cols]
+        assert (got - want).norm() <= 4e-6 * want.norm()  # a few fp32 roundings of 64 products
+
+
 def test_short_lists_and_strided_rows(dev, monkeypatch):
     # head 0: one tile per key block (fp32 bits); head 1: five; BLHD views
     print("case terms short lists", flush=True)
