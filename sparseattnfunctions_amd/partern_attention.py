@@ -364,11 +364,18 @@ def _similarity_gram(q, k, g: PatternGeometry, index_k):
     n = ctypes.c_int64(0)
     lib = _lib.load()
     _lib.check(lib.sa_pattern_sim_gram_workspace(qs.shape[0], F, ns, ctypes.byref(n)), "sa_pattern_sim_gram_workspace")
-    ws = torch.empty(n.value, dtype=torch.uint8, device=q.device)  # each position's products, until its sums are known
+    args = (qs.data_ptr(), ks.data_ptr(), qs.shape[0], F, ns, T, qs.shape[1], ks.shape[1], scale_factor,
+            composition_bias(g), G.data_ptr())
+    try:  # each position's products, until its sums are known
+        ws = torch.empty(n.value, dtype=torch.uint8, device=q.device)
+    except torch.cuda.OutOfMemoryError:  # two walks over the keys instead of one
+        ws = None
     with _lib.on(q.device):
-        _lib.check(lib.sa_pattern_sim_gram_ws(
-            qs.data_ptr(), ks.data_ptr(), qs.shape[0], F, ns, T, qs.shape[1], ks.shape[1], scale_factor,
-            composition_bias(g), G.data_ptr(), ws.data_ptr(), ws.numel(), _lib.stream_of(q)), "sa_pattern_sim_gram_ws")
+        if ws is not None:
+            _lib.check(lib.sa_pattern_sim_gram_ws(*args, ws.data_ptr(), ws.numel(), _lib.stream_of(q)),
+                       "sa_pattern_sim_gram_ws")
+        else:
+            _lib.check(lib.sa_pattern_sim_gram(*args, _lib.stream_of(q)), "sa_pattern_sim_gram")
     return G
 
 

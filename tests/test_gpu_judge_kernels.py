@@ -85,3 +85,32 @@ def test_sim_gram_one_walk(dev, F, ns, T, amp):
     # products of two probabilities: 2^-126 of the largest are lost
     assert torch.allclose(two, probs, rtol=4e-5, atol=1e-9), (two - probs).abs().max()
     assert torch.allclose(one, probs, rtol=4e-5, atol=1e-9), (one - probs).abs().max()
+
+
+def test_judge_without_memory_for_the_workspace(dev, monkeypatch):
+    print("case unified_judge without the Gram workspace", flush=True)
+    geo = pa.PatternGeometry(frames=5, height=20, width=24, text_length=30, sample_num=100)
+    g = torch.Generator().manual_seed(3)
+    q, k = (torch.randn(1, 6, geo.L, 64, generator=g) for _ in range(2))
+    for x in (q, k):  # half of the heads repeat one frame
+        frames = x[:, :3, 30:].view(1, 3, 5, 480, 64)
+        frames.copy_(frames[:, :, :1] + 0.1 * frames)
+    q, k = q.bfloat16().to(dev), k.bfloat16().to(dev)
+    torch.manual_seed(3)
+    draws = (torch.randperm(geo.S)[:100], pa.get_indexs(geo)[1], pa.get_indexs(geo)[1])
+    want = pa.unified_judge(q, k, geo, draws)
+    _, sim = pa.judge_similarity(q, k, geo, draws[1], return_sim=True)
+    empty, refused = torch.empty, []
+
+    def full(*size, **kw):
+        if kw.get("dtype") == torch.uint8:
+            refused.append(size)
+            raise torch.cuda.OutOfMemoryError("no memory")
+        return empty(*size, **kw)
+
+    monkeypatch.setattr(torch, "empty", full)
+    got = pa.unified_judge(q, k, geo, draws)
+    _, sim2 = pa.judge_similarity(q, k, geo, draws[1], return_sim=True)
+    assert len(refused) == 3
+    assert torch.equal(got, want) and want.any() and not want.all()
+    assert torch.allclose(sim, sim2, rtol=4e-5)  # products of fp32 probabilities, as above
