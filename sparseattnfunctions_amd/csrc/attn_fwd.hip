@@ -89,7 +89,8 @@ struct FwdArgs {
   // forms the output. `order` is not read.
   int n_parts;
   float* ws;
-  int shared_from;  // kShare: the first dispatch group whose items are shared by four waves each
+  int shared_from;  // kShare: the first dispatch group whose items are shared by four waves each,
+  int share_min;    // if the longest of the group's lists has at least this many entries
   const int32_t* kv_idx;
   const int32_t* kv_cnt;
   int max_cnt;
@@ -345,7 +346,20 @@ __global__ __launch_bounds__(256, kD == 64 ? 2 : 1) void bsa_fwd_kernel(FwdArgs 
   int slot = blockIdx.x * kWaves + wave;
   if (shared) {  // a shared group is four workgroups, on the group's XCD
     const int y = blockIdx.x - a.shared_from;
-    slot = 4 * (a.shared_from + 8 * (y >> 5) + (y & 7)) + ((y >> 3) & 3);
+    const int first = 4 * (a.shared_from + 8 * (y >> 5) + (y & 7)), part = (y >> 3) & 3;
+    slot = first + part;
+    if (kPool == 0 && a.share_min > 0 && first < a.n_slots) {  // (n_slots is a multiple of four)
+      // Lane l looks at the list of slot l % 4: one load of each kind for the group.
+      const int j = first + (lane & (kWaves - 1));
+      const int it = a.order ? a.order[j] : xcd_item(a, j);
+      bool share = it >= kSharedItem;
+      if (it >= 0 && it < a.n_items) share = a.kv_cnt[a.list_bh_stride ? it : it % a.nqb] >= a.share_min;
+      if (__ballot(share) == 0) {  // the first workgroup runs all four
+        if (part > 0) return;
+        shared = false;
+        slot = first + wave;
+      }
+    }
   }
   if (slot >= a.n_slots) return;
   // Key-range parts exist for plain lists only; the other variants compile without them.
@@ -1637,6 +1651,7 @@ size_t split_workspace_bytes(int64_t n_items, int D, int parts) {
 // per item down (316 -> 339 us, [2, 30, 12000, 64] with a tenth of the blocks).
 constexpr int64_t kShareRound = 1024;
 constexpr int64_t kShareMax = 704;
+constexpr int kResident = 512;  // workgroups of these kernels that the card holds at once
 
 // extra: slots past plain_slots, three for each item that already has a group of its own. Only a long
 // order has any (build_work_order), and it is then run by a kernel that shares its items.
@@ -1645,9 +1660,23 @@ int shared_from(int64_t n_slots, int64_t extra) {
   return (int)((left > 0 && left <= kShareMax ? n_slots - left : n_slots) / kWaves);
 }
 
+// The shortest list worth sharing behind `from` unshared groups: a group of shorter ones keeps one wave
+// per item, in the first of its four workgroups. While all workgroups fit the card beside half of it,
+// lists of one tile gain already (192 of 1 216 slots: 12.8 / 11.6 us at 2 tiles, 23.0 / 17.9 at 8).
+// Measured beyond, one wave per item against four (us, lists of one length): workgroups that fit the
+// last round, 512 of 2 560 slots, 2 tiles 20.0 / 21.0, 6 tiles 30.4 / 30.3, 8 tiles 35.6 / 34.4; that
+// do not, 416 of 1 440, 4 tiles 16.4 / 20.8, 8 tiles 23.4 / 24.3, 16 tiles 37.7 / 34.4, of 3 488, 12
+// tiles 59.6 / 61.2; more than the card holds, 704 of 704, 4 tiles 10.3 / 13.3, 8 tiles 14.3 / 16.5,
+// 20 tiles 26.8 / 25.6.
+int share_min(int n_slots, int from) {
+  const int wgs = n_slots - kWaves * from, room = kResident - from % kResident;
+  return wgs <= kResident / 2 ? 0 : wgs <= room ? 8 : wgs <= kResident ? 16 : 20;
+}
+
 template <bool kBias, bool kMask, typename T, int kDV, bool kK16, int kPool = 0>
 void launch_shared(FwdArgs a, int from, hipStream_t s) {
   a.shared_from = from;
+  a.share_min = share_min(a.n_slots, from);  // (pooling lists are dense: their width has decided)
   const int64_t left = a.n_slots / kWaves - from;
   const dim3 g((unsigned)(from + (left + 7) / 8 * 32)), blk(64 * kWaves);
   hipLaunchKernelGGL((bsa_fwd_kernel<kBias, kMask, kPool, T, 64, kDV, kK16, true>), g, blk, 0, s, a);
@@ -1661,7 +1690,8 @@ void launch_variant(const FwdArgs& a, dim3 g, dim3 blk, hipStream_t s, bool mask
   if constexpr (kD == 64) {
     const bool may_share = a.n_parts == 1 && !(mask && pool_cols);
     const int64_t extra = a.order ? std::max<int64_t>(a.n_slots - plain_slots(a.n_items), 0) : 0;
-    const int from = may_share ? shared_from(a.n_slots, extra) : a.n_slots / kWaves;
+    int from = may_share ? shared_from(a.n_slots, extra) : a.n_slots / kWaves;
+    if (a.max_cnt < share_min(a.n_slots, from)) from = a.n_slots / kWaves;
     if (from < a.n_slots / kWaves || (may_share && extra > 0)) {
       if (pool_cols == 32) return launch_shared<false, false, T, 64, false, 32>(a, from, s);
       if (pool_cols == 64) return launch_shared<false, false, T, 64, false, 64>(a, from, s);

@@ -43,6 +43,49 @@ def test_lists_of_every_length(H, dtype, biased):
     assert torch.all(out[0, H - 1, :64] == 0)  # an empty list
 
 
+# Remainders whose short lists keep one wave each (`share_min`): 704 of 704 slots (from 20 tiles on),
+# 416 of 1 440 (16), 512 of 2 560 (8) and 320 of 2 368 (8), in groups of both kinds; and lists that
+# are all shorter, decided by their width.
+@pytest.mark.parametrize("H,nkb", [(70, 24), (144, 24), (256, 24), (236, 24), (70, 19), (144, 8), (256, 7)])
+@pytest.mark.parametrize("mode", ["bf16", "bias", "fp16", "plain order", "text rows"])
+def test_short_lists_keep_one_wave(H, nkb, mode):
+    print(f"case shared items short lists H={H} nkb={nkb} {mode}", flush=True)
+    dev, Lq, Lk = torch.device("cuda:0"), 617, 64 * nkb - 5
+    nqb = math.ceil(Lq / 64)
+    g = torch.Generator().manual_seed(H + nkb)
+    dtype = torch.float16 if mode == "fp16" else torch.bfloat16
+    q, k, v = (torch.randn(1, H, L, 64, generator=g).to(dtype) for L in (Lq, Lk, Lk))
+    # heads of empty and short lists, of long ones, and of both in one group
+    longest = torch.tensor([3, nkb, 12, 0])[torch.arange(H) % 4]
+    count = (torch.rand(H, nqb, generator=g) * (longest[:, None] + 1)).long()
+    count[:, 4] = longest
+    mask = torch.arange(nkb) < count[..., None].clamp(max=nkb)
+    text = 1 if mode == "text rows" else 0
+    mask[:, :text] = True
+    mask = mask[None]
+    bias = torch.randn(1, H, Lk, generator=g) if mode == "bias" else None
+    kv = kv_list_from_mask(mask.to(dev), 1, H, nqb, nkb)
+    if text:
+        kv.row_blocks = 0.1
+    out = torch.full((1, H, Lq, 64), math.nan, dtype=dtype, device=dev)
+    if mode == "plain order":  # no work order: the items by index
+        lib, st = _lib.load(), [_lib.i64(*t.to(dev).stride()[:3]) for t in (q, k, v)]
+        d = [t.to(dev) for t in (q, k, v)]
+        _lib.check(lib.sa_block_sparse_fwd(d[0].data_ptr(), st[0], d[1].data_ptr(), st[1], d[2].data_ptr(), st[2],
+                                           out.data_ptr(), st[0], 1, H, Lq, Lk, 64, kv.idx.data_ptr(),
+                                           kv.cnt.data_ptr(), kv.max_cnt, None, None, 0.125, None, 0,
+                                           _lib.stream_of(out)), "sa_block_sparse_fwd")
+    else:
+        block_sparse_attention(q.to(dev), k.to(dev), v.to(dev), kv, 0.125, out=out, n_text_blocks=text,
+                               key_bias=None if bias is None else bias.to(dev))
+    assert torch.isfinite(out).all()
+    heads = sorted({(0, h) for h in (0, 1, 2, 3, H // 2 + 1, H - 2, H - 1)})
+    want = masked_attention(q, k, v, mask, 0.125, key_bias=bias, heads=heads)
+    for b, h in heads:
+        err = (out[b, h].cpu().double() - want[b, h].nan_to_num()).abs()
+        assert err.max() <= 2e-2 and err.mean() <= 2e-3, (h, err.max().item())
+
+
 @pytest.mark.parametrize("H,block,causal", [(1, 64, False), (70, 32, False), (104, 64, False), (104, 64, True)])
 def test_pooled_map(H, block, causal):
     print(f"case shared items pooled H={H} block={block} causal={causal}", flush=True)
