@@ -103,7 +103,7 @@ int sa_cell_tile_masks(int block_m, int block_n, uint64_t* masks, int64_t* n_pat
  *             added to the scaled scores (proportional attention, MergeAttention.py:33-48).
  *   sm_scale  > 0 and finite.
  *   work_order nullable int32 [n_slots] from sa_attn_work_order (device copy): dispatch
- *             slot -> list row, -1 = idle. NULL gives each XCD a contiguous range of rows.
+ *             slot -> list row, -1 = idle. NULL visits rows in index order.
  * One wave per query block; at head dim 64 the blocks of a last round that leaves most of the card
  * idle run on four waves each, merged on chip (sa_block_sparse_fwd_split is the variant for few
  * query blocks over long lists, through a workspace).

@@ -79,9 +79,9 @@ struct FwdArgs {
   int64_t o_sb, o_sh, o_sl;
   int H, Lq, Lk, nqb, nkb;
   int n_items;             // B*H*nqb
-  const int32_t* order;    // dispatch slot -> item (bh*nqb + qb), -1 = idle; may be null: xcd_item
+  const int32_t* order;    // dispatch slot -> item (bh*nqb + qb), -1 = idle; may be null: xcd_ranges
   int n_slots;
-  int longest_last;        // without an order: each XCD's items in descending order
+  int xcd_ranges;          // without an order: range_item's ranges, else item = slot (xcd_ranges_pay)
   // Key-range split (n_parts > 1; plain lists only): slot (bh * n_parts + p) * nqb + qb
   // computes list positions [cnt * p / n_parts, cnt * (p + 1) / n_parts) of item bh * nqb + qb
   // and stores its unnormalised partial to ws[item * n_parts + p] (kSplitFloats each: acc
@@ -128,14 +128,15 @@ struct FwdArgs {
   const uint32_t* k16_norm2;
 };
 
-// Item of a dispatch slot without a work order: as sa_attn_work_order places them, each XCD (group
-// w of four slots runs on XCD w % 8) a contiguous range of items; -1 = idle.
-__device__ inline int xcd_item(const FwdArgs& a, int slot) {
+// Item of a dispatch slot in ranges: as sa_attn_work_order places them, each XCD (group w of four
+// slots runs on XCD w % 8) a contiguous range of items, from its start or (kDown) from its end; -1 = idle.
+template <bool kDown>
+__device__ inline int range_item(const FwdArgs& a, int slot) {
   const int w = slot / kWaves, x = w & 7;
   const int lo = (int)(((int64_t)a.n_items * x) >> 3), hi = (int)(((int64_t)a.n_items * (x + 1)) >> 3);
   const int i = (w >> 3) * kWaves + slot % kWaves;
   if (i >= hi - lo) return -1;
-  return a.longest_last ? hi - 1 - i : lo + i;
+  return kDown ? hi - 1 - i : lo + i;
 }
 
 __device__ inline sa_bf16x8 as_bf16x8(uint4 x) { return __builtin_bit_cast(sa_bf16x8, x); }
@@ -351,7 +352,7 @@ __global__ __launch_bounds__(256, kD == 64 ? 2 : 1) void bsa_fwd_kernel(FwdArgs 
     if (kPool == 0 && a.share_min > 0 && first < a.n_slots) {  // (n_slots is a multiple of four)
       // Lane l looks at the list of slot l % 4: one load of each kind for the group.
       const int j = first + (lane & (kWaves - 1));
-      const int it = a.order ? a.order[j] : xcd_item(a, j);
+      const int it = a.order ? a.order[j] : j;  // (pooling launches alone take ranges)
       bool share = it >= kSharedItem;
       if (it >= 0 && it < a.n_items) share = a.kv_cnt[a.list_bh_stride ? it : it % a.nqb] >= a.share_min;
       if (__ballot(share) == 0) {  // the first workgroup runs all four
@@ -373,8 +374,9 @@ __global__ __launch_bounds__(256, kD == 64 ? 2 : 1) void bsa_fwd_kernel(FwdArgs 
     part = rem / a.nqb;
     item = bh_s * a.nqb + (rem - part * a.nqb);
   } else {
-    if (!a.order) item = xcd_item(a, slot);
-    else item = kShare ? a.order[slot] : order_item(a.order, slot);
+    if (a.order) item = kShare ? a.order[slot] : order_item(a.order, slot);
+    else if (kPool != 0 && (kShare || a.xcd_ranges)) item = range_item<kMask>(a, slot);
+    else item = slot;
     item = __builtin_amdgcn_readfirstlane(item);
     if (kShare && a.order && item >= kSharedItem) {  // the group's four slots hold one item
       if (shared && (slot & (kWaves - 1)) != 0) return;  // (the same for the whole workgroup)
@@ -1155,7 +1157,7 @@ __global__ __launch_bounds__(128, 2) void bsa_fwd_pair_kernel(FwdArgs a) {
   const int x = blockIdx.x;
   const int slot = 4 * (8 * (x >> 5) + (x & 7)) + ((x >> 3) & 3);
   int item = -1;
-  if (slot < a.n_slots) item = __builtin_amdgcn_readfirstlane(a.order ? order_item(a.order, slot) : xcd_item(a, slot));
+  if (slot < a.n_slots) item = __builtin_amdgcn_readfirstlane(a.order ? order_item(a.order, slot) : slot);
   // Both waves take the same branch: no barrier is left unmatched.
   if (item < 0 || item >= a.n_items) return;
   const int bh = item / a.nqb;
@@ -1492,7 +1494,7 @@ __global__ __launch_bounds__(128, 2) void bsa_fwd_pair_kernel(FwdArgs a) {
 
 namespace {
 
-// Slots that n_items take with one item each (in xcd_item's and sa_attn_work_order's layout).
+// Slots that n_items take with one item each (in ranges of eight XCDs, sa_attn_work_order's layout).
 int64_t plain_slots(int64_t n_items) { return ((n_items + 7) / 8 + kWaves - 1) / kWaves * 8 * kWaves; }
 
 // The work order; with share_text a text row's item takes a whole group of four slots, each
@@ -1673,6 +1675,29 @@ int share_min(int n_slots, int from) {
   return wgs <= kResident / 2 ? 0 : wgs <= room ? 8 : wgs <= kResident ? 16 : 20;
 }
 
+// Whether a pooling launch, which has no work order, runs in ranges (range_item). They keep an XCD on
+// few heads, and causal lists, which grow with the query block, start with the longest; but causal
+// ranges hold equal numbers of rows and not of tiles (equal only where the heads deal out evenly),
+// and in a launch of one round the long rows meet on the same CUs. Measured on causal maps, index
+// order against ranges (us): head dim 64, [1, 16, 9000] 309 / 301, [2, 16, 8192] 518 / 383, [2, 30,
+// 17776] 3 385 / 3 142, [1, 30, 8192] 517 / 401, but [2, 15, 4200] 132 / 150, [1, 15, 17776] 959 /
+// 1 013, [1, 24, 4200] at 0.88 and [1, 27, 6000] at 0.94 of the rate; head dim 128, [1, 16, 9000] 849 /
+// 602, but [1, 15, 6000] at 0.94. Dense maps gain 1-5 % with 32-key columns and lose up to 2 %
+// otherwise ([1, 12, 4000] 87.9 / 89.9, head dim 128 [1, 15, 17776] 3 532 / 3 540); a shared
+// remainder takes the items that sa_attn_work_order puts last, so that a dense launch with an order
+// has the same bits.
+bool xcd_ranges_pay(int BH, int64_t n_items, int D, int max_cnt, int pool_cols, bool causal) {
+  if (!pool_cols) return false;
+  const bool even = BH % 8 == 0;
+  if (causal && D == 64)
+    return even ? n_items > 2112 || (n_items > 1024 && n_items <= 1408) : BH >= 16 && n_items > 2880;
+  if (causal) return n_items > (even ? 1024 : 1440);
+  if (D != 64) return false;
+  const int64_t n_slots = plain_slots(n_items);
+  const int from = shared_from(n_slots, 0);
+  return pool_cols == 32 || (from < n_slots / kWaves && max_cnt >= share_min((int)n_slots, from));
+}
+
 template <bool kBias, bool kMask, typename T, int kDV, bool kK16, int kPool = 0>
 void launch_shared(FwdArgs a, int from, hipStream_t s) {
   a.shared_from = from;
@@ -1688,7 +1713,8 @@ template <typename T, int kD>
 void launch_variant(const FwdArgs& a, dim3 g, dim3 blk, hipStream_t s, bool mask, bool bias, int pool_cols,
                     bool v32 = false) {
   if constexpr (kD == 64) {
-    const bool may_share = a.n_parts == 1 && !(mask && pool_cols);
+    // (A sharing pooling kernel runs in ranges, for which n_slots has to hold whole ones.)
+    const bool may_share = a.n_parts == 1 && (!pool_cols || (!mask && a.xcd_ranges));
     const int64_t extra = a.order ? std::max<int64_t>(a.n_slots - plain_slots(a.n_items), 0) : 0;
     int from = may_share ? shared_from(a.n_slots, extra) : a.n_slots / kWaves;
     if (a.max_cnt < share_min(a.n_slots, from)) from = a.n_slots / kWaves;
@@ -1772,10 +1798,11 @@ int launch_fwd(const uint16_t* q, const int64_t q_strides[3], const uint16_t* k,
   SA_REQUIRE(!o_rows || o_dst_rows > 0, "%s: o_rows given with o_dst_rows=%d", fn, o_dst_rows);
   const int64_t n_items = (int64_t)B * H * nqb;
   SA_REQUIRE(n_items < (1LL << 30), "%s: too many query blocks", fn);
+  const bool ranges = !work_order && xcd_ranges_pay(B * H, n_items, D, max_cnt, pool_cols, kv_slot != nullptr);
   if (work_order) {
     SA_REQUIRE(n_slots > 0 && n_slots % kWaves == 0, "%s: n_slots must be a positive multiple of 4", fn);
-  } else {  // xcd_item: each of the eight XCDs' ranges in whole groups
-    n_slots = plain_slots(n_items);
+  } else {
+    n_slots = ranges ? plain_slots(n_items) : (n_items + kWaves - 1) / kWaves * kWaves;
   }
   // 16-byte vector accesses: base pointers 16-byte aligned, row strides multiples of 8 elements.
   const void* ptrs[4] = {q, k, v, out};
@@ -1807,9 +1834,7 @@ int launch_fwd(const uint16_t* q, const int64_t q_strides[3], const uint16_t* k,
   a.n_items = (int)n_items;
   a.order = work_order;
   a.n_slots = (int)n_slots;
-  // Causal lists grow with the query block: the longest start first (and each XCD keeps to its
-  // heads: [2, 30, 17776, 64] pooled 3.29 -> 3.06 ms, in ascending order 3.25).
-  a.longest_last = pool_cols && kv_slot ? 1 : 0;
+  a.xcd_ranges = ranges;
   a.n_parts = 1;
   a.ws = nullptr;
   a.k16 = k16;

@@ -100,6 +100,28 @@ def test_pooled_map(H, block, causal):
         assert torch.allclose(po[:, h:h + 1].cpu().double(), want_po, rtol=5e-3, atol=1e-9)
 
 
+# Causal maps on both sides of the lines between index order and ranges (`xcd_ranges_pay`): 1 600
+# and 2 160 items of heads that deal out evenly, 2 870 and 2 890 of others, and dense maps whose
+# remainder is not shared.
+@pytest.mark.parametrize("H,block,causal", [(160, 64, True), (216, 32, True), (287, 64, True), (289, 128, True),
+                                            (85, 64, False), (85, 32, False), (85, 128, False)])
+def test_pooled_map_placement(H, block, causal):
+    print(f"case pooled placement H={H} block={block} causal={causal}", flush=True)
+    dev, L = torch.device("cuda:0"), 617
+    g = torch.Generator().manual_seed(H + block)
+    q, k, v = (torch.randn(1, H, L, 64, generator=g).bfloat16() for _ in range(3))
+    o, po = attn_with_pooling(q.to(dev), k.to(dev), v.to(dev), causal, 0.125, block)
+    for h in {0, H // 8, H // 2, H - 1}:
+        want_o, want_po = pooled_attention(*(t[:, h:h + 1] for t in (q, k, v)), causal, 0.125, block)
+        err = (o[:, h:h + 1].cpu().double() - want_o).abs()
+        assert err.max() <= 2e-2 and err.mean() <= 2e-3
+        assert torch.allclose(po[:, h:h + 1].cpu().double(), want_po, rtol=5e-3, atol=1e-9)
+    assert torch.isfinite(o).all() and torch.isfinite(po).all()
+    # a head's rows do not depend on where they run
+    alone, alone_po = attn_with_pooling(*(t[:, :1].to(dev) for t in (q, k, v)), causal, 0.125, block)
+    assert (o[:, :1] - alone).abs().max() <= 2e-2 and torch.allclose(po[:, :1], alone_po, rtol=5e-3, atol=1e-9)
+
+
 # Text rows in groups of their own before rows of one wave each: remainders shared (the
 # text rows apart) and not, and every row a text row.
 @pytest.mark.parametrize("H,text", [(71, 2), (74, 3), (90, 2), (104, 1), (72, 10)])
