@@ -203,8 +203,9 @@ int sa_block_sparse_fwd_f32(const float* q, const int64_t q_strides[3], const fl
  * than sa_block_sparse_fwd_f32's. The call first writes the split k and v to the workspace
  * (`sa_block_sparse_fwd_f32_terms_workspace` bytes, 256-byte aligned). Heads in which a |k| or |v|
  * reaches 2^60 (inf and NaN included) or, other than 0, lies below 2^-80, query blocks (halves at
- * D = 128) with such a |q|, and heads with fewer than 3/2 listed tiles per key block are computed
- * as sa_block_sparse_fwd_f32 does.
+ * D = 128) with such a |q|, and heads with too few listed tiles per key block for the split to pay
+ * (3/2 to 9/4, by size; none at D = 64 up to 128 query blocks) are computed as
+ * sa_block_sparse_fwd_f32 does.
  */
 int sa_block_sparse_fwd_f32_terms_workspace(int B, int H, int Lk, int D, int64_t* bytes);
 int sa_block_sparse_fwd_f32_terms(const float* q, const int64_t q_strides[3], const float* k,

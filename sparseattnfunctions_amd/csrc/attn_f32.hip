@@ -69,6 +69,7 @@ struct F32Args {
   // bsa_fwd_f32_terms_kernel: the split operands and the per-key-block flags (f32_terms_kernel).
   const uint8_t* planes;
   const uint4* flags;
+  int plain_after;  // bsa_fwd_f32_kernel follows for the heads flagged kTermSkip
 };
 
 __device__ inline sa_f32x4 mfma16x4(float a, float b, sa_f32x4 c) {
@@ -271,6 +272,11 @@ __device__ __forceinline__ void f32_store(const F32Args& a, int bh, int qb, int 
   }
 }
 
+// Bits of |x| (see f32_terms_kernel).
+constexpr uint32_t kTermMax = 0x5d800000u;  // 2^60
+constexpr uint32_t kTermMin = 0x17800000u;  // 2^-80: 2^18 products that lose 2^-126 lose 2^-28 of a value
+constexpr uint32_t kTermSkip = 0xffffffffu;  // no |x| has these bits
+
 template <int kD, int kPool>
 __global__ __launch_bounds__(64 * kWavesF32, kD == 64 ? 2 : 1) void bsa_fwd_f32_kernel(F32Args a) {
   static_assert(kD == 64 || kD == 128, "head dim 64 or 128");
@@ -283,6 +289,8 @@ __global__ __launch_bounds__(64 * kWavesF32, kD == 64 ? 2 : 1) void bsa_fwd_f32_
   if (item < 0 || item >= a.n_items) return;
   const int bh = item / a.nqb;
   const int qb = item - bh * a.nqb;
+  // Behind bsa_fwd_f32_terms_kernel: the heads that it left (plain lists, so kv_rep = 1).
+  if (a.flags && a.flags[(int64_t)bh * a.nkb].x != kTermSkip) return;
   sa_f32x4 acc[kD / 16][4];
   float m[4], l[4];
   f32_rows<kD, kPool, 4>(a, bh, qb, 0, 0, 1, lane, acc, m, l);
@@ -306,13 +314,8 @@ __global__ __launch_bounds__(64 * kWavesF32, kD == 64 ? 2 : 1) void bsa_fwd_f32_
 // its products with probabilities far enough above 2^-126. Other heads run in fp32. (One value
 // decides for its head: a column or block of small values beside ordinary ones would lose its
 // low terms however large the head's maximum is.)
-// A head whose lists hold fewer than 3/2 tiles per key block is not worth the pass: its blocks
-// are only flagged (kTermSkip) and it runs in fp32. Measured on [2, 30, 17776, 64] (fp32 kernel
-// against this path, us): 2.1 tiles per block 586 / 609, 2.7 695 / 659, 4.3 993 / 801; with one
-// tile per block of [2, 30, 3000, 64] 49 / 92.
-constexpr uint32_t kTermMax = 0x5d800000u;  // 2^60
-constexpr uint32_t kTermMin = 0x17800000u;  // 2^-80: 2^18 products that lose 2^-126 lose 2^-28 of a value
-constexpr uint32_t kTermSkip = 0xffffffffu;  // no |x| has these bits
+// A head whose lists hold too few tiles to be worth the pass (terms_min_tiles4) is only flagged
+// (kTermSkip) and runs in fp32.
 
 template <int kD>
 struct TermLayout {
@@ -366,6 +369,9 @@ struct TermArgs {
   int Hk, Lk, nkb;
   const int32_t* kv_cnt;  // [B * Hk][nqb] list lengths, or null: every block is split
   int nqb, max_cnt;
+  int min_tiles4;  // listed tiles per four key blocks from which splitting pays,
+  int together;    // by the launch's mean, unless a head is far off; else by each head's
+  uint32_t lists;  // B * Hk * nqb
   uint8_t* planes;
   uint32_t* flags;  // [B * Hk * nkb][4]
 };
@@ -382,13 +388,21 @@ __global__ __launch_bounds__(256) void f32_terms_kernel(TermArgs a) {
   const int bh = (int)(blk / a.nkb);
   const int kb = (int)(blk - (int64_t)bh * a.nkb);
   if (a.kv_cnt) {
+    auto count = [&](int64_t row) { return min(max(a.kv_cnt[row], 0), a.max_cnt); };
     int64_t n = 0;
-    for (int i = threadIdx.x; i < a.nqb; i += 256) n += min(max(a.kv_cnt[(int64_t)bh * a.nqb + i], 0), a.max_cnt);
+    for (int i = threadIdx.x; i < a.nqb; i += 256) n += count((int64_t)bh * a.nqb + i);
+    // 64 of the launch's lists, at scattered places, the same in every wave.
+    int64_t m = a.together ? count((uint32_t)lane * 2654435761u % a.lists) : 0;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
+    for (int o = 32; o > 0; o >>= 1) {
+      n += __shfl_xor(n, o);
+      m += __shfl_xor(m, o);
+    }
     if (lane == 0) tiles[wave] = n;
     __syncthreads();
-    if (2 * (tiles[0] + tiles[1] + tiles[2] + tiles[3]) < 3 * (int64_t)a.nkb) {
+    int min4 = a.min_tiles4;
+    if (a.together) min4 = m * a.nqb * 4 < (int64_t)min4 * a.nkb * 64 ? max(min4, 12) : min(min4, 5);
+    if (4 * (tiles[0] + tiles[1] + tiles[2] + tiles[3]) < min4 * (int64_t)a.nkb) {
       if (threadIdx.x < 4) a.flags[blk * 4 + threadIdx.x] = kTermSkip;
       return;
     }
@@ -531,6 +545,7 @@ __global__ __launch_bounds__(256, 2) void bsa_fwd_f32_terms_kernel(F32Args a) {
   f32_u32x4 qhi[kG][kDS];
   f32_u32x4* ql = q_lds[wave];
   bool use_terms = (uint32_t)__builtin_amdgcn_readfirstlane((int)fl[0].x) != kTermSkip;
+  if (!use_terms && a.plain_after) return;
   if (use_terms) {
     // The flags of the head's blocks and of this wave's query rows.
     uint32_t worst = 0u;
@@ -857,6 +872,25 @@ void launch_terms_pool(const F32Args& a, hipStream_t s) {
   else hipLaunchKernelGGL((bsa_fwd_f32_terms_kernel<kD, kPool, 1>), grid, blk, 0, s, a);
 }
 
+// Heads with few tiles are not worth splitting k and v (12 D bytes per key). At head dim 64:
+//   up to kTermsAlways query blocks every head is split: the workgroups are too few for its cost to show
+//     ([1, 4, 2048] of one tile per key block 17.8 us, the fp32 kernel 17.6, of 1.6 tiles 22.5 / 56.8);
+//   up to kTermsInline a head of fewer than 3/2 tiles per key block runs in fp32 where it is, four waves
+//     sharing a unit: [1, 8, 4096] of 1.3 tiles 32 us (fp32 kernel 49), but of one tile 23 (19), [1, 16,
+//     4096] 42 (23);
+//   beyond, bsa_fwd_f32_kernel follows for such heads (one wave per unit; 3-7 us where there are none),
+//     and all heads go by the launch's mean unless one is far from it: with heads on both sides of the line
+//     each kernel leaves most of the card idle ([2, 30, 3000] of 1.8 tiles 176 us, all on one side 134).
+// Measured there by tiles per key block, 1 / 1.6 / 2 / 3 (us; the fp32 kernel alone, with every head
+// below 3/2 inline, and this): [2, 30, 3000] 50, 115, 131, 197 / 110, 153, 127, 140 / 61, 125, 135, 148;
+// [1, 30, 8192] 66, 137, 172, 231 / 143, 186, 172, 191 / 79, 151, 185, 200; [2, 30, 17776] 275, 464,
+// 557, 769 / 327, 587, 581, 661 / 305, 494, 586, 677.
+// Head dim 128 keeps 3/2 and one kernel at all sizes: its fp32 kernel fits one wave per SIMD, and [1, 15,
+// 17776] of one tile takes it 199 us where the inline path takes 174.
+constexpr int64_t kTermsAlways = 128;
+constexpr int64_t kTermsInline = 1024;
+int terms_min_tiles4(int64_t units) { return units <= 2048 ? 6 : units <= 3072 ? 7 : units <= 6144 ? 8 : 9; }
+
 template <int kD>
 int launch_terms(F32Args& a, int B, void* ws, int pool_cols, void* stream, const char* fn) {
   const int Hk = a.H / a.kv_rep;
@@ -868,6 +902,11 @@ int launch_terms(F32Args& a, int B, void* ws, int pool_cols, void* stream, const
   t.Hk = Hk; t.Lk = a.Lk; t.nkb = a.nkb;
   t.kv_cnt = a.list_bh_stride ? a.kv_cnt : nullptr;  // lists shared by the heads are dense
   t.nqb = a.nqb; t.max_cnt = a.max_cnt;
+  if (kD == 64 && a.n_items <= kTermsAlways) t.kv_cnt = nullptr;
+  t.together = kD == 64 && t.kv_cnt && a.n_items > kTermsInline;
+  t.min_tiles4 = t.together ? terms_min_tiles4(a.n_items) : 6;
+  t.lists = (uint32_t)B * Hk * a.nqb;
+  a.plain_after = t.together;
   t.planes = static_cast<uint8_t*>(ws);
   t.flags = reinterpret_cast<uint32_t*>(t.planes + blocks * TermLayout<kD>::kTile);
   hipStream_t s = sa::as_stream(stream);
@@ -878,6 +917,11 @@ int launch_terms(F32Args& a, int B, void* ws, int pool_cols, void* stream, const
   if (pool_cols == 32) launch_terms_pool<kD, 32>(a, s);
   else if (pool_cols == 64) launch_terms_pool<kD, 64>(a, s);
   else launch_terms_pool<kD, 0>(a, s);
+  if (a.plain_after) {
+    if (int rc = sa::check_launch(fn)) return rc;
+    const dim3 grid((unsigned)(a.n_slots / kWavesF32)), blk(64 * kWavesF32);
+    hipLaunchKernelGGL((bsa_fwd_f32_kernel<kD, 0>), grid, blk, 0, s, a);
+  }
   return sa::check_launch(fn);
 }
 
@@ -941,6 +985,9 @@ int launch_f32(const float* q, const int64_t q_strides[3], const float* k, const
   a.pool_ncol = pool_cols ? a.nkb * (kBlk / pool_cols) : 0;
   a.pool_lse = pool_lse;
   a.pool_lpad = nqb * kBlk;
+  a.planes = nullptr;
+  a.flags = nullptr;
+  a.plain_after = 0;
   SA_REQUIRE(pool_cols == 0 || (pool_r && pool_lse), "%s: pooling needs its buffers", fn);
   if (terms_ws) return D == 64 ? launch_terms<64>(a, B, terms_ws, pool_cols, stream, fn)
                                : launch_terms<128>(a, B, terms_ws, pool_cols, stream, fn);

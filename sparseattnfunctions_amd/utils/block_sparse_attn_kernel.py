@@ -123,10 +123,10 @@ def prepare_fp16_keys(k: torch.Tensor) -> Optional[FP16Keys]:
     return FP16Keys(k_in, ws, stream, event)
 
 
-# fp32 launches of at least this many query blocks run on split bf16 operands. Splitting k and v
-# is one launch more (37 -> 41 us a call where the host bounds it) and pays from two listed tiles
-# per key block, which the library counts per head: 16 blocks of a tenth of the keys each take
-# 66 -> 42 us a call, two heads of 32 blocks with a quarter 159 -> 37 us.
+# fp32 launches with at least this many query blocks per head run on split bf16 operands. Splitting k
+# and v is one launch more (37 -> 41 us a call where the host bounds it); whether it pays for a head's
+# lists the library decides on the device. 16 blocks of a tenth of the keys each take 66 -> 42 us a
+# call, two heads of 32 blocks with a quarter 159 -> 37 us.
 F32_TERMS_BLOCKS = 8
 
 

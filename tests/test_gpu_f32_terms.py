@@ -138,6 +138,45 @@ def test_short_lists_and_strided_rows(dev, monkeypatch):
     assert (new - old).abs().max() <= 4e-5
 
 
+# Heads with too few tiles per key block beside one that takes the split operands, past the size from
+# which the fp32 kernel runs them: its bits. Groups of four units that straddle heads, an empty list,
+# an order with text rows first. (At head dim 128 they stay in the split operands' kernel.)
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("H,Lq,Lk,text", [(27, 64 * 41 - 7, 64 * 41 - 7, 0), (47, 64 * 23, 64 * 23 + 1, 0),
+                                          (83, 64 * 13 - 1, 64 * 13 - 1, 1), (160, 64 * 40, 64 * 40, 0)])
+def test_heads_of_short_lists(dev, monkeypatch, D, H, Lq, Lk, text):
+    print(f"case terms heads of short lists D={D} H={H} {Lq} {Lk} text={text}", flush=True)
+    nqb, nkb = math.ceil(Lq / 64), math.ceil(Lk / 64)
+    q, k, v = _rand(1, 1, H, Lq, D).to(dev), _rand(2, 1, H, Lk, D).to(dev), _rand(3, 1, H, Lk, D).to(dev)
+    i, j = torch.arange(nqb)[:, None], torch.arange(nkb)
+    mask = (i % nkb == j).repeat(1, H, 1, 1)
+    mask[:, 1] = True  # the one head of long lists
+    mask[0, 2, 3] = False  # an empty list
+    kv = kv_list_from_mask(mask.to(dev), 1, H, nqb, nkb)
+    args = (q, k, v, kv, 0.125, None, None, text)
+    new, old = bsk.block_sparse_attention(*args), _plain(monkeypatch, *args)
+    short = [h for h in range(H) if h != 1]
+    if D == 64:
+        assert torch.equal(new[:, short], old[:, short])
+    assert torch.all(new[0, 2, 192:256] == 0)
+    assert not torch.equal(new[:, 1], old[:, 1])
+    assert (new - old).abs().max() <= 4e-5
+
+
+# Few query blocks (up to 128): every head is split, those of one tile per key block too.
+def test_short_lists_of_a_small_launch(dev, monkeypatch):
+    print("case terms short lists of a small launch", flush=True)
+    q, k, v = (_rand(i, 1, 3, 1000, 64) for i in (7, 8, 9))
+    mask = torch.eye(16, dtype=torch.bool).repeat(1, 3, 1, 1)
+    mask[0, 1, 5] = False
+    kv = kv_list_from_mask(mask.to(dev), 1, 3, 16, 16)
+    args = (q.to(dev), k.to(dev), v.to(dev), kv, 0.125)
+    new, old = bsk.block_sparse_attention(*args), _plain(monkeypatch, *args)
+    want = masked_attention(q, k, v, mask, 0.125)
+    assert (new.cpu().double() - want).abs().max() <= 2e-5 and torch.all(new[0, 1, 320:384] == 0)
+    assert not torch.equal(new, old)
+
+
 # The pooled map beside one-wave units (more than 6 144) and shared ones, partial last blocks,
 # grouped key heads; bars of the fp32 pooling tests.
 @pytest.mark.parametrize("H,Hk,L,D,bs,causal", [(130, 130, 3077, 64, 64, False), (130, 65, 3077, 64, 32, True),
