@@ -986,7 +986,8 @@ __global__ __launch_bounds__(256, 2) void simgram_kernel(SimGramArgs a) {
       if (!finish() || tiles == n_tiles) break;
     }
     drop_unused();
-    // The rows' factors by flat column; the lane's own stores to ws come back in order.
+    // The rows' factors by flat column. Below every lane reads the products that lanes 0 .. 31 stored to
+    // ws: a wave's accesses to memory take effect in its program order, so no wait is needed.
 #pragma unroll
     for (int g = 0; g < kSgGroups; ++g)
       if (hh == 0) L[32 * g + col] = inv[g];

@@ -449,8 +449,8 @@ def unified_judge(q, k, geometry: PatternGeometry = DEFAULT, draws=None):
     else:
         idx_q, ik1, ik2 = draws
     B, H = q.shape[:2]
-    # The sparsity judge (written probabilities and a latency-bound top-k pass) runs on a
-    # second stream (default priority) beside the two similarity judges (exp2/VALU-bound).
+    # The sparsity judge (a few score walks with LDS histograms) runs on a second stream (default
+    # priority) beside the two similarity judges; all three are VALU-bound.
     main = torch.cuda.current_stream(q.device)
     side = _side_stream(q.device) if OVERLAP_JUDGE else main
     side.wait_stream(main)
